@@ -20,15 +20,15 @@ constexpr int kIcpVals = 32;               // per-workgroup ICP partial record (
 // kCoarse^3 cells centred on block (0, 0, 0); cells outside it count as near.
 constexpr int kCoarse = 64;
 constexpr int kCoarseWords = kCoarse * kCoarse * kCoarse / 32;
-// Block-level bitmaps over the same window (kWin^3 blocks centred on block
-// (0, 0, 0), x fastest): "near" (an allocated block with an observed voxel
-// below the far threshold) and "dilated" (a near block within one block).
+// Block-level bits over the same window (kWin^3 blocks centred on block
+// (0, 0, 0)): "near" (an allocated block with an observed voxel below the far
+// threshold) and "dilated" (a near block within one block), stored in bricks
+// of 4^3 blocks, and the allocated blocks as a plain bitmap (x fastest).
 // Blocks outside the window are looked up through the hash table.
 constexpr int kWin = kCoarse * 8;
 constexpr size_t kWinWords = (size_t)kWin * kWin * kWin / 32;
-// Mid-level cells of 4^3 blocks over the same window (kCell4^3 cells).
-constexpr int kCell4 = kWin / 4;
-constexpr int kCell4Words = kCell4 * kCell4 * kCell4 / 32;
+constexpr int kBricks = kWin / 4;  // bricks per axis
+constexpr size_t kBrickCount = (size_t)kBricks * kBricks * kBricks;
 
 // per-volume counters, int32 each
 enum Ctr : int {
@@ -80,10 +80,11 @@ struct DmView {
   int32_t *free_list;   // num_blocks: pool indices returned by deletion (HashTable::DeleteBlock
                         // + Heap::Append), taken back by later insertions
   uint8_t *blk_near;    // num_blocks: 1 when an observed voxel lies below the raycast far threshold
-  uint32_t *nearmap;    // kWinWords: window bit of every block with blk_near set
-  uint32_t *dilmap;     // kWinWords: window bit of every block within one block of a near block
-  uint32_t *coarse;     // kCoarse^3 bits: cell of 8^3 blocks holds a block with its dilmap bit set
-  uint32_t *cell4;      // kCell4^3 bits: cell of 4^3 blocks holds a block with its dilmap bit set
+  // kBrickCount records {x: dilated, y: near}, one bit per block of the brick
+  // (x + 4 y + 16 z): one 16-byte load tells the raycast whether the block is
+  // dilated, whether its whole brick is clear, and which blocks beside it are near
+  ulonglong2 *bricks;
+  uint32_t *coarse;     // kCoarse^3 bits: cell of 8^3 blocks holds a block with its dilated bit set
   uint32_t *allocmap;   // kWinWords: window bit of every allocated block (the allocation's
                         // table test; blocks outside the window go through the hash table)
   uint64_t *dset;       // per-frame new-key set, dset_mask + 1 slots, 0 = empty
@@ -152,7 +153,7 @@ void launch_delete(const DmView *view, const int4 *req, int n, unsigned long lon
 // live blocks whose centre lies farther than radius from c, appended to req
 // (capacity: the pool size) with *nreq counting them
 void launch_select_far(const DmView *view, const double c[3], double radius, int4 *req, int *nreq, hipStream_t st);
-void rebuild_far_maps(const Launch &L);  // clear and rebuild nearmap/dilmap/cell4/coarse/allocmap (not for graph capture)
+void rebuild_far_maps(const Launch &L);  // clear and rebuild bricks/coarse/allocmap (not for graph capture)
 void launch_source_maps(const Launch &L);
 // ICP linearisation at one level (one FP32 record per workgroup); with solve,
 // a second kernel sums the records and takes the Gauss-Newton step on the
