@@ -727,7 +727,31 @@ struct BlockWin {
   unsigned resolved;   // bit k < 8: LDS slot k holds the pool index; bits 8, 9, 10: the ray
                        // runs towards -x, -y, -z (the window extends that way)
   int *slot;           // this thread's slots: slot[k * 256], k = x + 2y + 4z
+  unsigned long long *cache;  // the workgroup's block pointers (find_block_shared)
 };
+
+// find_block through a small direct-mapped cache in LDS that the rays of a
+// workgroup share: an entry holds (occupied bit | window coordinates) << 32 |
+// pool index (-1 = unallocated), read and written as one 64-bit word, so a
+// reader sees either an older block's entry (a miss) or a whole new one.  A
+// 16x16 tile's rays end on a few dozen blocks and make about 1600 lookups
+// together; from the table in HBM one is 2000 to 4000 cycles that nothing else
+// of the ray can overlap (16 sessions: 0.857 -> 0.756 ms, 640x480 / 8 mm alone
+// 193 -> 168 us, 320x240 / 2 cm 152 -> 133 us).  Blocks outside the window are
+// looked up directly.
+constexpr int kBlkCache = 256;
+__device__ __forceinline__ int find_block_shared(const DmView &v, int x, int y, int z, unsigned long long *cache) {
+  const unsigned X = x + kWin / 2, Y = y + kWin / 2, Z = z + kWin / 2;
+  if (X >= (unsigned)kWin || Y >= (unsigned)kWin || Z >= (unsigned)kWin) return find_block(v, x, y, z);
+  const uint32_t tag = 0x80000000u | (Z << 18) | (Y << 9) | X;
+  unsigned long long *e = cache + ((X & 7u) | ((Y & 7u) << 3) | ((Z & 3u) << 6));
+  const unsigned long long w = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if ((uint32_t)(w >> 32) == tag) return (int)(uint32_t)w;
+  const int ptr = find_block(v, x, y, z);
+  __hip_atomic_store(e, ((unsigned long long)tag << 32) | (uint32_t)ptr, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_WORKGROUP);
+  return ptr;
+}
 
 // voxel word of global voxel (gx, gy, gz) through the hash table
 __device__ __forceinline__ uint64_t voxel_lookup(const DmView &v, int gx, int gy, int gz) {
@@ -840,7 +864,7 @@ __device__ __forceinline__ bool interp_axes(const DmView &v, const AxisSample &X
   while (todo) {
     const int k = __builtin_ctz(todo);
     todo &= todo - 1u;
-    const int ptr = find_block(v, W.wx + (k & 1), W.wy + ((k >> 1) & 1), W.wz + (k >> 2));
+    const int ptr = find_block_shared(v, W.wx + (k & 1), W.wy + ((k >> 1) & 1), W.wz + (k >> 2), W.cache);
     W.slot[k * 256] = ptr < 0 ? v.num_blocks : ptr;  // unallocated: the pool's all-zero block
     W.resolved |= 1u << k;
   }
@@ -950,7 +974,7 @@ __device__ __forceinline__ void hit_stencil(const DmView &v, const AxisSample &X
   while (todo) {
     const int k = __builtin_ctz(todo);
     todo &= todo - 1u;
-    const int ptr = find_block(v, W.wx + (k & 1), W.wy + ((k >> 1) & 1), W.wz + (k >> 2));
+    const int ptr = find_block_shared(v, W.wx + (k & 1), W.wy + ((k >> 1) & 1), W.wz + (k >> 2), W.cache);
     W.slot[k * 256] = ptr < 0 ? v.num_blocks : ptr;
     W.resolved |= 1u << k;
   }
@@ -1243,10 +1267,14 @@ __global__ __launch_bounds__(256, 6) void k_raycast(const DmView *__restrict__ v
   const f3 po = mk(T.m[3], T.m[7], T.m[11]) * inv_vs;
   const f3 pd = rot(T, mk(((float)u - s.cx) * ifx, ((float)r - s.cy) * ify, 1.0f)) * inv_vs;
   __shared__ int win_lds[8 * 256];
+  __shared__ unsigned long long blk_cache[kBlkCache];
+  blk_cache[threadIdx.x] = 0ull;
+  __syncthreads();
   BlockWin c;
   c.wx = 0x3fffffff; c.wy = 0; c.wz = 0;
   c.resolved = (pd.x < 0.f ? 0x100u : 0u) | (pd.y < 0.f ? 0x200u : 0u) | (pd.z < 0.f ? 0x400u : 0u);
   c.slot = win_lds + threadIdx.x;
+  c.cache = blk_cache;
   float z = v.min_depth, pz = 0.f, ps = 0.f, zh = 0.f, zprev = 0.f;
   bool pobs = false, hit = false, prev_fast = false;
   const int nbeam = beam_steps(v, s, T, po, inv_vs, ifx, ify, u, r, tw_log2, big, max_steps);

@@ -44,3 +44,25 @@ def test_raycast_empty_space_bits(room, shift):
     assert hit.mean() > 0.8 and np.mean((gd > 0) == hit) >= 0.999
     tol = 1e-5 if max(np.abs(shift)) < 8 else 3e-5
     assert np.mean(np.abs(gd - od)[hit & (gd > 0)] <= tol) >= 0.999
+
+
+# The wavefront's shared first steps and the workgroup's shared block pointers
+# at image sizes that leave partial tiles and at a field of view so wide that
+# the bundle bound ends the shared steps early (fx = 40 at 96 columns), close
+# and far minimum depths.  Same bounds as above.
+@pytest.mark.parametrize("rows,cols,fx,dmin", [(1, 1, 60.0, 0.3), (7, 9, 12.0, 0.3), (17, 33, 30.0, 0.1),
+                                              (96, 97, 40.0, 0.3), (130, 63, 400.0, 1.2)])
+def test_raycast_ragged_views(room, rows, cols, fx, dmin):
+    depth, poses = room
+    props = small_tsdf(min_sensor_depth=dmin)
+    vol = dm.TsdfVolume(props, SENS["rows"], SENS["cols"])
+    for f in range(3):
+        vol.IntegrateScan(depth[f], None, SENS, poses[f].astype(np.float32))
+    sens = dict(rows=rows, cols=cols, fx=fx, fy=fx, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    Tf = poses[1].astype(np.float32)
+    gd = vol.Raycast(Tf, sens)[0]
+    od = mirror(vol, props).raycast(Tf.astype(np.float64), sens)[0]
+    hit = od > 0
+    assert np.mean((gd > 0) == hit) >= 0.999
+    both = hit & (gd > 0)
+    assert both.sum() == 0 or np.mean(np.abs(gd - od)[both] <= 1e-5) >= 0.999
