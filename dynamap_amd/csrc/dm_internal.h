@@ -48,6 +48,7 @@ enum Ctr : int {
   C_NNEW = 12,       // keys inserted by the last allocation
   C_ICP_STOP = 13,   // level + 1 of the ICP level that ended early this frame, 0 = none
   C_NUM_FREE = 14,   // freed pool indices waiting in free_list (a stack; reused first)
+  C_ICP_TICKET = 15, // workgroups of the running linearisation that have stored their record (0 between launches)
   C_COUNT = 16
 };
 
@@ -156,8 +157,8 @@ void launch_select_far(const DmView *view, const double c[3], double radius, int
 void rebuild_far_maps(const Launch &L);  // clear and rebuild bricks/coarse/allocmap (not for graph capture)
 void launch_source_maps(const Launch &L);
 // ICP linearisation at one level (one FP32 record per workgroup); with solve,
-// a second kernel sums the records and takes the Gauss-Newton step on the
-// device.
+// each session's last workgroup sums the records and takes the Gauss-Newton
+// step on the device.
 void launch_icp_reduce(const Launch &L, int level, int it, bool solve);
 void launch_pose_begin(const Launch &L);
 void launch_pose_log(const Launch &L, const int *dest, double *log);

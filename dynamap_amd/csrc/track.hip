@@ -8,9 +8,10 @@
 // Per iteration the reduction kernel evaluates one Gauss-Newton linearisation
 // per pixel and reduces the 30 sums (21 of J J^T, 6 of J r, counts) with a
 // wavefront shuffle tree plus an LDS stage into one record per workgroup; the
-// solve kernel adds the records in FP64 in a fixed order, solves the damped
-// 6x6 system with an FP64 LDL^T and composes the SE(3) increment on the
-// device, so a frame's iterations run back to back without a host round trip.
+// session's last workgroup adds the records in FP64 in a fixed order, solves
+// the damped 6x6 system with an FP64 LDL^T and composes the SE(3) increment, so
+// an iteration is one launch and a frame's iterations run back to back without
+// a host round trip.
 #include "dm_device.h"
 #include "dm_solve.h"
 
@@ -229,44 +230,243 @@ __device__ __forceinline__ void icp_features(const DmView &v, int level, const I
   }
 }
 
-// The damped Gauss-Newton step from the summed records: Tinc <- exp(xi)
-// Tinc.  On the session's last iteration of the frame apply the reference's
-// guard (gnSolver.cu:426-428) and set the frame pose T = Tprev * Tinc.
-__device__ void icp_step_device(const DmView &v, int level, int it, const double *sums) {
-  double A[36], b[6], xi[6], E[16];
-  sym6_from_upper(sums, A);
-  for (int k = 0; k < 6; ++k) b[k] = sums[21 + k];
-  icp_step(A, b, it, (double)v.lambda, xi);
+// ---- the Gauss-Newton step on the device
+// Value of lane `l` (uniform) in every lane.
+__device__ __forceinline__ double lane_f64(double x, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+// Largest value of lanes 0..31, ignoring NaN.
+__device__ __forceinline__ double max_f64(double a, double b) { return b > a || a != a ? b : a; }
+__device__ __forceinline__ double half_max(double x) {
+  x = max_f64(x, dpp_f64<0xb1>(x));
+  x = max_f64(x, dpp_f64<0x4e>(x));
+  x = max_f64(x, dpp_f64<0x141>(x));
+  x = max_f64(x, dpp_f64<0x140>(x));
+  return max_f64(x, __shfl_xor(x, 16, 64));
+}
+
+// Scratch of the step in LDS.
+struct IcpStepLds {
+  double part[32][32];    // sums of 8 leaves each, by value
+  double pd[PD_COUNT];    // the session's pose block
+  double m[16], t[16];    // matrices handed between lanes
+};
+
+// A record value: written by other workgroups of the same launch, so it is
+// read past this XCD's caches.
+__device__ __forceinline__ float record_value(const float *p) {
+  return __hip_atomic_load((const __attribute__((address_space(1))) float *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The damped Gauss-Newton step of one session, by one workgroup of 256
+// threads once every record of the linearisation is stored.
+// Sum: leaf t of 256 adds records t, t + 256, ... in order, and the leaves are
+// added by the balanced tree over their index, in FP64 (host replica:
+// icp_sum_records).  32 lanes read the 128 bytes of one record.
+// Step: wavefront 0 holds row i of the 6x6 system in lane i; each operation is
+// icp_step's and se3_exp's own, in the same order, but a column's entries (and
+// an element each of the 4x4 products) are computed side by side, and the
+// pose block is read once into LDS at the start and written once.  Bound by the
+// chain of dependent FP64 operations and loads: about 6 us.  One thread doing
+// all of it, with a memory round trip for each pose entry it changed, took 11
+// to 13 us.
+// Tinc <- exp(xi) Tinc.  On the session's last iteration of the frame apply
+// the reference's guard (gnSolver.cu:426-428) and set T = Tprev * Tinc.
+__device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepLds &S) {
+  const int k = threadIdx.x & 31, j = threadIdx.x >> 5;
+  if (threadIdx.x < PD_COUNT) S.pd[threadIdx.x] = v.posed[threadIdx.x];
+  auto value = [&](int t) { return record_value(v.partials + (size_t)min(t, nwg - 1) * kIcpVals + k); };
+#pragma unroll 1
+  for (int h = 0; h < 2; ++h) {  // leaves 128 h .. 128 h + 127
+    // every load unconditional (past the end: the last record, not added), so
+    // that 16 are in flight together
+    float x[2][8];
+    const int t0 = 128 * h + 8 * j;
+    if (128 * h < nwg) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) x[q >> 3][q & 7] = value(t0 + 64 * (q >> 3) + (q & 7));
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      double l[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) l[q] = t0 + 64 * g + q < nwg ? 0.0 + (double)x[g][q] : 0.0;
+      for (int t = t0 + 64 * g + 256; t < nwg; t += 256) {  // more than 256 records (512x512 pixels)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[g][q] = value(t + q);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) l[q] = t + q < nwg ? l[q] + (double)x[g][q] : l[q];
+      }
+      S.part[16 * h + 8 * g + j][k] = ((l[0] + l[1]) + (l[2] + l[3])) + ((l[4] + l[5]) + (l[6] + l[7]));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  double part[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    double l[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) l[q] = S.part[8 * g + q][k];
+    part[g] = ((l[0] + l[1]) + (l[2] + l[3])) + ((l[4] + l[5]) + (l[6] + l[7]));
+  }
+  const double sum = (part[0] + part[1]) + (part[2] + part[3]);
+  // icp_step: row `lane` of A (lanes 0..5), scaled by 1 / max(A), damped
+  const double s0 = lane_f64(sum, 0);
+  double mx = half_max(lane < 21 ? sum : s0);
+  mx = s0 != s0 ? s0 : lane_f64(mx, 0);
+  double xi[6] = {0, 0, 0, 0, 0, 0};
+  if (mx > 0.0) {
+    const double sc = 1.0 / mx;
+    const double alpha = (double)v.lambda * (mx * sc) / (double)it;
+    const int row = lane < 6 ? lane : 5;
+    double A[6], L[6], D[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+      const int r0 = min(row, c), c0 = max(row, c);
+      A[c] = __shfl(sum, 6 * r0 - (r0 * (r0 - 1)) / 2 + c0 - r0, 64) * sc;
+      if (c == row) A[c] += alpha;
+    }
+    double y = -__shfl(sum, 21 + row, 64) * sc;
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {  // column c of L, one row per lane
+      double d = lane_f64(A[c], c), a = A[c];
+#pragma unroll
+      for (int q = 0; q < c; ++q) {
+        const double lc = lane_f64(L[q], c);
+        d -= lc * lc * D[q];
+        a -= L[q] * lc * D[q];
+      }
+      D[c] = d;
+      ok = ok && d > 0.0;
+      L[c] = a / d;
+    }
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {  // forward substitution
+      const double yq = lane_f64(y, q);
+      if (row > q) y -= L[q] * yq;
+    }
+    double dr = D[0];
+#pragma unroll
+    for (int q = 1; q < 6; ++q) dr = row == q ? D[q] : dr;
+    y /= dr;
+#pragma unroll
+    for (int i = 5; i >= 0; --i) {  // back substitution
+      double a = lane_f64(y, i);
+#pragma unroll
+      for (int q = i + 1; q < 6; ++q) a -= lane_f64(L[i], q) * xi[q];
+      xi[i] = a;
+    }
+    if (!ok)
+#pragma unroll
+      for (int q = 0; q < 6; ++q) xi[q] = 0.0;
+  }
+  double E[16];
   se3_exp(xi, E);
-  double *Tinc = v.posed + PD_TINC;
-  mat4_mul(E, Tinc, Tinc);
-  for (int k = 0; k < 6; ++k) v.posed[PD_ACC + k] += xi[k];
+  const int r4 = (lane >> 2) & 3, c4 = lane & 3, e = lane & 15;
+#pragma unroll
+  for (int q = 0; q < 16; ++q)
+    if (e == q) S.m[q] = E[q];
+  const double *Ti = S.pd + PD_TINC;
+  double tinc = S.m[4 * r4] * Ti[c4] + S.m[4 * r4 + 1] * Ti[4 + c4] + S.m[4 * r4 + 2] * Ti[8 + c4] +
+                S.m[4 * r4 + 3] * Ti[12 + c4];
   // gnSolver.cu:413-415: the level ends once the summed twist changed by at
   // most min_increment since the last step that did not end a level
-  const bool stop = level_converged(v.posed + PD_ACC, v.posed + PD_PREVACC, (double)v.min_inc);
-  if (stop) v.ctr[C_ICP_STOP] = level + 1;
+  double acc[6], prev[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    acc[q] = S.pd[PD_ACC + q] + xi[q];
+    prev[q] = S.pd[PD_PREVACC + q];
+  }
+  const bool stop = level_converged(acc, prev, (double)v.min_inc);
+#pragma unroll
+  for (int q = 0; q < 6; ++q)
+    if (lane == q) {
+      v.posed[PD_ACC + q] = acc[q];
+      v.posed[PD_PREVACC + q] = prev[q];
+    }
+  if (stop && lane == 0) v.ctr[C_ICP_STOP] = level + 1;
   bool last = it == v.iters[level] || stop;
   for (int l = 0; l < level; ++l) last = last && v.iters[l] == 0;
   if (last) {
-    const double *acc = v.posed + PD_ACC;
     const double ssum = acc[0] + acc[1] + acc[2] + acc[3] + acc[4] + acc[5];
     if (ssum != ssum || isinf(ssum) || ssum >= (double)v.max_inc) {
-      for (int k = 0; k < 16; ++k) Tinc[k] = (k % 5 == 0) ? 1.0 : 0.0;
-      atomicAdd(&v.ctr[C_ICP_FAIL], 1);
+      tinc = r4 == c4 ? 1.0 : 0.0;
+      if (lane == 0) atomicAdd(&v.ctr[C_ICP_FAIL], 1);
     }
-    double *T = v.posed + PD_T;
-    mat4_mul(v.posed + PD_TPREV, Tinc, T);
-    for (int k = 0; k < 16; ++k) v.posef[PF_T + k] = (float)T[k];
-    rigid_inverse_ff(v.posef + PF_T, v.posef + PF_TINV);
+    if (lane < 16) S.t[e] = tinc;
+    const double *Tp = S.pd + PD_TPREV;
+    const double T = Tp[4 * r4] * S.t[c4] + Tp[4 * r4 + 1] * S.t[4 + c4] + Tp[4 * r4 + 2] * S.t[8 + c4] +
+                     Tp[4 * r4 + 3] * S.t[12 + c4];
+    const double Tf = (double)(float)T;  // the inverse is the float pose's
+    if (lane < 16) S.m[e] = Tf;
+    const double inv = r4 == 3 ? (c4 == 3 ? 1.0 : 0.0)
+                       : c4 < 3 ? S.m[4 * c4 + r4]
+                                : -(S.m[r4] * S.m[3] + S.m[4 + r4] * S.m[7] + S.m[8 + r4] * S.m[11]);
+    if (lane < 16) {
+      v.posed[PD_T + e] = T;
+      v.posef[PF_T + e] = (float)T;
+      v.posef[PF_TINV + e] = (float)inv;
+    }
   }
-  for (int k = 0; k < 16; ++k) v.posef[PF_TINC + k] = (float)Tinc[k];
+  if (lane < 16) {
+    v.posed[PD_TINC + e] = tinc;
+    v.posef[PF_TINC + e] = (float)tinc;
+  }
+}
+
+// Value k of the workgroup's record into v.partials, then, with solve, the
+// step by the workgroup that is the session's last to do so (threads < kVals
+// call with their value, the others with any; all threads call).
+// Records and tickets pass between XCDs, whose L2s are not coherent within a
+// launch.  A device-scope release would write back the whole L2 (about 0.5 us
+// each, serialised per XCD: 4800 workgroups lost 0.28 ms to it); instead the
+// record is stored write-through (agent-scope atomic stores), wavefront 0 waits
+// for its stores to complete there, and only then takes its ticket; the last
+// one reads the records past its caches.  Tickets of one counter are served
+// about 80 ns apart (300 workgroups: 24 us), so the workgroups of a group of 16
+// count among themselves, in an unused value of the group's first record, and
+// each group's last one counts for the session.
+// The step in the reduction's launch saves a launch per iteration, most of
+// them no-ops because the level has converged: at 640x480 reduction and step
+// took 18 + 13 us at level 0 and 1.1 + 1.1 us when converged, now 26 and 1.1;
+// a 320x240 frame's 19 iterations 148 -> 136 us of kernels and 19 launches less.
+constexpr int kIcpGroup = 16;
+__device__ __forceinline__ void icp_record(const DmView &v, float val, int level, int it, int nwg, int solve,
+                                           IcpStepLds &S) {
+  if (threadIdx.x < kVals)
+    __hip_atomic_store(v.partials + (size_t)blockIdx.x * kIcpVals + threadIdx.x, val, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  if (!solve) return;
+  __shared__ int last;
+  if (threadIdx.x < 64) {  // the wavefront that stored the record
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (threadIdx.x == 0) {
+      const int g = blockIdx.x / kIcpGroup, ng = (nwg + kIcpGroup - 1) / kIcpGroup;
+      int *gt = (int *)(v.partials + (size_t)g * kIcpGroup * kIcpVals + 31);
+      int l = 0;
+      if (__hip_atomic_fetch_add(gt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+          min(kIcpGroup, nwg - g * kIcpGroup) - 1) {
+        __hip_atomic_store(gt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        l = __hip_atomic_fetch_add(&v.ctr[C_ICP_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
+      }
+      last = l;
+    }
+  }
+  __syncthreads();
+  if (!last) return;
+  if (threadIdx.x == 0) v.ctr[C_ICP_TICKET] = 0;
+  icp_finish(v, level, it, nwg, S);
 }
 
 // One linearisation: every thread accumulates 4 pixels (strided by 256 for
 // coalescing) in FP32; a wavefront tree (wave_sum: DPP row permutes, then
 // two shuffles) and an LDS stage reduce them to one record per workgroup.
 __global__ __launch_bounds__(256) void k_icp_reduce(const DmView *__restrict__ views, const int *__restrict__ active,
-                                                     int level, int it) {
+                                                     int level, int it, int solve) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
@@ -293,10 +493,13 @@ __global__ __launch_bounds__(256) void k_icp_reduce(const DmView *__restrict__ v
     for (int k = 0; k < kVals; ++k) red[wave][k] = vals[k];
   }
   __syncthreads();
+  float val = 0.f;
   if (threadIdx.x < kVals) {
     const int k = threadIdx.x;
-    v.partials[(size_t)blockIdx.x * kIcpVals + k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+    val = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
   }
+  __shared__ IcpStepLds step;
+  icp_record(v, val, level, it, nwg, solve, step);
 }
 
 // The same linearisation on the matrix cores: each pixel's 16-float feature
@@ -311,7 +514,8 @@ __global__ __launch_bounds__(256) void k_icp_reduce(const DmView *__restrict__ v
 typedef float icp_f4 __attribute__((ext_vector_type(4)));
 constexpr int kFeatPitch = 17;  // LDS row pitch (floats): rows of a wave fall on distinct banks
 __global__ __launch_bounds__(256) void k_icp_reduce_mfma(const DmView *__restrict__ views,
-                                                          const int *__restrict__ active, int level, int it) {
+                                                          const int *__restrict__ active, int level, int it,
+                                                          int solve) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
@@ -349,13 +553,13 @@ __global__ __launch_bounds__(256) void k_icp_reduce_mfma(const DmView *__restric
 #pragma unroll
   for (int e = 0; e < 4; ++e) tile[wave][(4 * (lane >> 4) + e) * 16 + (lane & 15)] = acc[e];
   __syncthreads();
+  float val = 0.f;
   if (threadIdx.x < kVals) {
     const int k = threadIdx.x;
     auto T = [&](int r, int c) {
       const int o = r * 16 + c;
       return (tile[0][o] + tile[1][o]) + (tile[2][o] + tile[3][o]);
     };
-    float val;
     if (k < 21) {
       int a = 0, kk = k;
       while (kk >= 6 - a) { kk -= 6 - a; ++a; }
@@ -370,41 +574,9 @@ __global__ __launch_bounds__(256) void k_icp_reduce_mfma(const DmView *__restric
     } else {
       val = T(15, 15);
     }
-    v.partials[(size_t)blockIdx.x * kIcpVals + k] = val;
   }
-}
-
-// Sum the records in FP64 in a fixed order (thread t takes records t, t+256,
-// ...; wave_sum's tree per wavefront; (w0 + w1) + (w2 + w3); host replica:
-// icp_sum_records) and take the Gauss-Newton step (one workgroup per session).
-__global__ __launch_bounds__(256) void k_icp_solve(const DmView *__restrict__ views, const int *__restrict__ active,
-                                                    int level, int it) {
-  const int slot_ = active[blockIdx.x];
-  if (slot_ < 0) return;
-  const DmView &v = views[slot_];
-  if (v.ctr[C_HAS_MODEL] == 0 || it > v.iters[level] || v.ctr[C_ICP_STOP] == level + 1) return;
-  const int nwg = icp_wg_count((v.rows >> level) * (v.cols >> level));
-  double acc[kVals];
-#pragma unroll
-  for (int k = 0; k < kVals; ++k) acc[k] = 0.0;
-  for (int w = threadIdx.x; w < nwg; w += 256) {
-    const float *rec = v.partials + (size_t)w * kIcpVals;
-#pragma unroll
-    for (int k = 0; k < kVals; ++k) acc[k] += (double)rec[k];
-  }
-#pragma unroll
-  for (int k = 0; k < kVals; ++k) acc[k] = wave_sum(acc[k]);
-  __shared__ double dred[4][kVals];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < kVals; ++k) dred[wave][k] = acc[k];
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  double sums[kVals];
-  for (int k = 0; k < kVals; ++k) sums[k] = (dred[0][k] + dred[1][k]) + (dred[2][k] + dred[3][k]);
-  icp_step_device(v, level, it, sums);
+  __shared__ IcpStepLds step;
+  icp_record(v, val, level, it, nwg, solve, step);
 }
 
 // Start of a frame: Tprev <- T when a model exists, otherwise T <- Tinit;
@@ -444,14 +616,8 @@ void launch_source_maps(const Launch &L) {
 void launch_icp_reduce(const Launch &L, int level, int it, bool solve) {
   if (L.nact <= 0) return;
   const int P = L.max_pixels >> (2 * level);
-  if (L.icp_mfma)
-    hipLaunchKernelGGL(k_icp_reduce_mfma, dim3((unsigned)icp_wg_count(P), (unsigned)L.nact), dim3(256), 0, L.stream,
-                       L.views, L.active, level, it);
-  else
-    hipLaunchKernelGGL(k_icp_reduce, dim3((unsigned)icp_wg_count(P), (unsigned)L.nact), dim3(256), 0, L.stream,
-                       L.views, L.active, level, it);
-  if (solve)
-    hipLaunchKernelGGL(k_icp_solve, dim3((unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active, level, it);
+  hipLaunchKernelGGL(L.icp_mfma ? k_icp_reduce_mfma : k_icp_reduce, dim3((unsigned)icp_wg_count(P), (unsigned)L.nact),
+                     dim3(256), 0, L.stream, L.views, L.active, level, it, solve ? 1 : 0);
 }
 
 void icp_sum_records(const float *part, int nwg, double *sums) {

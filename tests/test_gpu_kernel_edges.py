@@ -66,3 +66,29 @@ def test_raycast_ragged_views(room, rows, cols, fx, dmin):
     assert np.mean((gd > 0) == hit) >= 0.999
     both = hit & (gd > 0)
     assert both.sum() == 0 or np.mean(np.abs(gd - od)[both] <= 1e-5) >= 0.999
+
+
+# One linearisation record per 1024 pixels, 16 records per ticket group, 256
+# leaves in the sum of the records: frames of 1, 16, 17, 256 and 257 records at
+# level 0.  The host path sums the same records in the same order and takes the
+# same FP64 step, so the increments agree to FP64 rounding (sin and cos of the
+# two sides may differ in the last bit).
+@pytest.mark.parametrize("variant", ["shuffle", "mfma"])
+@pytest.mark.parametrize("rows,cols", [(24, 40), (128, 128), (130, 128), (512, 512), (513, 512)])
+def test_icp_step_record_counts(rows, cols, variant):
+    f = 0.82 * cols
+    sens = dict(rows=rows, cols=cols, fx=f, fy=f, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    sc = configs.Scene(1, configs.SEED_BASE + 1002)
+    poses = sc.trajectory(2, configs.SEED_BASE + 1002)
+    frames = [sc.render(p, sens, 7, noise=False)[0] for p in poses]
+    s = dm.Session(small_tsdf(), configs.ICP_DEPTH, sens, np.eye(4))
+    for l in range(3):
+        v, n, i = s.source_maps(frames[0], None, l)
+        s.set_model_maps(l, v, n, i)
+    s.source_maps(frames[1], None, 0)
+    s.set_icp_reduce(variant)
+    dev = [s.icp_track(solve_on_host=False) for _ in range(3)]
+    host = s.icp_track(solve_on_host=True)
+    assert np.linalg.norm(host[:3, 3]) > 1e-4
+    for T in dev:
+        np.testing.assert_allclose(T, host, rtol=0, atol=1e-12)
