@@ -15,6 +15,8 @@ template <class T> __device__ __forceinline__ T ldg(const T *p) {
   return *(const __attribute__((address_space(1))) T *)p;
 }
 
+template <class T> __device__ __forceinline__ void stg(T *p, T x) { *(__attribute__((address_space(1))) T *)p = x; }
+
 struct f3 { float x, y, z; };
 __device__ __forceinline__ f3 mk(float x, float y, float z) { return f3{x, y, z}; }
 __device__ __forceinline__ f3 operator+(f3 a, f3 b) { return mk(a.x + b.x, a.y + b.y, a.z + b.z); }
@@ -38,6 +40,12 @@ __device__ __forceinline__ M4 load_m4(const float *p) {
   M4 r;
 #pragma unroll
   for (int k = 0; k < 16; ++k) r.m[k] = p[k];
+  return r;
+}
+__device__ __forceinline__ M4 load_m4g(const float *p) {  // from global memory
+  M4 r;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) r.m[k] = ldg(p + k);
   return r;
 }
 // include/math/utils_matrix.h:923-930: ((m11 x + m12 y) + m13 z) + m14*1

@@ -15,6 +15,10 @@
 
 namespace dm {
 
+typedef unsigned long u64;  // uint64_t
+typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ Intr intr_of(const DmView &v) {
   return Intr{v.rows, v.cols, v.fx, v.fy, v.cx, v.cy};
 }
@@ -356,62 +360,110 @@ __global__ void k_alloc_close(const DmView *__restrict__ views, const int *__res
 
 // ---------------------------------------------------------------------------
 // Integration (IntegrateScanKernel, tsdf.cu:267-344; merge geom_Types.h:79-102)
-// One workgroup per voxel block (grid-stride over the allocated blocks), two
-// voxels per thread, coalesced 8-byte voxel words; unchanged voxels are not
-// written back.
+// One wavefront per voxel block: lane (y, z) takes the 8 voxels of its row
+// along x, so the rows' 64 words are one coalesced access per x and the parts
+// of the camera transform that depend on y and z are computed once for 8
+// voxels.  Unchanged voxels are not written back.
 // One colour channel of Voxel::mergeVoxel (geom_Types.h:85-90):
 // uchar((c*w + c_new) / (w + 1)) with the float quotient truncated.  Here n =
 // c*w + c_new and m = w + 1 are integers (c, c_new, w <= 255, so n < 2^16 and
 // n/m <= 255), and the correctly rounded float quotient truncates to
 // floor(n/m): a non-integer n/m lies at least 1/m >= 2^-8 from the integers,
 // far beyond the quotient's rounding error (2^-24 * 255).  floor(n/m) is
-// taken as trunc((n + 1/2) * rm) with rm = rcp(m) (v_rcp_f32, 1 ulp):
+// taken as trunc((n + 1/2) * rm), of which this is the product, with rm =
+// rcp(m) (v_rcp_f32, 1 ulp):
 // (n + 1/2)/m lies at least 1/(2m) >= 2^-9 from every integer, while the
 // reciprocal's and the product's rounding move it by at most
 // 255.5 * (2^-23 + 2^-24) < 2^-14.
-__device__ __forceinline__ uint32_t merge_channel(uint32_t c, uint32_t w, uint32_t c_new, float rm) {
-  return (uint32_t)(((float)(c * w + c_new) + 0.5f) * rm);
+__device__ __forceinline__ float merge_channel(float c, float w, float c_new, float rm) {
+  return __builtin_fmaf(c, w, c_new + 0.5f) * rm;  // c w + c_new + 1/2 is exact
 }
 
-// One voxel of IntegrateScanKernel (tsdf.cu:301-341): returns the new voxel
-// word (the old one when the voxel is not updated).
-__device__ __forceinline__ uint64_t integrate_voxel(const DmView &v, const Intr &s, const M4 &Ti, f3 pos, int t,
-                                                    uint64_t old) {
-  const float vs = v.voxel_size, tau = v.trunc;
-  const int bx = t >> 6, by = (t >> 3) & 7, bz = t & 7;
-  const f3 vp = mk(pos.x + (float)bx * vs, pos.y + (float)by * vs, pos.z + (float)bz * vs);
-  const f3 vc = xform(Ti, vp);
+// a / b, correctly rounded, with b's reciprocal shared between quotients: the
+// steps of the IEEE division (reciprocal, one Newton step, two residual
+// corrections) without the scaling that it needs for extreme exponents.  The
+// caller keeps |b| and a nonzero |a| within 2^-80 .. 2^80.  (Compared with a / b
+// on 1.7e10 pairs, every mantissa of b and every b from 1 to 256 with every
+// mantissa of a among them; sqrt_nr with sqrtf on every x in 2^-90 .. 2^90: no
+// difference.)
+__device__ __forceinline__ float recip_nr(float b) {
+  const float r = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float div_nr(float a, float b, float r) {
+  float q = a * r;
+  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+}
+// sqrt(x), correctly rounded, for x within 2^-96 .. 2^96: Goldschmidt steps from
+// the hardware's reciprocal square root, then a residual correction.
+__device__ __forceinline__ float sqrt_nr(float x) {
+  const float r = __builtin_amdgcn_rsqf(x);
+  float g = x * r, h = 0.5f * r;
+  const float e = __builtin_fmaf(-h, g, 0.5f);
+  g = __builtin_fmaf(g, e, g);
+  h = __builtin_fmaf(h, e, h);
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+
+// Pixel and camera distance of one voxel (tsdf.cu:301-318) at camera
+// coordinates vc: the pixel's index, or -1 outside the image.
+__device__ __forceinline__ int voxel_pixel(const Intr &s, f3 vc, float &dist) {
   int pu, pv;
   project(vc, s, pu, pv);
-  if (!(pu >= 0 && pv >= 0 && pu < s.cols && pv < s.rows)) return old;
-  const int idx = pv * s.cols + pu;
+  dist = norm(mk(0.f, 0.f, 0.f) - vc);
+  return pu >= 0 && pv >= 0 && pu < s.cols && pv < s.rows ? pv * s.cols + pu : -1;
+}
+// The same values where every operand is of ordinary size: the quotients share
+// one reciprocal, and roundf(x) for the pixels that matter is trunc(x +
+// pred(1/2)) with the image test on that sum (x = -1/2, which rounds to -1,
+// gives a negative sum).
+constexpr float kOrdLo = 0x1p-40f, kOrdHi = 0x1p40f;
+__device__ __forceinline__ bool ordinary(const Intr &s, f3 vc) {
+  return (vc.z > kOrdLo) & (fmaxf(fmaxf(fabsf(s.fx * vc.x), fabsf(s.fy * vc.y)),
+                                  vc.x * vc.x + vc.y * vc.y + vc.z * vc.z) < kOrdHi);
+}
+__device__ __forceinline__ int voxel_pixel_ord(const Intr &s, float rows, float cols, f3 vc, float &dist) {
+  const float half = 0x1.fffffep-2f;
+  const float r = recip_nr(vc.z);
+  const float su = (div_nr(s.fx * vc.x, vc.z, r) + s.cx) + half, sv = (div_nr(s.fy * vc.y, vc.z, r) + s.cy) + half;
+  dist = sqrt_nr(vc.x * vc.x + vc.y * vc.y + vc.z * vc.z);
+  const bool in = (su >= 0.f) & (sv >= 0.f) & (su < cols) & (sv < rows);
+  return in ? (int)sv * s.cols + (int)su : -1;
+}
+
+// One voxel's update (tsdf.cu:319-341) at camera distance vox with the pixel's
+// record sp (idx < 0: no pixel): the new voxel word, the old one when it is not
+// updated.  col: some colour of the wavefront's voxel or pixel is set.
+__device__ __forceinline__ uint64_t integrate_voxel(float tau, float max_weight, int idx, float vox, uint64_t sp,
+                                                    uint64_t old, bool col) {
   // |getPoint3d(pu, pv, d)| from the allocation pass, sign bit set when
   // d == max_depth (no band update); NaN when d is out of [min_depth,
   // max_depth] or NaN, where the reference's comparisons all fail and the
   // voxel keeps its value
-  const uint64_t sp = ldg((const uint64_t *)(v.surf + idx));
   const float sv = __uint_as_float((uint32_t)sp);
   const uint32_t prgb = (uint32_t)(sp >> 32);
-  if (sv != sv) return old;
   const float surf = fabsf(sv);
-  const float vox = norm(mk(0.f, 0.f, 0.f) - vc);
-  float nsdf;
-  if (vox > surf - tau && vox < surf + tau && !signbit(sv)) nsdf = surf - vox;
-  else if (vox < surf - tau) nsdf = tau;
-  else return old;
-  const uint32_t nr = prgb & 0xff, ng = (prgb >> 8) & 0xff, nb = (prgb >> 16) & 0xff;
+  const bool band = (vox > surf - tau) & (vox < surf + tau) & !signbit(sv);
+  const bool upd = (idx >= 0) & (band | (vox < surf - tau));
+  const float nsdf = band ? surf - vox : tau;
   const uint32_t rgbw = vox_rgbw(old);
-  const uint32_t wi = rgbw >> 24;
-  const float w = (float)wi;
-  const float sdf = (vox_sdf(old) * w + nsdf * 1.0f) / (w + 1.0f);
-  const float rm = __builtin_amdgcn_rcpf((float)(wi + 1u));
-  const uint32_t cr = merge_channel(rgbw & 0xff, wi, nr, rm);
-  const uint32_t cg = merge_channel((rgbw >> 8) & 0xff, wi, ng, rm);
-  const uint32_t cb = merge_channel((rgbw >> 16) & 0xff, wi, nb, rm);
-  int nw = (int)wi + 1;
-  if (nw > v.max_weight) nw = v.max_weight;
-  const uint32_t nrgbw = cr | (cg << 8) | (cb << 16) | ((uint32_t)nw << 24);
-  return ((uint64_t)nrgbw << 32) | (uint64_t)__float_as_uint(sdf);
+  const float w = (float)(rgbw >> 24), m = w + 1.0f;
+  const float num = vox_sdf(old) * w + nsdf * 1.0f;
+  const float rm = __builtin_amdgcn_rcpf(m);
+  float sdf = div_nr(num, m, __builtin_fmaf(__builtin_fmaf(-m, rm, 1.0f), rm, rm));
+  const bool odd = !(fabsf(num) > 0x1p-80f) | !(fabsf(num) < 0x1p80f);
+  if (__ballot(odd)) {  // also exact zeros: rare
+    if (odd) sdf = num / m;
+  }
+  uint32_t nrgbw = (uint32_t)fminf(m, max_weight) << 24;
+  if (col) {  // colour 0 merged with colour 0 stays 0
+    const uint32_t cr = (uint32_t)merge_channel((float)(rgbw & 0xff), w, (float)(prgb & 0xff), rm);
+    const uint32_t cg = (uint32_t)merge_channel((float)((rgbw >> 8) & 0xff), w, (float)((prgb >> 8) & 0xff), rm);
+    const uint32_t cb = (uint32_t)merge_channel((float)((rgbw >> 16) & 0xff), w, (float)((prgb >> 16) & 0xff), rm);
+    nrgbw |= cr | (cg << 8) | (cb << 16);
+  }
+  return upd ? ((uint64_t)nrgbw << 32) | (uint64_t)__float_as_uint(sdf) : old;
 }
 
 // Far threshold of the raycast's empty-space test: a sample whose voxels all
@@ -460,55 +512,144 @@ template <int S> __device__ __forceinline__ bool nbr_side(int x, int side, int &
   return c1 != c0;
 }
 
+// A wavefront takes a chunk of blocks, one lane per block for what concerns a
+// whole block (freed, the reference's block-centre cull, its old empty-space
+// bits), then walks the visible ones.  A block has two dependent loads, its
+// words and its pixels' records; the next block's words are in flight while
+// this one's voxels are updated.  Straight code for ordinary operands, decided
+// once per block, lets those loads stay in flight (a branch per voxel made the
+// wavefront wait for all of them).
+// Bound by those latencies and the bytes: 16 sessions 365 -> 244 us (855 MB:
+// 3.5 TB/s), 640x480 / 8 mm 45 -> 33 us, 4 mm 328 -> 219 us, 320x240 / 2 cm
+// 13.5 -> 9.4 us.  Before, a workgroup took a block, every wavefront
+// repeated its tests, each voxel its whole transform and two IEEE divisions
+// (1418 VALU instructions per wavefront of the 16-session launch, now 892).
 __global__ __launch_bounds__(256) void k_integrate(const DmView *__restrict__ views, const int *__restrict__ active) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
-  const int nalloc = v.ctr[C_NUM_ALLOC];
+  const int nalloc = ldg(v.ctr + C_NUM_ALLOC);
   const Intr s = intr_of(v);
-  const M4 Ti = load_m4(v.posef + PF_TINV);
+  const M4 Ti = load_m4g(v.posef + PF_TINV);
   const float vs = v.voxel_size, tau = v.trunc;
   const double half = 0.5 * (double)vs * 8.0;
   const float far_thr = far_threshold(tau);
+  const float max_weight = (float)v.max_weight, rowsf = (float)s.rows, colsf = (float)s.cols;
+  const uint64_t *surf = (const uint64_t *)v.surf;
+  uint64_t *vox = v.vox;
+  uint8_t *blk_near = v.blk_near;
+  const int4 *block_key = v.block_key;
   // the raycast's empty-space bits are rebuilt by k_dilate_near: the coarse
   // map is cleared whole, the bricks where the near blocks of the previous
   // frame set bits (whole records: k_dilate_near sets every bit again that a
   // block still near asks for)
-  for (int w = blockIdx.x * 256 + threadIdx.x; w < kCoarseWords; w += gridDim.x * 256) v.coarse[w] = 0u;
+  for (int w = blockIdx.x * 256 + threadIdx.x; w < kCoarseWords; w += gridDim.x * 256) stg(v.coarse + w, 0u);
+  const int lane = threadIdx.x & 63;
+  const int nwave = gridDim.x * 4, wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chunk = min(64, (nalloc + nwave - 1) / nwave);  // blocks of the wavefront at a time
   int nvis = 0;
-  for (int blk = blockIdx.x; blk < nalloc; blk += gridDim.x) {
-    const int4 key = v.block_key[blk];
-    if (key.w == 0) continue;  // freed pool index (uniform per workgroup)
-    if (threadIdx.x < 8 && v.blk_near[blk]) {
-      const int e = threadIdx.x;
-      int xl, xh, yl, yh, zl, zh;
-      if (nbr_side<2>(key.x, e & 1, xl, xh) && nbr_side<2>(key.y, (e >> 1) & 1, yl, yh) &&
-          nbr_side<2>(key.z, e >> 2, zl, zh))
-        v.bricks[brick_index(xl, yl, zl)] = make_ulonglong2(0ull, 0ull);
+  for (int base = wave * chunk; base < nalloc; base += nwave * chunk) {
+    const int blk = base + lane;
+    int kx = 0, ky = 0, kz = 0;
+    bool vis = false, was_near = false;
+    if (lane < chunk && blk < nalloc) {
+      const i32x4 key = ldg(reinterpret_cast<const i32x4 *>(block_key) + blk);
+      was_near = ldg(blk_near + blk) != 0;
+      kx = key.x; ky = key.y; kz = key.z;
+      vis = key.w != 0;  // 0: freed pool index
+      was_near = was_near && vis;
     }
-    const f3 pos = mk((float)key.x * vs * 8.0f, (float)key.y * vs * 8.0f, (float)key.z * vs * 8.0f);
-    const f3 pc = xform(Ti, pos);
-    if (pc.z < 0) continue;
+    const f3 pc = xform(Ti, mk((float)kx * vs * 8.0f, (float)ky * vs * 8.0f, (float)kz * vs * 8.0f));
     const f3 bc = mk((float)((double)pc.x + half), (float)((double)pc.y + half), (float)((double)pc.z + half));
     int iu, iv;
     project(bc, s, iu, iv);
-    if (!(iu >= 0 && iv >= 0 && iu < s.cols && iv < s.rows)) continue;
-    ++nvis;
-    uint64_t *bv = v.vox + (size_t)blk * kBlockVox;
-    bool near = false;
+    vis = vis && !(pc.z < 0) && iu >= 0 && iv >= 0 && iu < s.cols && iv < s.rows;
+    unsigned long long todo = __ballot(vis), nearm = 0ull;
+    nvis += __popcll(todo);
+    u64 nxt[8];
+    auto fetch = [&](int q) {
+      const u64 *w = vox + (size_t)(base + q) * kBlockVox + lane;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int t = threadIdx.x + 256 * h;
-      const uint64_t old = bv[t];
-      const uint64_t nword = integrate_voxel(v, s, Ti, pos, t, old);
-      if (nword != old) bv[t] = nword;
-      near |= (nword >> 56) != 0 && vox_sdf(nword) < far_thr;
+      for (int x = 0; x < 8; ++x) nxt[x] = ldg(w + 64 * x);
+    };
+    if (todo) fetch(__builtin_ctzll(todo));
+    if (was_near)
+      for (int e = 0; e < 8; ++e) {
+        int xl, xh, yl, yh, zl, zh;
+        if (nbr_side<2>(kx, e & 1, xl, xh) && nbr_side<2>(ky, (e >> 1) & 1, yl, yh) &&
+            nbr_side<2>(kz, e >> 2, zl, zh))
+          stg(reinterpret_cast<u64x2 *>(v.bricks) + brick_index(xl, yl, zl), u64x2{0ull, 0ull});
+      }
+    while (todo) {
+      const int q = __builtin_ctzll(todo);
+      todo &= todo - 1ull;
+      const float bx = (float)__builtin_amdgcn_readlane(kx, q) * vs * 8.0f;
+      const float by = (float)__builtin_amdgcn_readlane(ky, q) * vs * 8.0f;
+      const float bz = (float)__builtin_amdgcn_readlane(kz, q) * vs * 8.0f;
+      u64 *bv = vox + (size_t)(base + q) * kBlockVox + lane;
+      const float py = by + (float)(lane >> 3) * vs, pz = bz + (float)(lane & 7) * vs;
+      // xform's products with y and z
+      const float xy = Ti.m[1] * py, xz = Ti.m[2] * pz, yy = Ti.m[5] * py, yz = Ti.m[6] * pz, zy = Ti.m[9] * py,
+                  zz = Ti.m[10] * pz;
+      auto camera = [&](int x) {
+        const float px = bx + (float)x * vs;
+        return mk(Ti.m[0] * px + xy + xz + Ti.m[3], Ti.m[4] * px + yy + yz + Ti.m[7],
+                  Ti.m[8] * px + zy + zz + Ti.m[11]);
+      };
+      // every rounded operation above is monotone in x, so a camera
+      // coordinate lies between its values at the row's ends: ordinary there is
+      // ordinary along the row
+      const bool ord = __ballot(!(ordinary(s, camera(0)) & ordinary(s, camera(7)))) == 0ull;
+      bool near = false;
+      if (ord) {
+        u64 sp[8];
+        int idx[8];
+        float dist[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) idx[x] = voxel_pixel_ord(s, rowsf, colsf, camera(x), dist[x]);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) sp[x] = ldg(surf + max(idx[x], 0));
+        u64 old[8];
+        uint32_t any = 0u;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          old[x] = nxt[x];
+          any |= (uint32_t)(old[x] >> 32) & 0xffffffu;
+        }
+        if (todo) fetch(__builtin_ctzll(todo));
+#pragma unroll
+        for (int x = 0; x < 8; ++x) any |= (uint32_t)(sp[x] >> 32);
+        const bool col = __ballot(any != 0u) != 0ull;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          const u64 nword = integrate_voxel(tau, max_weight, idx[x], dist[x], sp[x], old[x], col);
+          if (nword != old[x]) stg(bv + 64 * x, nword);
+          near |= (nword >> 56) != 0 && vox_sdf(nword) < far_thr;
+        }
+      } else {
+#pragma unroll 1
+        for (int x = 0; x < 8; ++x) {
+          const u64 old = ldg(bv + 64 * x);
+          float dist;
+          const int idx = voxel_pixel(s, camera(x), dist);
+          const u64 nword = integrate_voxel(tau, max_weight, idx, dist, ldg(surf + max(idx, 0)), old, true);
+          if (nword != old) stg(bv + 64 * x, nword);
+          near |= (nword >> 56) != 0 && vox_sdf(nword) < far_thr;
+        }
+        if (todo) fetch(__builtin_ctzll(todo));
+      }
+      // block summary used by the raycast's empty-space test
+      if (__ballot(near) != 0ull) nearm |= 1ull << q;
     }
-    // block summary used by the raycast's empty-space test
-    near = __syncthreads_or(near);
-    if (threadIdx.x == 0) v.blk_near[blk] = near ? 1 : 0;
+    if (vis) stg(blk_near + blk, (uint8_t)((nearm >> lane) & 1ull));
   }
-  if (threadIdx.x == 0 && nvis) atomicAdd(&v.ctr[C_NVIS], nvis);
+  __shared__ int vis_sum[4];
+  if (lane == 0) vis_sum[threadIdx.x >> 6] = nvis;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int n = vis_sum[0] + vis_sum[1] + vis_sum[2] + vis_sum[3];
+    if (n) atomicAdd(&v.ctr[C_NVIS], n);
+  }
 }
 
 // Rebuild the raycast's empty-space bits from the near blocks (after the
@@ -1076,7 +1217,6 @@ __device__ __forceinline__ void hit_stencil(const DmView &v, const AxisSample &X
 // widened by a margin far larger than its error, so it is conservative: a
 // sample it calls far is far for the exact evaluation too.
 // Record of a brick: x = dilated bits, y = near bits.
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u64x2 load_brick(const DmView &v, uint32_t b) {
   return ldg(reinterpret_cast<const u64x2 *>(v.bricks) + b);
 }

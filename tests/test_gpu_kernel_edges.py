@@ -92,3 +92,51 @@ def test_icp_step_record_counts(rows, cols, variant):
     assert np.linalg.norm(host[:3, 3]) > 1e-4
     for T in dev:
         np.testing.assert_allclose(T, host, rtol=0, atol=1e-12)
+
+
+# The integration's wavefronts take chunks of the pool: one workgroup (64
+# blocks per wavefront and round), an odd number, and more wavefronts than
+# blocks give the same poses, bit for bit.
+def test_integration_chunks():
+    depth, _, poses = configs.make_sequence("rigid-320x240-2cm", 4)
+    w = configs.WORKLOADS["rigid-320x240-2cm"]
+    got = []
+    for wg in (1, 3, 2048, 4096):
+        srv = dm.Server(1, 240, 320)
+        srv.add_trace(w["tsdf"], w["icp"], w["sensor"], poses[0], depth)
+        srv.set_shapes(integrate_workgroups=wg)
+        got.append(srv.run(0, 0, 4, want_poses=True)["poses"])
+        srv.close()
+    for g in got[1:]:
+        np.testing.assert_array_equal(g, got[0])
+
+
+# Integration against the FP32 transcription where the straight code's range
+# ends: a camera turned about its own axis inside blocks it has mapped (blocks
+# that cross the camera plane), and voxels of 2e-9 m and 1e4 m, whose squared
+# distances leave the range at one end.
+@pytest.mark.parametrize("scale", [1.0, 1e-7, 5e5])
+def test_integration_operand_range(room, scale):
+    import oracle_lib as O
+    depth, poses = room
+    base = small_tsdf()
+    props = dict(base, voxel_size=base["voxel_size"] * scale, truncation_distance=base["truncation_distance"] * scale,
+                 max_sensor_depth=base["max_sensor_depth"] * scale, min_sensor_depth=base["min_sensor_depth"] * scale)
+    vol = dm.TsdfVolume(props, SENS["rows"], SENS["cols"])
+    ora = O.OracleVolume(props, 32)
+    for f, yaw in enumerate((0.0, 0.7, -0.9)):
+        c, s = np.cos(yaw), np.sin(yaw)
+        R = np.eye(4)
+        R[:3, :3] = [[c, 0, s], [0, 1, 0], [-s, 0, c]]
+        T = (poses[0] @ R).astype(np.float64)
+        T[:3, 3] *= scale
+        Tf, d = T.astype(np.float32), (depth[f] * np.float32(scale)).astype(np.float32)
+        vol.IntegrateScan(d, None, SENS, Tf)
+        ora.integrate_scan(d, None, SENS, Tf.astype(np.float64))
+    gx, gs, _, gw = vol.blocks()
+    ox, os_, _, ow = ora.blocks()
+    gi, oi = np.lexsort(gx.T[::-1]), np.lexsort(ox.T[::-1])
+    np.testing.assert_array_equal(gx[gi], ox[oi])
+    np.testing.assert_array_equal(gw[gi], ow[oi])
+    np.testing.assert_array_equal(gs[gi], os_[oi].astype(np.float32))
+    assert (gw > 0).any()
