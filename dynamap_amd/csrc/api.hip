@@ -135,7 +135,7 @@ int Sess::init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols) {
   DM_TRY(dalloc(&d_ray_rgb, P * 3));
   DM_TRY(dalloc(&d_view, 1));
   DM_TRY(dalloc(&d_active, 1));
-  pinned_bytes = P * 7 + 64;
+  pinned_bytes = P * 7 + 1024;
   DM_HIP(hipHostMalloc((void **)&h_pinned, pinned_bytes, hipHostMallocDefault));
   // identity poses
   double I[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
@@ -151,7 +151,8 @@ int Sess::init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols) {
   h.dist_max = 0.1f; h.w_photo = 0.f; h.lambda = 0.02f; h.max_inc = 0.3f;
   int zero = 0;
   DM_HIP(hipMemcpyAsync(d_active, &zero, sizeof(int), hipMemcpyHostToDevice, stream));
-  DM_TRY(push_view());
+  push_view();
+  DM_HIP(hipGetLastError());
   DM_HIP(hipStreamSynchronize(stream));
   return DM_OK;
 }
@@ -162,16 +163,15 @@ void Sess::release() {
   allocs.clear();
   if (h_pinned) hipHostFree(h_pinned);
   h_pinned = nullptr;
+  for (hipEvent_t &e : ev_out) {
+    if (e) hipEventDestroy(e);
+    e = nullptr;
+  }
   if (stream) hipStreamDestroy(stream);
   stream = nullptr;
 }
 
-int Sess::push_view() {
-  DM_HIP(hipMemcpyAsync(d_view, &h, sizeof(DmView), hipMemcpyHostToDevice, stream));
-  // the host copy may change before the copy runs: wait for it
-  DM_HIP(hipStreamSynchronize(stream));
-  return DM_OK;
-}
+void Sess::push_view(const float *pose) { launch_set_view(d_view, h, pose, stream); }
 
 Launch Sess::launch() const {
   Launch L;
@@ -199,30 +199,70 @@ int Sess::set_sensor(const dm_sensor *s) {
   return DM_OK;
 }
 
-int Sess::set_pose_f(const float pose[16]) {
-  float pf[32];
-  double pd[16];
-  for (int k = 0; k < 16; ++k) { pf[k] = pose[k]; pd[k] = (double)pose[k]; }
-  rigid_inverse_ff(pose, pf + 16);
-  DM_HIP(hipMemcpyAsync(h.posef + PF_T, pf, 32 * sizeof(float), hipMemcpyHostToDevice, stream));
-  DM_HIP(hipMemcpyAsync(h.posed + PD_T, pd, 16 * sizeof(double), hipMemcpyHostToDevice, stream));
+// The view (and pose) of a frame that is about to be staged: the staging
+// buffers are the session's own, so the view is known before the copies.  A
+// call that staged a frame has waited for it before it returned, so the pinned
+// buffer is free unless a call failed halfway.
+int Sess::frame_from_host(const float *host_depth, const uint8_t *host_rgb, const float *pose) {
+  DM_HIP(hipStreamSynchronize(stream));
+  h.depth = d_depth;
+  h.rgb = host_rgb ? d_rgb : nullptr;
+  push_view(pose);
+  return DM_OK;
+}
+int Sess::stage_depth(const float *host_depth) {
+  const size_t P = (size_t)h.rows * h.cols;
+  memcpy(h_pinned, host_depth, P * 4);
+  DM_HIP(hipMemcpyAsync(d_depth, h_pinned, P * 4, hipMemcpyHostToDevice, stream));
+  return DM_OK;
+}
+int Sess::stage_rgb(const uint8_t *host_rgb) {
+  if (!host_rgb) return DM_OK;
+  const size_t P = (size_t)h.rows * h.cols;
+  memcpy(h_pinned + P * 4, host_rgb, P * 3);
+  DM_HIP(hipMemcpyAsync(d_rgb, h_pinned + P * 4, P * 3, hipMemcpyHostToDevice, stream));
+  return DM_OK;
+}
+
+int Sess::reserve_out() {
+  const size_t P = (size_t)max_rows * max_cols;
+  if (!d_pack) DM_TRY(dalloc(&d_pack, P * 7, false));
+  for (hipEvent_t &e : ev_out)
+    if (!e) DM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return DM_OK;
+}
+
+// The results pass through the two halves of the frame's pinned buffer: while
+// one chunk is moved to the caller's memory, the next is on its way.
+int Sess::read_out(const Out *out, int n) {
+  const size_t half = ((size_t)max_rows * max_cols * 7 / 2 + 63) & ~(size_t)63;
+  struct Chunk { uint8_t *dst; const uint8_t *src; size_t bytes; };
+  std::vector<Chunk> chunks;
+  for (int k = 0; k < n; ++k)
+    for (size_t o = 0; o < out[k].bytes; o += half)
+      chunks.push_back({(uint8_t *)out[k].dst + o, (const uint8_t *)out[k].src + o, std::min(half, out[k].bytes - o)});
+  auto issue = [&](size_t c) -> int {
+    if (c >= chunks.size()) return DM_OK;
+    DM_HIP(hipMemcpyAsync(h_pinned + (c & 1) * half, chunks[c].src, chunks[c].bytes, hipMemcpyDeviceToHost, stream));
+    DM_HIP(hipEventRecord(ev_out[c & 1], stream));
+    return DM_OK;
+  };
+  DM_TRY(issue(0));
+  DM_TRY(issue(1));
+  for (size_t c = 0; c < chunks.size(); ++c) {
+    DM_HIP(hipEventSynchronize(ev_out[c & 1]));
+    memcpy(chunks[c].dst, h_pinned + (c & 1) * half, chunks[c].bytes);
+    DM_TRY(issue(c + 2));
+  }
   DM_HIP(hipStreamSynchronize(stream));
   return DM_OK;
 }
 
-int Sess::stage_frame(const float *host_depth, const uint8_t *host_rgb) {
-  const size_t P = (size_t)h.rows * h.cols;
+int Sess::read_small(void *dst, const void *src, size_t bytes) {
+  uint8_t *slot = h_pinned + (((size_t)max_rows * max_cols * 7 + 191) & ~(size_t)63);  // past both halves
+  DM_HIP(hipMemcpyAsync(slot, src, bytes, hipMemcpyDeviceToHost, stream));
   DM_HIP(hipStreamSynchronize(stream));
-  memcpy(h_pinned, host_depth, P * 4);
-  DM_HIP(hipMemcpyAsync(d_depth, h_pinned, P * 4, hipMemcpyHostToDevice, stream));
-  h.depth = d_depth;
-  if (host_rgb) {
-    memcpy(h_pinned + P * 4, host_rgb, P * 3);
-    DM_HIP(hipMemcpyAsync(d_rgb, h_pinned + P * 4, P * 3, hipMemcpyHostToDevice, stream));
-    h.rgb = d_rgb;
-  } else {
-    h.rgb = nullptr;
-  }
+  memcpy(dst, slot, bytes);
   return DM_OK;
 }
 
@@ -294,11 +334,16 @@ static int run_icp(Sess &S, bool host_solve) {
   return DM_OK;
 }
 
-static int process_frame(Sess &S, bool host_solve, double *pose_out) {
+// One frame whose view is set.  Host inputs (host_depth non-null) are staged
+// here: the filter, which needs the depth alone, runs while the colour is copied.
+static int process_frame(Sess &S, const float *host_depth, const uint8_t *host_rgb, bool host_solve,
+                         double *pose_out) {
   const Launch L = S.launch();
+  launch_pose_begin(L);
+  if (host_depth) DM_TRY(S.stage_depth(host_depth));
   if (S.filt_r > 0)
     launch_bilateral(S.h.depth, S.d_depth_f, S.h.rows, S.h.cols, S.filt_r, S.filt_sd, S.filt_ss, S.stream);
-  launch_pose_begin(L);
+  if (host_depth) DM_TRY(S.stage_rgb(host_rgb));
   launch_source_maps(L);
   DM_TRY(run_icp(S, host_solve));
   launch_alloc(L);
@@ -306,8 +351,7 @@ static int process_frame(Sess &S, bool host_solve, double *pose_out) {
   launch_raycast(L);
   DM_HIP(hipGetLastError());
   double T[16];
-  DM_HIP(hipMemcpyAsync(T, S.h.posed + PD_T, sizeof T, hipMemcpyDeviceToHost, S.stream));
-  DM_HIP(hipStreamSynchronize(S.stream));
+  DM_TRY(S.read_small(T, S.h.posed + PD_T, sizeof T));
   if (pose_out) memcpy(pose_out, T, sizeof T);
   S.frames++;
   return DM_OK;
@@ -385,9 +429,9 @@ static int volume_frame(dm_volume *vol, const float *depth, const uint8_t *rgb, 
                         const float pose[16], bool integrate) {
   if (!vol || !depth || !pose) { set_error("null argument"); return DM_E_INVALID; }
   DM_TRY(vol->set_sensor(sensor));
-  DM_TRY(vol->stage_frame(depth, rgb));
-  DM_TRY(vol->set_pose_f(pose));
-  DM_TRY(vol->push_view());
+  DM_TRY(vol->frame_from_host(depth, rgb, pose));
+  DM_TRY(vol->stage_depth(depth));
+  DM_TRY(vol->stage_rgb(rgb));
   const Launch L = vol->launch();
   launch_alloc(L);
   if (integrate) launch_integrate(L);
@@ -409,35 +453,29 @@ int dm_volume_raycast(dm_volume *vol, const float pose[16], const dm_sensor *sen
                       float *host_vertex, float *host_normal, uint8_t *host_rgb) {
   if (!vol || !pose) { set_error("null argument"); return DM_E_INVALID; }
   DM_TRY(vol->set_sensor(sensor));
-  DM_TRY(vol->set_pose_f(pose));
-  vol->h.ray_depth = vol->d_ray_depth;
-  vol->h.ray_rgb = vol->d_ray_rgb;
-  DM_TRY(vol->push_view());
-  launch_raycast(vol->launch());
-  vol->h.ray_depth = nullptr;
-  vol->h.ray_rgb = nullptr;
-  DM_HIP(hipGetLastError());
+  DM_TRY(vol->reserve_out());
+  vol->push_view(pose);
+  Launch L = vol->launch();
+  L.ray_depth = vol->d_ray_depth;
+  L.ray_rgb = vol->d_ray_rgb;
+  launch_raycast(L);
   const size_t P = (size_t)vol->h.rows * vol->h.cols;
-  std::vector<float4> vt(P), nt(P);
-  DM_HIP(hipMemcpyAsync(vt.data(), vol->h.tvert[0], P * 16, hipMemcpyDeviceToHost, vol->stream));
-  DM_HIP(hipMemcpyAsync(nt.data(), vol->h.tnorm[0], P * 16, hipMemcpyDeviceToHost, vol->stream));
-  if (host_depth)
-    DM_HIP(hipMemcpyAsync(host_depth, vol->d_ray_depth, P * 4, hipMemcpyDeviceToHost, vol->stream));
-  if (host_rgb) DM_HIP(hipMemcpyAsync(host_rgb, vol->d_ray_rgb, P * 3, hipMemcpyDeviceToHost, vol->stream));
-  DM_HIP(hipStreamSynchronize(vol->stream));
-  DM_TRY(vol->push_view());
-  for (size_t i = 0; i < P; ++i) {
-    if (host_vertex) { host_vertex[3 * i] = vt[i].x; host_vertex[3 * i + 1] = vt[i].y; host_vertex[3 * i + 2] = vt[i].z; }
-    if (host_normal) { host_normal[3 * i] = nt[i].x; host_normal[3 * i + 1] = nt[i].y; host_normal[3 * i + 2] = nt[i].z; }
-  }
-  return DM_OK;
+  float *v3 = host_vertex ? vol->d_pack : nullptr, *n3 = host_normal ? vol->d_pack + 3 * P : nullptr;
+  if (v3 || n3) launch_pack_maps(vol->h.tvert[0], vol->h.tnorm[0], (int)P, v3, n3, nullptr, vol->stream);
+  DM_HIP(hipGetLastError());
+  Sess::Out out[4];
+  int n = 0;
+  if (host_vertex) out[n++] = {host_vertex, v3, P * 12};
+  if (host_normal) out[n++] = {host_normal, n3, P * 12};
+  if (host_depth) out[n++] = {host_depth, vol->d_ray_depth, P * 4};
+  if (host_rgb) out[n++] = {host_rgb, vol->d_ray_rgb, P * 3};
+  return vol->read_out(out, n);
 }
 
 int dm_volume_num_allocated(dm_volume *vol, int32_t *n) {
   if (!vol || !n) { set_error("null argument"); return DM_E_INVALID; }
   int32_t c[C_COUNT];
-  DM_HIP(hipMemcpyAsync(c, vol->h.ctr, sizeof c, hipMemcpyDeviceToHost, vol->stream));
-  DM_HIP(hipStreamSynchronize(vol->stream));
+  DM_TRY(vol->read_small(c, vol->h.ctr, sizeof c));
   *n = c[C_NUM_ALLOC] - c[C_NUM_FREE];
   return DM_OK;
 }
@@ -654,7 +692,7 @@ int dm_volume_restore(dm_volume *vol, const void *buf, uint64_t size) {
   for (int l = 0; l < 3; ++l) S.h.iters[l] = H.iters[l];
   S.h.icp_dmin = H.icp_f[0]; S.h.icp_dmax = H.icp_f[1]; S.h.dist_max = H.icp_f[2];
   S.h.w_photo = H.icp_f[3]; S.h.lambda = H.icp_f[4]; S.h.max_inc = H.icp_f[5]; S.h.min_inc = H.icp_f[6];
-  DM_TRY(S.push_view());
+  S.push_view();
   rebuild_far_maps(S.launch());
   DM_HIP(hipGetLastError());
   DM_HIP(hipStreamSynchronize(S.stream));
@@ -694,7 +732,11 @@ int dm_session_create(const dm_tsdf_props *props, const dm_icp_props *icp, const
                                   s->stream);
     if (e != hipSuccess) r = hip_fail(e, "hipMemcpyAsync(init pose)");
   }
-  if (r == DM_OK) r = s->push_view();
+  if (r == DM_OK) {
+    s->push_view();
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) r = hip_fail(e, "session view");
+  }
   if (r != DM_OK) { s->release(); delete s; return r; }
   *out = s;
   return DM_OK;
@@ -712,9 +754,8 @@ dm_volume *dm_session_volume(dm_session *s) { return reinterpret_cast<dm_volume 
 int dm_session_process_frame(dm_session *s, const float *host_depth, const uint8_t *host_rgb, int32_t solve_on_host,
                              double pose_out[16]) {
   if (!s || !host_depth) { set_error("null argument"); return DM_E_INVALID; }
-  DM_TRY(s->stage_frame(host_depth, host_rgb));
-  DM_TRY(s->push_view());
-  return process_frame(*s, solve_on_host != 0, pose_out);
+  DM_TRY(s->frame_from_host(host_depth, host_rgb, nullptr));
+  return process_frame(*s, host_depth, host_rgb, solve_on_host != 0, pose_out);
 }
 
 int dm_session_process_frame_dev(dm_session *s, const float *dev_depth, const uint8_t *dev_rgb, int32_t solve_on_host,
@@ -722,8 +763,8 @@ int dm_session_process_frame_dev(dm_session *s, const float *dev_depth, const ui
   if (!s || !dev_depth) { set_error("null argument"); return DM_E_INVALID; }
   s->h.depth = dev_depth;
   s->h.rgb = dev_rgb;
-  DM_TRY(s->push_view());
-  return process_frame(*s, solve_on_host != 0, pose_out);
+  s->push_view();
+  return process_frame(*s, nullptr, nullptr, solve_on_host != 0, pose_out);
 }
 
 int dm_session_set_depth_filter(dm_session *s, int32_t radius, float sigma_depth, float sigma_space) {
@@ -736,36 +777,36 @@ int dm_session_set_depth_filter(dm_session *s, int32_t radius, float sigma_depth
   s->filt_sd = sigma_depth;
   s->filt_ss = sigma_space;
   s->h.depth_track = radius > 0 ? s->d_depth_f : nullptr;
-  DM_TRY(s->push_view());
+  s->push_view();
+  DM_HIP(hipGetLastError());
   DM_HIP(hipStreamSynchronize(s->stream));
   return DM_OK;
 }
 
 int dm_session_get_pose(dm_session *s, double pose[16]) {
   if (!s || !pose) { set_error("null argument"); return DM_E_INVALID; }
-  DM_HIP(hipMemcpyAsync(pose, s->h.posed + PD_T, 16 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-  DM_HIP(hipStreamSynchronize(s->stream));
-  return DM_OK;
+  return s->read_small(pose, s->h.posed + PD_T, 16 * sizeof(double));
 }
 
 int dm_session_source_maps(dm_session *s, const float *host_depth, const uint8_t *host_rgb, int32_t level,
                            float *host_vertex, float *host_normal, float *host_intensity) {
   if (!s || !host_depth || level < 0 || level >= kLevels) { set_error("invalid argument"); return DM_E_INVALID; }
-  DM_TRY(s->stage_frame(host_depth, host_rgb));
-  DM_TRY(s->push_view());
+  DM_TRY(s->reserve_out());
+  DM_TRY(s->frame_from_host(host_depth, host_rgb, nullptr));
+  DM_TRY(s->stage_depth(host_depth));
+  DM_TRY(s->stage_rgb(host_rgb));
   launch_source_maps(s->launch());
-  DM_HIP(hipGetLastError());
   const size_t P = (size_t)(s->h.rows >> level) * (s->h.cols >> level);
-  std::vector<float4> vt(P), nt(P);
-  DM_HIP(hipMemcpyAsync(vt.data(), s->h.svert[level], P * 16, hipMemcpyDeviceToHost, s->stream));
-  DM_HIP(hipMemcpyAsync(nt.data(), s->h.snorm[level], P * 16, hipMemcpyDeviceToHost, s->stream));
-  DM_HIP(hipStreamSynchronize(s->stream));
-  for (size_t i = 0; i < P; ++i) {
-    if (host_vertex) { host_vertex[3 * i] = vt[i].x; host_vertex[3 * i + 1] = vt[i].y; host_vertex[3 * i + 2] = vt[i].z; }
-    if (host_normal) { host_normal[3 * i] = nt[i].x; host_normal[3 * i + 1] = nt[i].y; host_normal[3 * i + 2] = nt[i].z; }
-    if (host_intensity) host_intensity[i] = vt[i].w;
-  }
-  return DM_OK;
+  float *v3 = host_vertex ? s->d_pack : nullptr, *n3 = host_normal ? s->d_pack + 3 * P : nullptr,
+        *it = host_intensity ? s->d_pack + 6 * P : nullptr;
+  if (v3 || n3 || it) launch_pack_maps(s->h.svert[level], s->h.snorm[level], (int)P, v3, n3, it, s->stream);
+  DM_HIP(hipGetLastError());
+  Sess::Out out[3];
+  int n = 0;
+  if (host_vertex) out[n++] = {host_vertex, v3, P * 12};
+  if (host_normal) out[n++] = {host_normal, n3, P * 12};
+  if (host_intensity) out[n++] = {host_intensity, it, P * 4};
+  return s->read_out(out, n);
 }
 
 int dm_session_set_model_maps(dm_session *s, int32_t level, const float *host_vertex, const float *host_normal,
@@ -821,31 +862,18 @@ int dm_session_icp_system(dm_session *s, int32_t level, const double Tinc[16], d
 
 int dm_session_icp_track(dm_session *s, int32_t solve_on_host, double Tinc_out[16]) {
   if (!s) { set_error("null argument"); return DM_E_INVALID; }
-  double pd[PD_COUNT] = {0};
-  for (int k = 0; k < 16; ++k) {
-    const double I = (k % 5 == 0) ? 1.0 : 0.0;
-    pd[PD_T + k] = I; pd[PD_TPREV + k] = I; pd[PD_TINC + k] = I; pd[PD_TINIT + k] = I;
-  }
-  float pf[PF_COUNT];
-  for (int k = 0; k < PF_COUNT; ++k) pf[k] = (k % 16) % 5 == 0 ? 1.f : 0.f;
-  DM_HIP(hipMemcpyAsync(s->h.posed, pd, sizeof pd, hipMemcpyHostToDevice, s->stream));
-  DM_HIP(hipMemcpyAsync(s->h.posef, pf, sizeof pf, hipMemcpyHostToDevice, s->stream));
-  const int one = 1, zero = 0;
-  DM_HIP(hipMemcpyAsync(s->h.ctr + C_HAS_MODEL, &one, 4, hipMemcpyHostToDevice, s->stream));
-  DM_HIP(hipMemcpyAsync(s->h.ctr + C_ICP_STOP, &zero, 4, hipMemcpyHostToDevice, s->stream));
-  DM_HIP(hipStreamSynchronize(s->stream));
+  launch_track_reset(s->h, s->stream);
   DM_TRY(run_icp(*s, solve_on_host != 0));
-  DM_HIP(hipMemcpyAsync(pd, s->h.posed, sizeof pd, hipMemcpyDeviceToHost, s->stream));
-  DM_HIP(hipStreamSynchronize(s->stream));
-  if (Tinc_out) memcpy(Tinc_out, pd + PD_TINC, 16 * sizeof(double));
+  double T[16];
+  DM_TRY(s->read_small(T, s->h.posed + PD_TINC, sizeof T));
+  if (Tinc_out) memcpy(Tinc_out, T, sizeof T);
   return DM_OK;
 }
 
 int dm_session_icp_increment(dm_session *s, double twist[6]) {
   if (!s || !twist) { set_error("null argument"); return DM_E_INVALID; }
   double acc[6];
-  DM_HIP(hipMemcpyAsync(acc, s->h.posed + PD_ACC, sizeof acc, hipMemcpyDeviceToHost, s->stream));
-  DM_HIP(hipStreamSynchronize(s->stream));
+  DM_TRY(s->read_small(acc, s->h.posed + PD_ACC, sizeof acc));
   // gnSolver.cu:426-428: a NaN, infinite or too large sum is replaced by zero
   const double ssum = acc[0] + acc[1] + acc[2] + acc[3] + acc[4] + acc[5];
   const bool reset = ssum != ssum || std::isinf(ssum) || ssum >= (double)s->h.max_inc;

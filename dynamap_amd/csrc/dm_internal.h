@@ -115,9 +115,6 @@ struct DmView {
   float *posef;         // PF_COUNT
   float *partials;      // ICP partial sums: max_wg * kIcpVals
   int max_wg;
-  // optional raycast outputs (level 0), may be null
-  float *ray_depth;
-  uint8_t *ray_rgb;
   // tracking parameters
   int iters[kLevels];
   float icp_dmin, icp_dmax, dist_max, w_photo, lambda, max_inc, min_inc;
@@ -135,6 +132,8 @@ struct Launch {
   int ray_tw_log2 = 4;  // raycast tile: 2^ray_tw_log2 x (256 >> ray_tw_log2) pixels
   int integ_wg = 2048;  // integration workgroups per session
   int icp_mfma = 0;     // ICP linearisation on the matrix cores (k_icp_reduce_mfma) instead of the shuffle tree
+  float *ray_depth = nullptr;  // raycast depth and colour for the host (one session's launches only)
+  uint8_t *ray_rgb = nullptr;
   hipStream_t stream;
 };
 
@@ -161,6 +160,16 @@ void launch_source_maps(const Launch &L);
 // step on the device.
 void launch_icp_reduce(const Launch &L, int level, int it, bool solve);
 void launch_pose_begin(const Launch &L);
+// Store a session's view record and, with pose, its frame pose (T and its
+// inverse): the values travel as kernel arguments, so nothing is staged and
+// nothing is waited for.
+void launch_set_view(DmView *d_view, const DmView &h, const float *pose, hipStream_t st);
+// Identity poses, model present, no converged level: tracking on its own.
+void launch_track_reset(const DmView &h, hipStream_t st);
+// Packed copies of a level's maps for the host: xyz triples (and the
+// intensity), any output may be null.
+void launch_pack_maps(const float4 *vert, const float4 *norm, int n, float *v3, float *n3, float *inten,
+                      hipStream_t st);
 void launch_pose_log(const Launch &L, const int *dest, double *log);
 void launch_bilateral(const float *in, float *out, int rows, int cols, int r, float sigma_d, float sigma_s,
                       hipStream_t st);

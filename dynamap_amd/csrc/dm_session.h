@@ -43,6 +43,8 @@ struct Sess {
   size_t pinned_bytes = 0;
   float *d_ray_depth = nullptr;  // raycast outputs for host readback
   uint8_t *d_ray_rgb = nullptr;
+  float *d_pack = nullptr;       // packed maps for host readback (7 floats per pixel, allocated on first use)
+  hipEvent_t ev_out[2] = {nullptr, nullptr};
   float *d_depth_f = nullptr;    // bilateral-filtered depth for tracking (when enabled)
   int filt_r = 0;                // filter radius, 0 = off
   int icp_mfma = 0;              // ICP linearisation on the matrix cores (dm_session_set_icp_reduce)
@@ -53,11 +55,16 @@ struct Sess {
   int init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols);
   void release();
   template <class T> int dalloc(T **ptr, size_t count, bool zero = true);
-  int push_view();               // copy h to d_view (async on stream)
+  void push_view(const float *pose = nullptr);  // store h (and the frame pose) on the device, in stream order
   Launch launch() const;
   int set_sensor(const dm_sensor *s);
-  int set_pose_f(const float pose[16]);   // T and Tinv (float), T in double too
-  int stage_frame(const float *host_depth, const uint8_t *host_rgb);
+  int stage_depth(const float *host_depth);  // upload the frame through pinned memory; h.depth / h.rgb are set
+  int stage_rgb(const uint8_t *host_rgb);    // by frame_from_host
+  int frame_from_host(const float *host_depth, const uint8_t *host_rgb, const float *pose);
+  int reserve_out();
+  struct Out { void *dst; const void *src; size_t bytes; };
+  int read_out(const Out *out, int n);       // device results to host memory; waits
+  int read_small(void *dst, const void *src, size_t bytes);  // up to 1 KiB; waits for the stream
 };
 
 // bytes of device memory a session with these parameters needs

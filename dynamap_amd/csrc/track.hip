@@ -606,6 +606,66 @@ __global__ void k_pose_begin(const DmView *__restrict__ views, const int *__rest
   v.ctr[C_NVISIT] = 0;
 }
 
+struct PoseArg { float T[16], Ti[16]; };
+__global__ __launch_bounds__(256) void k_set_view(DmView *__restrict__ dst, DmView h, PoseArg p, int set_pose) {
+  const int t = threadIdx.x;
+  static_assert(sizeof(DmView) % 8 == 0 && sizeof(DmView) / 8 <= 256, "one word per thread");
+  if (t < (int)(sizeof(DmView) / 8)) ((uint64_t *)dst)[t] = ((const uint64_t *)&h)[t];
+  if (set_pose && t < 16) {
+    h.posef[PF_T + t] = p.T[t];
+    h.posef[PF_TINV + t] = p.Ti[t];
+    h.posed[PD_T + t] = (double)p.T[t];
+  }
+}
+void launch_set_view(DmView *d_view, const DmView &h, const float *pose, hipStream_t st) {
+  PoseArg p{};
+  if (pose) {
+    for (int k = 0; k < 16; ++k) p.T[k] = pose[k];
+    rigid_inverse_ff(p.T, p.Ti);
+  }
+  hipLaunchKernelGGL(k_set_view, dim3(1), dim3(256), 0, st, d_view, h, p, pose ? 1 : 0);
+}
+
+__global__ __launch_bounds__(128) void k_track_reset(double *__restrict__ posed, float *__restrict__ posef,
+                                                     int32_t *__restrict__ ctr) {
+  const int t = threadIdx.x;
+  if (t < PD_COUNT) {
+    const bool mat = t < PD_ACC || (t >= PD_TINIT && t < PD_PERSIST);
+    posed[t] = mat && (t & 15) % 5 == 0 ? 1.0 : 0.0;
+  }
+  if (t < PF_COUNT) posef[t] = (t & 15) % 5 == 0 ? 1.f : 0.f;
+  if (t == 0) {
+    ctr[C_HAS_MODEL] = 1;
+    ctr[C_ICP_STOP] = 0;
+  }
+}
+void launch_track_reset(const DmView &h, hipStream_t st) {
+  static_assert(PD_T % 16 == 0 && PD_TPREV % 16 == 0 && PD_TINC % 16 == 0 && PD_TINIT % 16 == 0 && PD_COUNT <= 128,
+                "matrices at multiples of 16");
+  hipLaunchKernelGGL(k_track_reset, dim3(1), dim3(128), 0, st, h.posed, h.posef, h.ctr);
+}
+
+__global__ __launch_bounds__(256) void k_pack_maps(const float4 *__restrict__ vert, const float4 *__restrict__ norm,
+                                                   int n, float *__restrict__ v3, float *__restrict__ n3,
+                                                   float *__restrict__ inten) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  if (v3 || inten) {
+    const float4 a = vert[i];
+    if (v3) { v3[3 * i] = a.x; v3[3 * i + 1] = a.y; v3[3 * i + 2] = a.z; }
+    if (inten) inten[i] = a.w;
+  }
+  if (n3) {
+    const float4 a = norm[i];
+    n3[3 * i] = a.x; n3[3 * i + 1] = a.y; n3[3 * i + 2] = a.z;
+  }
+}
+void launch_pack_maps(const float4 *vert, const float4 *norm, int n, float *v3, float *n3, float *inten,
+                      hipStream_t st) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_pack_maps, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, vert, norm, n, v3, n3, inten);
+}
+
 void launch_source_maps(const Launch &L) {
   if (L.nact <= 0) return;
   const int tot = L.max_pixels + L.max_pixels / 4 + L.max_pixels / 16 + 2;

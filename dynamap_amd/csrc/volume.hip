@@ -420,8 +420,9 @@ __device__ __forceinline__ int voxel_pixel(const Intr &s, f3 vc, float &dist) {
 // gives a negative sum).
 constexpr float kOrdLo = 0x1p-40f, kOrdHi = 0x1p40f;
 __device__ __forceinline__ bool ordinary(const Intr &s, f3 vc) {
-  return (vc.z > kOrdLo) & (fmaxf(fmaxf(fabsf(s.fx * vc.x), fabsf(s.fy * vc.y)),
-                                  vc.x * vc.x + vc.y * vc.y + vc.z * vc.z) < kOrdHi);
+  // bitwise: no branch between the tests
+  return (int)(vc.z > kOrdLo) & (int)(fmaxf(fmaxf(fabsf(s.fx * vc.x), fabsf(s.fy * vc.y)),
+                                            vc.x * vc.x + vc.y * vc.y + vc.z * vc.z) < kOrdHi);
 }
 __device__ __forceinline__ int voxel_pixel_ord(const Intr &s, float rows, float cols, f3 vc, float &dist) {
   const float half = 0x1.fffffep-2f;
@@ -452,7 +453,7 @@ __device__ __forceinline__ uint64_t integrate_voxel(float tau, float max_weight,
   const float num = vox_sdf(old) * w + nsdf * 1.0f;
   const float rm = __builtin_amdgcn_rcpf(m);
   float sdf = div_nr(num, m, __builtin_fmaf(__builtin_fmaf(-m, rm, 1.0f), rm, rm));
-  const bool odd = !(fabsf(num) > 0x1p-80f) | !(fabsf(num) < 0x1p80f);
+  const bool odd = (int)!(fabsf(num) > 0x1p-80f) | (int)!(fabsf(num) < 0x1p80f);
   if (__ballot(odd)) {  // also exact zeros: rare
     if (odd) sdf = num / m;
   }
@@ -599,7 +600,7 @@ __global__ __launch_bounds__(256) void k_integrate(const DmView *__restrict__ vi
       // every rounded operation above is monotone in x, so a camera
       // coordinate lies between its values at the row's ends: ordinary there is
       // ordinary along the row
-      const bool ord = __ballot(!(ordinary(s, camera(0)) & ordinary(s, camera(7)))) == 0ull;
+      const bool ord = __ballot(!((int)ordinary(s, camera(0)) & (int)ordinary(s, camera(7)))) == 0ull;
       bool near = false;
       if (ord) {
         u64 sp[8];
@@ -1374,7 +1375,8 @@ __device__ __forceinline__ int beam_steps(const DmView &v, const Intr &s, const 
 }
 
 __global__ __launch_bounds__(256, 6) void k_raycast(const DmView *__restrict__ views, const int *__restrict__ active,
-                                                        int tw_log2) {
+                                                        int tw_log2, float *__restrict__ ray_depth,
+                                                        uint8_t *__restrict__ ray_rgb) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
@@ -1529,9 +1531,9 @@ __global__ __launch_bounds__(256, 6) void k_raycast(const DmView *__restrict__ v
   }
   v.tvert[0][i] = vert;
   v.tnorm[0][i] = nrm;
-  if (v.ray_depth) v.ray_depth[i] = dout;
-  if (v.ray_rgb) {
-    uint8_t *o = v.ray_rgb + 3 * (size_t)i;
+  if (ray_depth) ray_depth[i] = dout;
+  if (ray_rgb) {
+    uint8_t *o = ray_rgb + 3 * (size_t)i;
     o[0] = (uint8_t)cr; o[1] = (uint8_t)cg; o[2] = (uint8_t)cb;
   }
   // coarser model levels by nearest subsampling
@@ -1608,7 +1610,7 @@ void launch_raycast(const Launch &L) {
   const int tw = 1 << L.ray_tw_log2, th = 256 >> L.ray_tw_log2;
   const unsigned tiles = (unsigned)(((L.max_cols + tw - 1) / tw) * ((L.max_rows + th - 1) / th));
   hipLaunchKernelGGL(k_raycast, dim3(tiles, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active,
-                     L.ray_tw_log2);
+                     L.ray_tw_log2, L.ray_depth, L.ray_rgb);
 }
 
 }  // namespace dm

@@ -68,10 +68,10 @@ class TsdfVolume:
     def Raycast(self, pose, sensor):
         """depth, vertex, normal, rgb of the model seen from `pose`."""
         r, c = sensor["rows"], sensor["cols"]
-        d = np.zeros((r, c), np.float32)
-        v = np.zeros((r, c, 3), np.float32)
-        n = np.zeros((r, c, 3), np.float32)
-        rgb = np.zeros((r, c, 3), np.uint8)
+        d = np.empty((r, c), np.float32)
+        v = np.empty((r, c, 3), np.float32)
+        n = np.empty((r, c, 3), np.float32)
+        rgb = np.empty((r, c, 3), np.uint8)
         pf = np.ascontiguousarray(pose, np.float32)
         N.check(self._lib.dm_volume_raycast(self._h, N.ptr(pf), C.byref(_sensor(sensor)), N.ptr(d), N.ptr(v),
                                             N.ptr(n), N.ptr(rgb)))
@@ -578,9 +578,9 @@ class Session:
 
     def source_maps(self, depth, rgb, level):
         r, c = self.sensor["rows"] >> level, self.sensor["cols"] >> level
-        v = np.zeros((r, c, 3), np.float32)
-        n = np.zeros((r, c, 3), np.float32)
-        it = np.zeros((r, c), np.float32)
+        v = np.empty((r, c, 3), np.float32)
+        n = np.empty((r, c, 3), np.float32)
+        it = np.empty((r, c), np.float32)
         N.check(self._lib.dm_session_source_maps(self._h, N.ptr(_f32(depth)), N.ptr(_u8(rgb)), level, N.ptr(v),
                                                  N.ptr(n), N.ptr(it)))
         return v, n, it

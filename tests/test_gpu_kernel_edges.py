@@ -140,3 +140,22 @@ def test_integration_operand_range(room, scale):
     np.testing.assert_array_equal(gw[gi], ow[oi])
     np.testing.assert_array_equal(gs[gi], os_[oi].astype(np.float32))
     assert (gw > 0).any()
+
+
+# Host results pass in chunks of half the frame's pinned buffer: images from
+# one pixel up, smaller than the volume's frame, every output and fewer of them.
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 5), (33, 31), (240, 320)])
+def test_raycast_outputs_in_chunks(room, rows, cols):
+    import ctypes as C
+    from dynamap_amd import _native as N
+    depth, poses = room
+    vol = dm.TsdfVolume(small_tsdf(), SENS["rows"], SENS["cols"])
+    vol.IntegrateScan(depth[0], None, SENS, poses[0].astype(np.float32))
+    sens = dict(rows=rows, cols=cols, fx=0.8 * cols + 1, fy=0.8 * cols + 1, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    Tf = np.ascontiguousarray(poses[0], np.float32)
+    d, v, n, c = vol.Raycast(Tf, sens)
+    np.testing.assert_array_equal(v[..., 2], d)  # a vertex's z is its depth, 0 without a surface
+    assert np.array_equal(np.isnan(n[..., 0]), np.isnan(n[..., 2]))
+    only = np.full((rows, cols, 3), 7, np.float32)
+    N.check(N.lib().dm_volume_raycast(vol._h, N.ptr(Tf), C.byref(configs.sensor(sens)), None, None, N.ptr(only), None))
+    np.testing.assert_array_equal(only, n)
