@@ -856,7 +856,8 @@ __global__ __launch_bounds__(256) void kb_nr_invdiag(const b_nr_invdiag *__restr
 // vectors of its nodes' rows and writes m and the partials for the next
 // iteration.  Mathematically the standard PCG iteration (the same x_k), with
 // one kernel boundary per iteration.
-constexpr int kSpmvNodes = 16;  // wavefronts (nodes) per workgroup
+constexpr int kSpmvNodes = 16;           // nodes per workgroup
+constexpr int kPcgThreads = 16 * kSpmvNodes;  // 16 lanes (a DPP row) per node
 
 struct PcgState {
   double *x, *r, *u, *w;  // 6 N each: iterate, residual, u = M r, w = A u
@@ -871,52 +872,93 @@ struct PcgState {
   int nwg;                // workgroups of the start and iteration kernels (kSpmvNodes nodes each)
 };
 
-// Row `lane` (< 6) of (A v) at the wavefront's node, 0 in the other lanes.
-// Lane j takes the node's block entries j, j + 64, ... whole (a 6x6 block,
-// transposed for the lower triangle, times the column node's 6 values), so
-// a node's entries are one round of loads; the six row sums are then added
-// over the lanes by the fixed tree of wave_sum.
-__device__ __forceinline__ double spmv_node(const float *__restrict__ H, const int *__restrict__ row_start,
-                                            const uint2 *__restrict__ row_ec,
-                                            const double *__restrict__ v, int node, int nn, int lane) {
-  double acc[6] = {0, 0, 0, 0, 0, 0};
-  if (node < nn) {
-    const int k1 = row_start[node + 1];  // node is uniform in the wavefront: scalar loads
-    for (int k = row_start[node] + lane; k < k1; k += 64) {
-      const uint2 ec = row_ec[k];
-      const int blk = (int)(ec.x & 0x7fffffffu);
-      const bool tr = ec.x >> 31;
-      const float *B = H + 36 * (size_t)blk;
-      const double2 *V2 = reinterpret_cast<const double2 *>(v + 6 * (size_t)ec.y);
-      double vc[6];
+// Row `lane % 16` (< 6) of (A v) at `node`, 0 in the row's other lanes.  A
+// node has the 16 lanes of a DPP row, four nodes a wavefront: lane j takes
+// the node's block entries 16 q + j (+ 64, ...) of quarter q = 0..3 whole (a
+// 6x6 block, transposed for the lower triangle, times the column node's 6
+// values); each quarter's six row sums are added over the lanes by row_sum and
+// the quarters as (0 + 1) + (2 + 3).  A node has about 14 entries, so quarter 0
+// is nearly always all: one round of loads.  (A wavefront per node did the same
+// sums with 50 of its 64 lanes idle, and 16 wavefronts per CU contended for the
+// FP64 units: an iteration took 6.85 us at 4048 nodes and 12.2 us for four graphs
+// of 1150, now 5.3 and 6.6.)
+struct SpmvRows {
+  const int *start;     // first entry of each node's row (nn + 1)
+  const uint2 *ec;      // entries: block | transposed << 31, column node
+  const uint2 *first;   // the first 16 entries of each row, kNoEntry past the row's end: their address needs no
+                        // row offset, one memory latency less before the blocks' loads
+};
+constexpr uint32_t kNoEntry = 0xffffffffu;
+__device__ __forceinline__ void spmv_entry(const float *__restrict__ H, const double *__restrict__ v, uint2 ec,
+                                           double acc[6]) {
+  const bool tr = ec.x >> 31;
+  const double2 *V2 = reinterpret_cast<const double2 *>(v + 6 * (size_t)ec.y);
+  double vc[6];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const double2 d = V2[q];
-        vc[2 * q] = d.x; vc[2 * q + 1] = d.y;
-      }
-      const float4 *B4 = reinterpret_cast<const float4 *>(B);
-      float b[36];
+  for (int c = 0; c < 3; ++c) {
+    const double2 d = V2[c];
+    vc[2 * c] = d.x; vc[2 * c + 1] = d.y;
+  }
+  const float4 *B4 = reinterpret_cast<const float4 *>(H + 36 * (size_t)(ec.x & 0x7fffffffu));
+  float b[36];
 #pragma unroll
-      for (int q = 0; q < 9; ++q) {
-        const float4 f = B4[q];
-        b[4 * q] = f.x; b[4 * q + 1] = f.y; b[4 * q + 2] = f.z; b[4 * q + 3] = f.w;
-      }
+  for (int c = 0; c < 9; ++c) {
+    const float4 f = B4[c];
+    b[4 * c] = f.x; b[4 * c + 1] = f.y; b[4 * c + 2] = f.z; b[4 * c + 3] = f.w;
+  }
+#pragma unroll
+  for (int r = 0; r < 6; ++r) {
+    double sv = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) sv += (double)(tr ? b[6 * c + r] : b[6 * r + c]) * vc[c];
+    acc[r] += sv;
+  }
+}
+__device__ __forceinline__ double spmv_node(const float *__restrict__ H, SpmvRows R, const double *__restrict__ v,
+                                            int node, int nn, int lane16) {
+  const int nd = node < nn ? node : nn - 1;
+  const uint2 e0 = R.first[16 * (size_t)nd + lane16];
+  const int k0 = R.start[nd], k1 = node < nn ? R.start[nd + 1] : k0;
+  double sum[6] = {0, 0, 0, 0, 0, 0};
+  if (node < nn && e0.x != kNoEntry) spmv_entry(H, v, e0, sum);
+  if (__ballot(k1 - k0 > 16) == 0ull) {
+#pragma unroll
+    for (int r = 0; r < 6; ++r) sum[r] = row_sum(sum[r]);
+  } else {
+    // rows of more than 16 entries
+    for (int k = k0 + 64 + lane16; k < k1; k += 64) spmv_entry(H, v, R.ec[k], sum);
+#pragma unroll
+    for (int r = 0; r < 6; ++r) sum[r] = row_sum(sum[r]);
+    double q2[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 1
+    for (int q = 1; q < 4; ++q) {
+      double acc[6] = {0, 0, 0, 0, 0, 0};
+      for (int k = k0 + 16 * q + lane16; k < k1; k += 64) spmv_entry(H, v, R.ec[k], acc);
 #pragma unroll
       for (int r = 0; r < 6; ++r) {
-        double sv = 0.0;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) sv += (double)(tr ? b[6 * c + r] : b[6 * r + c]) * vc[c];
-        acc[r] += sv;
+        const double t = row_sum(acc[r]);
+        if (q == 1) sum[r] += t;
+        else if (q == 2) q2[r] = t;
+        else q2[r] += t;
       }
+      if (__ballot(k1 - k0 > 16 * (q + 1)) == 0ull) break;  // the other quarters are zero
     }
+#pragma unroll
+    for (int r = 0; r < 6; ++r) sum[r] += q2[r];
   }
   double out = 0.0;
 #pragma unroll
-  for (int r = 0; r < 6; ++r) {
-    const double t = wave_sum(acc[r]);
-    if (lane == r) out = t;
-  }
-  return node < nn ? out : 0.0;
+  for (int r = 0; r < 6; ++r)
+    if (lane16 == r) out = sum[r];
+  return out;
+}
+
+__global__ __launch_bounds__(256) void k_nr_row_first(const int *__restrict__ start, const uint2 *__restrict__ ec,
+                                                     int nn, uint2 *__restrict__ first) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= 16 * nn) return;
+  const int k = start[i >> 4] + (i & 15);
+  first[i] = k < start[(i >> 4) + 1] ? ec[k] : make_uint2(kNoEntry, 0u);
 }
 
 // The partials of r.u and w.u into half `half` of the partial array, one
@@ -939,7 +981,7 @@ __device__ __forceinline__ void pcg_partials(const PcgState &S, double ru, doubl
 // 1 rows 60 .. 95 (nodes 10 .. 15) in lanes 0 .. 35, so that each node's six
 // rows are in one wavefront; -1 for a lane without a row.
 constexpr int kPcgRows = 6 * kSpmvNodes;
-static_assert(kPcgRows == 96, "two update wavefronts of 60 and 36 rows");
+static_assert(kPcgRows == 96 && kPcgThreads == 256, "two update wavefronts of 60 and 36 rows, two that add the partials");
 __device__ __forceinline__ int pcg_row() {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   return wv == 0 ? (lane < 60 ? lane : -1) : wv == 1 ? (lane < 36 ? 60 + lane : -1) : -1;
@@ -948,8 +990,7 @@ __device__ __forceinline__ int pcg_row() {
 // Start: w = A u, m = M w, partials of r_0.u_0 and w_0.u_0 (x = 0, r = rhs and
 // u = M r are written by the preconditioner kernel).
 __device__ __forceinline__ void d_pcg_start(PcgState S, const float *__restrict__ H,
-                                            const int *__restrict__ row_start, const uint2 *__restrict__ row_ec,
-                                            const double *__restrict__ Minv, int nn) {
+                                            SpmvRows R, const double *__restrict__ Minv, int nn) {
   __shared__ double nl[kPcgRows];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int i = pcg_row();
@@ -962,9 +1003,9 @@ __device__ __forceinline__ void d_pcg_start(PcgState S, const float *__restrict_
 #pragma unroll
     for (int c = 0; c < 6; ++c) mrow[c] = Minv[6 * e + c];
   }
-  const int node = blockIdx.x * kSpmvNodes + __builtin_amdgcn_readfirstlane(wv);
-  const double wn = spmv_node(H, row_start, row_ec, S.u, node, nn, lane);
-  if (lane < 6) nl[6 * wv + lane] = wn;
+  const int l16 = lane & 15, local = threadIdx.x >> 4;  // lane of the node's row, node in the workgroup
+  const double wn = spmv_node(H, R, S.u, blockIdx.x * kSpmvNodes + local, nn, l16);
+  if (l16 < 6) nl[6 * local + l16] = wn;
   __syncthreads();
   double w = 0.0;
   if (own) { w = nl[i]; S.w[e] = w; }
@@ -978,26 +1019,23 @@ __device__ __forceinline__ void d_pcg_start(PcgState S, const float *__restrict_
   pcg_partials(S, own ? rv * uv : 0.0, own ? w * uv : 0.0, 0);
   if (blockIdx.x == 0 && threadIdx.x == 0) { S.flag[0] = 0; S.flag[1] = 0; }
 }
-__global__ __launch_bounds__(64 * kSpmvNodes) void k_pcg_start(PcgState S, const float *__restrict__ H,
-                                                              const int *__restrict__ row_start,
-                                                              const uint2 *__restrict__ row_ec,
-                                                              const double *__restrict__ Minv, int nn) {
-  d_pcg_start(S, H, row_start, row_ec, Minv, nn);
+__global__ __launch_bounds__(kPcgThreads) void k_pcg_start(PcgState S, const float *__restrict__ H,
+                                                              SpmvRows R, const double *__restrict__ Minv, int nn) {
+  d_pcg_start(S, H, R, Minv, nn);
 }
 struct b_pcg_start {
   PcgState S;
   const float *H;
-  const int *row_start;
-  const uint2 *row_ec;
+  SpmvRows R;
   const double *Minv;
   int nn;
   unsigned grid;  // workgroups of this graph's launch
 };
 // k_pcg_start for a batch of graphs: graph blockIdx.y, its arguments in t[blockIdx.y]
-__global__ __launch_bounds__(64 * kSpmvNodes) void kb_pcg_start(const b_pcg_start *__restrict__ t) {
+__global__ __launch_bounds__(kPcgThreads) void kb_pcg_start(const b_pcg_start *__restrict__ t) {
   const b_pcg_start &a = t[blockIdx.y];
   if (blockIdx.x >= a.grid) return;
-  d_pcg_start(a.S, a.H, a.row_start, a.row_ec, a.Minv, a.nn);
+  d_pcg_start(a.S, a.H, a.R, a.Minv, a.nn);
 }
 
 // Iteration k: gamma = r.u and delta = w.u from the partials (wavefronts 2
@@ -1010,8 +1048,8 @@ __global__ __launch_bounds__(64 * kSpmvNodes) void kb_pcg_start(const b_pcg_star
 // of r.u and w.u.  The partials, the rows' operands and the SpMV's loads
 // are all issued before the first wait.
 __device__ __forceinline__ void d_pcg_iter(PcgState S, const float *__restrict__ H,
-                                           const int *__restrict__ row_start, const uint2 *__restrict__ row_ec,
-                                           const double *__restrict__ Minv, int nn, int it, const NrFrame *Fp) {
+                                           SpmvRows R, const double *__restrict__ Minv, int nn, int it,
+                                           const NrFrame *Fp) {
   __shared__ double nl[kPcgRows], wl[kPcgRows], l2[2], sc[5];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   // wavefronts 2 and 3: lane l adds partials l, l + 64, ... in order; the
@@ -1048,10 +1086,10 @@ __device__ __forceinline__ void d_pcg_iter(PcgState S, const float *__restrict__
 #pragma unroll
     for (int c = 0; c < 6; ++c) mrow[c] = Minv[6 * e + c];
   }
-  const int node = blockIdx.x * kSpmvNodes + __builtin_amdgcn_readfirstlane(wv);
+  const int l16 = lane & 15, local = threadIdx.x >> 4;  // lane of the node's row, node in the workgroup
   // (computed also after convergence, so that the flag's load is not on the SpMV's path)
-  const double n = spmv_node(H, row_start, row_ec, m_in, node, nn, lane);
-  if (lane < 6) nl[6 * wv + lane] = n;
+  const double n = spmv_node(H, R, m_in, blockIdx.x * kSpmvNodes + local, nn, l16);
+  if (l16 < 6) nl[6 * local + l16] = n;
   if (pw) {
     double pacc = 0.0;
 #pragma unroll
@@ -1105,28 +1143,25 @@ __device__ __forceinline__ void d_pcg_iter(PcgState S, const float *__restrict__
   }
   pcg_partials(S, own ? rv * uv : 0.0, own ? wn * uv : 0.0, (it + 1) & 1);
 }
-__global__ __launch_bounds__(64 * kSpmvNodes) void k_pcg_iter(PcgState S, const float *__restrict__ H,
-                                                             const int *__restrict__ row_start,
-                                                             const uint2 *__restrict__ row_ec,
-                                                             const double *__restrict__ Minv, int nn, int it,
-                                                             const NrFrame *Fp) {
-  d_pcg_iter(S, H, row_start, row_ec, Minv, nn, it, Fp);
+__global__ __launch_bounds__(kPcgThreads) void k_pcg_iter(PcgState S, const float *__restrict__ H,
+                                                             SpmvRows R, const double *__restrict__ Minv, int nn,
+                                                             int it, const NrFrame *Fp) {
+  d_pcg_iter(S, H, R, Minv, nn, it, Fp);
 }
 struct b_pcg_iter {
   PcgState S;
   const float *H;
-  const int *row_start;
-  const uint2 *row_ec;
+  SpmvRows R;
   const double *Minv;
   int nn;
   const NrFrame *Fp;
   unsigned grid;  // workgroups of this graph's launch
 };
 // k_pcg_iter for a batch of graphs: graph blockIdx.y, its arguments in t[blockIdx.y]
-__global__ __launch_bounds__(64 * kSpmvNodes) void kb_pcg_iter(const b_pcg_iter *__restrict__ t, int it) {
+__global__ __launch_bounds__(kPcgThreads) void kb_pcg_iter(const b_pcg_iter *__restrict__ t, int it) {
   const b_pcg_iter &a = t[blockIdx.y];
   if (blockIdx.x >= a.grid) return;
-  d_pcg_iter(a.S, a.H, a.row_start, a.row_ec, a.Minv, a.nn, it, a.Fp);
+  d_pcg_iter(a.S, a.H, a.R, a.Minv, a.nn, it, a.Fp);
 }
 
 // T_i <- exp(x_i) T_i, then the node's dual quaternion
@@ -1253,7 +1288,8 @@ struct dm_graph {
   int *blk_a = nullptr, *blk_b = nullptr, *cstart = nullptr, *row_start = nullptr;
   uint32_t *codes = nullptr, *row_ent = nullptr;
   float2 *cw = nullptr;  // per contribution: the weights of the block's two nodes at the vertex
-  uint2 *row_ec = nullptr;  // row entries for the SpMV: (row_ent, column node)
+  uint2 *row_ec = nullptr;     // row entries for the SpMV: (row_ent, column node)
+  uint2 *row_first = nullptr;  // the first 16 of each row (SpmvRows::first)
   // per-iteration buffers
   float *pv = nullptr, *pn = nullptr, *vdata = nullptr, *H = nullptr;
   double *edata = nullptr, *rhs = nullptr, *Minv = nullptr, *Hd = nullptr, *stats = nullptr, *stats_part = nullptr;
@@ -1293,6 +1329,8 @@ struct dm_graph {
   }
 };
 
+
+static SpmvRows rows_of(const dm_graph *g) { return {g->row_start, g->row_ec, g->row_first}; }
 
 static unsigned grid_of(long long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
@@ -1458,6 +1496,7 @@ static int graph_finish(dm_graph *g) {
   DM_TRY(g->dalloc(&g->row_ent, nrow));
   DM_TRY(g->dalloc(&g->row_ec, nrow));
   DM_TRY(g->dalloc(&g->row_start, nn + 1));
+  DM_TRY(g->dalloc(&g->row_first, 16 * nn));
   DM_HIP(hipMemcpyAsync(droff.p, roff.data(), nb * 8, hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_nr_row_emit, dim3(grid_of(nb)), dim3(256), 0, st, g->blk_a, g->blk_b, (int)nb,
                      droff.as<long long>(), rk0.as<uint32_t>(), rv0.as<uint32_t>());
@@ -1466,6 +1505,8 @@ static int graph_finish(dm_graph *g) {
                      g->row_start, (int)nn);
   hipLaunchKernelGGL(k_nr_row_ec, dim3(grid_of(nrow)), dim3(256), 0, st, rk1.as<uint32_t>(), g->row_ent, nrow,
                      g->row_ec);
+  hipLaunchKernelGGL(k_nr_row_first, dim3(grid_of(16 * nn)), dim3(256), 0, st, g->row_start, g->row_ec, (int)nn,
+                     g->row_first);
   DM_HIP(hipGetLastError());
   // state and per-iteration buffers
   DM_TRY(g->dalloc(&g->T, nn * 16));
@@ -1539,10 +1580,10 @@ static void nr_enqueue(dm_graph *g, int rows, int cols, int gn, int pcg_its, int
                          g->stats_part);
       hipLaunchKernelGGL(k_nr_stats_sum, dim3(1), dim3(64), 0, st, g->stats_part, g->stats);
     }
-    hipLaunchKernelGGL(k_pcg_start, dim3(pg), dim3(64 * kSpmvNodes), 0, st, S, g->H, g->row_start, g->row_ec,
+    hipLaunchKernelGGL(k_pcg_start, dim3(pg), dim3(kPcgThreads), 0, st, S, g->H, rows_of(g),
                        g->Minv, nn);
     for (int k = 0; k < pcg_its; ++k)
-      hipLaunchKernelGGL(k_pcg_iter, dim3(pg), dim3(64 * kSpmvNodes), 0, st, S, g->H, g->row_start, g->row_ec,
+      hipLaunchKernelGGL(k_pcg_iter, dim3(pg), dim3(kPcgThreads), 0, st, S, g->H, rows_of(g),
                          g->Minv, nn, k, F);
     hipLaunchKernelGGL(k_nr_update, dim3(grid_of(nn)), dim3(256), 0, st, S.x, g->T, nn, g->dq);
   }
@@ -1724,8 +1765,8 @@ static int batch_capture(dm_nonrigid_batch *b, int rows, int cols, int gn, int p
     inv[i] = {g->Hd, nn, g->Minv, g->rhs, S.x, S.r, S.u, grid_of(nn)};
     sta[i] = {g->vdata, g->nv, g->edata, ne, F, g->stats_part, (unsigned)kStatsWg};
     ssum[i] = {g->stats_part, g->stats, 1u};
-    pst[i] = {S, g->H, g->row_start, g->row_ec, g->Minv, nn, (unsigned)S.nwg};
-    pit[i] = {S, g->H, g->row_start, g->row_ec, g->Minv, nn, F, (unsigned)S.nwg};
+    pst[i] = {S, g->H, rows_of(g), g->Minv, nn, (unsigned)S.nwg};
+    pit[i] = {S, g->H, rows_of(g), g->Minv, nn, F, (unsigned)S.nwg};
     nup[i] = {S.x, g->T, nn, g->dq, grid_of(nn)};
   }
   BatchTables T;
@@ -1758,10 +1799,10 @@ static int batch_capture(dm_nonrigid_batch *b, int rows, int cols, int gn, int p
       hipLaunchKernelGGL(kb_nr_stats, dim3(max_grid(sta), Ky), dim3(256), 0, st, (const b_nr_stats *)(D + o_sta));
       hipLaunchKernelGGL(kb_nr_stats_sum, dim3(1, Ky), dim3(64), 0, st, (const b_nr_stats_sum *)(D + o_ssum));
     }
-    hipLaunchKernelGGL(kb_pcg_start, dim3(max_grid(pst), Ky), dim3(64 * kSpmvNodes), 0, st,
+    hipLaunchKernelGGL(kb_pcg_start, dim3(max_grid(pst), Ky), dim3(kPcgThreads), 0, st,
                        (const b_pcg_start *)(D + o_pst));
     for (int k = 0; k < pcg_its; ++k)
-      hipLaunchKernelGGL(kb_pcg_iter, dim3(max_grid(pit), Ky), dim3(64 * kSpmvNodes), 0, st,
+      hipLaunchKernelGGL(kb_pcg_iter, dim3(max_grid(pit), Ky), dim3(kPcgThreads), 0, st,
                          (const b_pcg_iter *)(D + o_pit), k);
     hipLaunchKernelGGL(kb_nr_update, dim3(max_grid(nup), Ky), dim3(256), 0, st, (const b_nr_update *)(D + o_nup));
   }
