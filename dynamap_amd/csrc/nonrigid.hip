@@ -638,31 +638,42 @@ __global__ __launch_bounds__(256) void kb_nr_terms(const NrTerms *__restrict__ t
   d_nr_terms<false>(a);
 }
 
-// ARAP Jacobian rows for component c: Ji = w [row c of -[a]x, e_c],
-// Jj = -w [row c of -[b]x, e_c]
-__device__ __forceinline__ void arap_rows(const double *ed, int c, double Ji[6], double Jj[6]) {
-  const double *A = ed, *B = ed + 3;
-  const double w = ed[6];
+// Sum of 48 values over the 16 lanes of a row: lane l ends with values
+// sum_base(l) .. + 2.  Each step a lane keeps half of its values and sends the
+// other half to its partner, which keeps those: the partners and so the sums
+// are row_sum's, with 45 additions instead of 4 x 48.  The partners' subsets
+// match because every bit of a subset is a sum of lane bits that row_sum's
+// later partners (mirrors, which flip several lane bits) leave alone.
+template <int kCtrl, int N> __device__ __forceinline__ void sum_half(double (&v)[48], bool upper) {
 #pragma unroll
-  for (int q = 0; q < 6; ++q) { Ji[q] = 0.0; Jj[q] = 0.0; }
-  if (c == 0) { Ji[1] = A[2]; Ji[2] = -A[1]; Jj[1] = B[2]; Jj[2] = -B[1]; }
-  if (c == 1) { Ji[0] = -A[2]; Ji[2] = A[0]; Jj[0] = -B[2]; Jj[2] = B[0]; }
-  if (c == 2) { Ji[0] = A[1]; Ji[1] = -A[0]; Jj[0] = B[1]; Jj[1] = -B[0]; }
-  Ji[3 + c] = 1.0;
-  Jj[3 + c] = 1.0;
-#pragma unroll
-  for (int q = 0; q < 6; ++q) { Ji[q] *= w; Jj[q] *= -w; }
+  for (int i = 0; i < N; ++i) {
+    const double keep = upper ? v[N + i] : v[i], send = upper ? v[i] : v[N + i];
+    v[i] = keep + dpp_f64<kCtrl>(send);
+  }
+}
+__device__ __forceinline__ int sum_scatter(double (&v)[48], int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+  sum_half<0xb1, 24>(v, b0 != b2);   // quad_perm [1, 0, 3, 2]
+  sum_half<0x4e, 12>(v, b1 != b2);   // quad_perm [2, 3, 0, 1]
+  sum_half<0x141, 6>(v, b2 != b3);   // row_half_mirror
+  sum_half<0x140, 3>(v, b3);         // row_mirror
+  return 24 * (b0 != b2) + 12 * (b1 != b2) + 6 * (b2 != b3) + 3 * b3;
 }
 
 // kAsmLanes lanes per block (4 blocks per wavefront): H_ab (and for a == b
 // the rhs, the damping and the FP64 block itself, inverted by k_nr_invdiag).
 // Lanes take contributions strided by kAsmLanes; the lane sums are combined
-// by the fixed DPP tree of row_sum within the block's lanes (one row of 16).
-// 16 lanes give each lane several independent gathers in flight and a
-// 4-level tree (a wavefront per block took about 153 us per assembly at
-// 4048 nodes, these about 65 us).
-// Launched at 3 waves per SIMD (168 VGPRs, a few spilled) rather than the
-// compiler's 2 (176 VGPRs): more blocks in flight.
+// by the fixed DPP tree of row_sum within the block's lanes (one row of 16),
+// which leaves three of the block's values in each lane to store.
+// Every sum keeps its operations and their order: motions that slide a
+// surface along itself are held by the damping alone, so that a last bit moves
+// them by 1e-5 of their size.  For the same reason the entries (r, q) and (q, r)
+// of a data term are computed on their own.
+// An ARAP edge's rows have three nonzero entries each, so a component adds 9
+// products (the others are zero).
+// Bound by FP64 issue and the gathers' latency: 28440 blocks in 40 us (49
+// with 36 products per ARAP component, all 42 sums in every lane and a block's
+// stores in one lane).
 constexpr int kAsmLanes = 16;
 __device__ __forceinline__ void d_nr_assemble(const int *__restrict__ blk_a, const int *__restrict__ blk_b,
                                               const int *__restrict__ cstart, const uint32_t *__restrict__ codes,
@@ -676,55 +687,62 @@ __device__ __forceinline__ void d_nr_assemble(const int *__restrict__ blk_a, con
   const NrFrame &F = *Fp;
   const int a = blk_a[blk], b = blk_b[blk];
   const bool diag = a == b;
-  double h[36], g[6];
+  double h[48];  // the block's 36 entries, its 6 of the rhs, padding
 #pragma unroll
-  for (int q = 0; q < 36; ++q) h[q] = 0.0;
-#pragma unroll
-  for (int q = 0; q < 6; ++q) g[q] = 0.0;
+  for (int q = 0; q < 48; ++q) h[q] = 0.0;
   const double lam = F.lambda;
-  // one contribution: a vertex's data term (weights wa, wb of the block's two
-  // nodes at the vertex, from cw) or an ARAP edge's rows
-  auto add_one = [&](uint32_t code, float2 w, float4 d0, float4 d1) {
-    if (!(code & kArapTag)) {
-      if (d1.w == 0.f) return;
-      const double wa = (double)w.x, wb = (double)w.y;
-      const double gv[6] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y};
-      const double s = wa * wb;
+  // one data contribution: weights wa, wb of the block's two nodes at the
+  // vertex (from cw), the vertex's record
+  auto add_data = [&](float2 w, float4 d0, float4 d1) {
+    if (d1.w == 0.f) return;
+    const double wa = (double)w.x, wb = (double)w.y;
+    const double gv[6] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y};
+    const double s = wa * wb;
 #pragma unroll
-      for (int r = 0; r < 6; ++r)
+    for (int r = 0; r < 6; ++r) {
+      const double sg = s * gv[r];
 #pragma unroll
-        for (int q = 0; q < 6; ++q) h[6 * r + q] += s * gv[r] * gv[q];
-      if (diag) {
-        const double rr = (double)d1.z;
+      for (int q = 0; q < 6; ++q) h[6 * r + q] += sg * gv[q];
+    }
+    if (diag) {
+      const double rr = (double)d1.z;
 #pragma unroll
-        for (int r = 0; r < 6; ++r) g[r] -= wa * gv[r] * rr;
-      }
-    } else {
-      const int e = (int)((code & ~kArapTag) >> 2), role = code & 3;
-      const double *ed = edata + 8 * (size_t)e;
-      const int i = e / kNK, j = nbr[e];
+      for (int r = 0; r < 6; ++r) h[36 + r] -= wa * gv[r] * rr;
+    }
+  };
+  // an ARAP edge: Jacobian rows of component c are Ji = w [row c of -[A]x, e_c]
+  // and Jj = -w [row c of -[B]x, e_c], row c of -[A]x being A_m2 at m1 and
+  // -A_m1 at m2 with (c, m1, m2) cyclic
+  auto add_arap = [&](uint32_t code) {
+    const int e = (int)((code & ~kArapTag) >> 2), role = code & 3;
+    const double *ed = edata + 8 * (size_t)e;
+    const int i = e / kNK, j = nbr[e];
+    const double w = ed[6];
+    // the block is (min, max): transpose the (i, j) product when i > j
+    const bool ui = role == 0 || (role == 2 && i <= j), wi = role == 0 || (role == 2 && i > j);
+    double ru[3], rw[3], rho[3];
+    const double su = ui ? w : -w, sw = wi ? w : -w;
 #pragma unroll
-      for (int c3 = 0; c3 < 3; ++c3) {
-        double Ji[6], Jj[6];
-        arap_rows(ed, c3, Ji, Jj);
-        const double rc = ed[6] * (ed[c3] - ed[3 + c3]);
-        // the block is (min, max): transpose the (i, j) product when i > j
-        // (values selected, not pointers, so the rows stay in registers)
-        const bool ui = role == 0 || (role == 2 && i <= j), wi = role == 0 || (role == 2 && i > j);
-        double U[6], W[6];
+    for (int c = 0; c < 3; ++c) {
+      const double ea = ed[c], eb = ed[3 + c];
+      ru[c] = ui ? ea : eb;
+      rw[c] = wi ? ea : eb;
+      rho[c] = w * (ea - eb);
+    }
 #pragma unroll
-        for (int r = 0; r < 6; ++r) {
-          U[r] = ui ? Ji[r] : Jj[r];
-          W[r] = wi ? Ji[r] : Jj[r];
-        }
+    for (int c = 0; c < 3; ++c) {
+      const int m1 = (c + 1) % 3, m2 = (c + 2) % 3;
+      // nonzero entries at m1, m2 and 3 + c
+      const double U[3] = {lam * (ru[m2] * su), lam * (-ru[m1] * su), lam * su};
+      const double W[3] = {rw[m2] * sw, -rw[m1] * sw, sw};
+      const int at[3] = {m1, m2, 3 + c};
 #pragma unroll
-        for (int r = 0; r < 6; ++r)
+      for (int r = 0; r < 3; ++r)
 #pragma unroll
-          for (int q = 0; q < 6; ++q) h[6 * r + q] += lam * U[r] * W[q];
-        if (role < 2)
+        for (int q = 0; q < 3; ++q) h[6 * at[r] + at[q]] += U[r] * W[q];
+      if (role < 2)
 #pragma unroll
-          for (int r = 0; r < 6; ++r) g[r] -= lam * U[r] * rc;
-      }
+        for (int r = 0; r < 3; ++r) h[36 + at[r]] -= U[r] * rho[c];
     }
   };
   // contributions c, c + kAsmLanes, ... in order, two at a time so that both
@@ -740,28 +758,26 @@ __device__ __forceinline__ void d_nr_assemble(const int *__restrict__ blk_a, con
     float4 a0 = z4, a1 = z4, b0 = z4, b1 = z4;
     if (!(k0 & kArapTag)) { const size_t v = k0 >> 4; a0 = V4[2 * v]; a1 = V4[2 * v + 1]; }
     if (!(k1 & kArapTag)) { const size_t v = k1 >> 4; b0 = V4[2 * v]; b1 = V4[2 * v + 1]; }
-    add_one(k0, w0, a0, a1);
-    if (has1) add_one(k1, w1, b0, b1);
+    if (k0 & kArapTag) add_arap(k0);
+    else add_data(w0, a0, a1);
+    if (has1) {
+      if (k1 & kArapTag) add_arap(k1);
+      else add_data(w1, b0, b1);
+    }
   }
   static_assert(kAsmLanes == 16, "a block's lanes are one DPP row");
-  auto lanes_sum = [](double x) { return row_sum(x); };
+  const int base = sum_scatter(h, lane);
 #pragma unroll
-  for (int q = 0; q < 36; ++q) h[q] = lanes_sum(h[q]);
-#pragma unroll
-  for (int q = 0; q < 6; ++q) g[q] = lanes_sum(g[q]);  // zero off the diagonal
-  if (lane != 0) return;
-  if (diag)
-#pragma unroll
-    for (int r = 0; r < 6; ++r) h[7 * r] += F.damping;
-  float *Hb = H + 36 * (size_t)blk;
-#pragma unroll
-  for (int q = 0; q < 36; ++q) Hb[q] = (float)h[q];
-  if (!diag) return;
-#pragma unroll
-  for (int r = 0; r < 6; ++r) rhs[6 * a + r] = g[r];
-  double *D = Hd + 36 * (size_t)a;
-#pragma unroll
-  for (int q = 0; q < 36; ++q) D[q] = h[q];
+  for (int t = 0; t < 3; ++t) {
+    const int o = base + t;
+    if (o < 36) {
+      const double x = diag && o % 7 == 0 ? h[t] + F.damping : h[t];
+      H[36 * (size_t)blk + o] = (float)x;
+      if (diag) Hd[36 * (size_t)a + o] = x;
+    } else if (o < 42 && diag) {
+      rhs[6 * a + o - 36] = h[t];
+    }
+  }
 }
 #define DM_ASM_BOUNDS __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 __global__ DM_ASM_BOUNDS void k_nr_assemble(const int *__restrict__ blk_a, const int *__restrict__ blk_b,

@@ -159,3 +159,36 @@ def test_raycast_outputs_in_chunks(room, rows, cols):
     only = np.full((rows, cols, 3), 7, np.float32)
     N.check(N.lib().dm_volume_raycast(vol._h, N.ptr(Tf), C.byref(configs.sensor(sens)), None, None, N.ptr(only), None))
     np.testing.assert_array_equal(only, n)
+
+
+# One Gauss-Newton step against the FP64 oracle on random clouds (normals in
+# every direction, so that every motion is observable and the step is unique):
+# 5 nodes, 16 (one workgroup of the PCG), 17 (one node in a second), and 300,
+# some of whose rows have more than 16 blocks.  PCG runs to its tolerance.  The GPU
+# stores the blocks in FP32 (6e-8 relative); with the damping and the weights
+# here the systems' condition numbers stay below 1e4, so 1e-3 of the largest
+# motion bounds the difference.
+@pytest.mark.parametrize("nodes", [5, 16, 17, 300])
+def test_nonrigid_step_node_counts(nodes):
+    import oracle_lib as O
+    from test_oracle_nonrigid import random_cloud
+    V, Nn = random_cloud(6000, 11)
+    ids = np.linspace(0, len(V) - 1, nodes).astype(np.int32)
+    lo, hi = V.min(0), V.max(0)
+    size = float((hi - lo).max())
+    dgw = 2.0 * size / nodes ** (1 / 3)
+    g = dm.DefGraph(V, Nn, dgw=dgw, node_ids=ids)
+    o = O.OracleGraph(V, Nn, dgw=dgw, bits=64, node_ids=ids)
+    shift = 0.004 * np.stack([np.sin(V[:, 1] / size * 3), np.cos(V[:, 2] / size * 3), np.sin(V[:, 0] / size * 3)], 1)
+    target = (V + shift).astype(np.float32)
+    kw = dict(gn_iterations=1, pcg_iterations=400, pcg_tol=1e-9, damping=1.0)
+    dm.NonRigidICP(**kw).solve_mesh(g, target, Nn, np.eye(4))
+    o.solve_mesh(target, Nn, np.eye(4), **kw)
+    Tg, To = g.transforms(), o.transforms().reshape(-1, 4, 4)
+    moved = np.abs(To - np.eye(4)).max()
+    assert moved > 1e-4
+    assert np.abs(Tg - To).max() <= 1e-3 * moved
+    if nodes == 300:  # the longest row, from the vertices' node pairs, has more than 16 blocks
+        nn = g.vertex_neighbours()[0]
+        pairs = np.unique(np.concatenate([nn[:, [a, b]] for a in range(4) for b in range(4)]), axis=0)
+        assert np.bincount(pairs[:, 0]).max() > 16
