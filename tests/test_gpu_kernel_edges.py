@@ -192,3 +192,30 @@ def test_nonrigid_step_node_counts(nodes):
         nn = g.vertex_neighbours()[0]
         pairs = np.unique(np.concatenate([nn[:, [a, b]] for a in range(4) for b in range(4)]), axis=0)
         assert np.bincount(pairs[:, 0]).max() > 16
+
+
+# Nearest nodes where a query's lanes change in number (64 below 16384 queries,
+# 8 below 65536, then 1) and where the nodes fill, miss and pass a tile of 1024.
+# Whole coordinates: squared distances are exact and full of ties, which go to
+# the lower index.
+@pytest.mark.parametrize("nodes,verts", [(5, 16383), (1023, 16384), (1025, 65535), (1024, 65536), (2049, 300)])
+def test_nearest_nodes_lanes_and_ties(nodes, verts):
+    rng = np.random.default_rng(nodes + verts)
+    cell = rng.permutation(41 ** 3)[:max(verts, nodes)]
+    V = np.stack([cell // 1681, cell // 41 % 41, cell % 41], 1).astype(np.float32)
+    Nn = np.tile(np.float32([0, 0, 1]), (len(V), 1))
+    ids = rng.permutation(len(V))[:nodes].astype(np.int32)
+    g = dm.DefGraph(V, Nn, dgw=20.0, node_ids=ids)
+    vid, nbr, _ = g.nodes()
+    P, Q = V.astype(np.int64), V[vid].astype(np.int64)
+
+    def expect(rows, own):
+        key = (((rows[:, None] - Q[None]) ** 2).sum(2)) * nodes + np.arange(nodes)
+        if own is not None:
+            key[np.arange(len(rows)), own] = 1 << 40
+        return np.sort(np.partition(key, 3, 1)[:, :4], 1) % nodes
+
+    np.testing.assert_array_equal(nbr, expect(Q, np.arange(nodes)))
+    vnn = g.vertex_neighbours()[0]
+    for a in range(0, len(P), 8192):
+        np.testing.assert_array_equal(vnn[a:a + 8192], expect(P[a:a + 8192], None))
