@@ -8,15 +8,15 @@
 // Passes (all on the volume's stream):
 //   1. gather the per-bucket occupancy counts, exclusive-scan them, and write
 //      the pool index of every occupied slot at its canonical position;
-//   2. k_mc_count: one workgroup per block, one thread per cell.  The block's
-//      voxels plus a one-voxel halo (10^3 sdf values and observed flags) are
-//      staged in LDS; each cell takes its 8 strict trilinear corner samples
-//      from there, stores its cube index (0 = no triangles) and the
-//      workgroup sums the triangle count of the block;
+//   2. k_mc_count: one wavefront per block.  The block's voxels plus a
+//      one-voxel halo (10^3 sdf values, and bit rows of observed and sign) are
+//      staged in LDS; cells that can hold a surface are listed, take their 8
+//      strict trilinear corner samples from there and store their cube index
+//      (0 = no triangles), and the block's triangles are summed;
 //   3. exclusive scan of the per-block counts;
-//   4. k_mc_emit: blocks with triangles rescan their cells' counts in LDS,
-//      recompute the corner samples of active cells, and write positions,
-//      colours and edge ids at their canonical offset.
+//   4. k_mc_emit: blocks with triangles recompute the corner samples of their
+//      cells, scan the cells' counts, and write positions, colours and edge ids
+//      at their canonical offset.
 // Cell rules (K): cell centre g * vs, corners at +-vs/2, strict trilinear
 // samples (any corner voxel of weight 0 gives no sample), the reference's
 // corner-bit convention, Bourke's tables, the 1e-5 snaps of
@@ -44,7 +44,6 @@ __constant__ int8_t c_edge_axis[12] = {0, 1, 0, 1, 0, 1, 0, 1, 2, 2, 2, 2};
 __constant__ uint8_t c_corner_bit[8] = {8, 128, 1, 16, 4, 64, 2, 32};
 
 constexpr int kHalo = 10;         // block edge + one voxel each side
-constexpr int kCellThreads = 512;
 
 __global__ __launch_bounds__(256) void k_gather_counts(const DmView *__restrict__ vp, int *__restrict__ counts) {
   const DmView &v = *vp;
@@ -66,58 +65,18 @@ __global__ __launch_bounds__(256) void k_block_list(const DmView *__restrict__ v
 }
 
 // ---------------------------------------------------------------- cells
-struct Halo {
-  float sdf[kHalo * kHalo * kHalo];
-  uint8_t obs[kHalo * kHalo * kHalo];
-  int nb[27];
-};
-
-// Stage the block's voxels and a one-voxel halo.  All threads call it.
-__device__ void load_halo(const DmView &v, int kx, int ky, int kz, Halo &H) {
-  const int t = threadIdx.x;
-  if (t < 27) H.nb[t] = find_block(v, kx + t % 3 - 1, ky + (t / 3) % 3 - 1, kz + t / 9 - 1);
-  __syncthreads();
-  for (int h = t; h < kHalo * kHalo * kHalo; h += blockDim.x) {
-    const int lx = h / 100 - 1, ly = (h / 10) % 10 - 1, lz = h % 10 - 1;
-    const int ox = lx < 0 ? 0 : (lx > 7 ? 2 : 1), oy = ly < 0 ? 0 : (ly > 7 ? 2 : 1), oz = lz < 0 ? 0 : (lz > 7 ? 2 : 1);
-    const int ptr = H.nb[ox + 3 * oy + 9 * oz];
-    uint64_t w = 0;
-    if (ptr >= 0) w = v.vox[(size_t)ptr * kBlockVox + ((lx + 8) & 7) * 64 + ((ly + 8) & 7) * 8 + ((lz + 8) & 7)];
-    H.sdf[h] = vox_sdf(w);
-    H.obs[h] = (uint8_t)((w >> 56) != 0);
-  }
-  __syncthreads();
-}
-
-// Voxel at global index g: from the halo when inside it, else from the table.
-__device__ __forceinline__ bool halo_voxel(const DmView &v, const Halo &H, int kx, int ky, int kz, int gx, int gy,
-                                           int gz, float &sdf) {
-  const int hx = gx - 8 * kx + 1, hy = gy - 8 * ky + 1, hz = gz - 8 * kz + 1;
-  if ((unsigned)hx < kHalo && (unsigned)hy < kHalo && (unsigned)hz < kHalo) {
-    const int h = hx * 100 + hy * 10 + hz;
-    sdf = H.sdf[h];
-    return H.obs[h] != 0;
-  }
-  BlockCache bc;
-  bc.init();
-  const uint64_t w = voxel_at(v, gx, gy, gz, bc);
-  sdf = vox_sdf(w);
-  return (w >> 56) != 0;
-}
-
 struct BoxArg {
   int use;
   double lo[3], hi[3];
 };
 
-// Corner positions and samples of cell (gx, gy, gz); false when the cell is
-// outside the box or a sample is missing.  Each sample is
-// TrilinearInterpolation (meshExtractor.cu:22-93), strict: false when any of
-// its 8 voxels is unobserved.  The corner samples sit at c +- vs/2 per axis,
-// and every per-axis quantity of the interpolation (the voxel indices of
+// Each corner sample is TrilinearInterpolation (meshExtractor.cu:22-93), strict:
+// none when any of its 8 voxels is unobserved.  The samples sit at c +- vs/2 per
+// axis, and every per-axis quantity of the interpolation (the voxel indices of
 // dual = p - vs/2 and dual + vs, the weight p/vs - floor(p/vs)) depends only
-// on the axis and the sign, so it is evaluated once per (axis, sign) and
-// combined: the same arithmetic as interpolating each corner on its own.
+// on the axis, the cell's coordinate on it and the sign: 48 values per block,
+// evaluated once by 48 lanes, where each cell combines 6 of them with the same
+// arithmetic as interpolating each corner on its own.
 struct AxisCorner {
   float p;     // corner coordinate c +- vs/2
   int i0, i1;  // voxel indices of dual + 0 and dual + vs
@@ -134,94 +93,245 @@ __device__ __forceinline__ AxisCorner axis_corner(float c, float off, float vs) 
   return a;
 }
 
-__device__ __forceinline__ bool halo_axis_ok(const AxisCorner *A, int k) {
-  const int lo = 8 * k - 1, hi = 8 * k + 8;
-  return A[0].i0 >= lo && A[0].i1 >= lo && A[1].i0 >= lo && A[1].i1 >= lo && A[0].i0 <= hi && A[0].i1 <= hi &&
-         A[1].i0 <= hi && A[1].i1 <= hi;
+// Orders a wavefront's LDS writes before its later reads by other lanes.
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// The 8 corner samples of a cell (kWant: positions and values, else only
-// the cube index).  Each voxel comes from the block's LDS halo; a cell whose
-// indices leave the halo (only through rounding at huge coordinates) reads
-// them through the hash table in a rolled loop.
-template <bool kWant>
-__device__ __forceinline__ bool cell_eval(const DmView &v, const Halo &H, int kx, int ky, int kz, int gx, int gy,
-                                          int gz, const BoxArg &box, f3 *pc, float *d, int &cube) {
-  const float vs = v.voxel_size;
-  const f3 c = mk((float)gx * vs + 0.f, (float)gy * vs + 0.f, (float)gz * vs + 0.f);
-  if (box.use && ((double)c.x < box.lo[0] || (double)c.y < box.lo[1] || (double)c.z < box.lo[2] ||
-                  (double)c.x > box.hi[0] || (double)c.y > box.hi[1] || (double)c.z > box.hi[2]))
-    return false;
-  const float P = vs / 2.f, M = -P;
-  const AxisCorner X[2] = {axis_corner(c.x, M, vs), axis_corner(c.x, P, vs)};
-  const AxisCorner Y[2] = {axis_corner(c.y, M, vs), axis_corner(c.y, P, vs)};
-  const AxisCorner Z[2] = {axis_corner(c.z, M, vs), axis_corner(c.z, P, vs)};
-  // corner c: offsets (cx, cy, cz) = (0,0,0) (1,0,0) (0,1,0) (0,0,1) (1,1,0) (0,1,1) (1,0,1) (1,1,1)
-  constexpr uint8_t cxm = 0xD2, cym = 0xB4, czm = 0xE8;
-  cube = 0;
-  if (halo_axis_ok(X, kx) && halo_axis_ok(Y, ky) && halo_axis_ok(Z, kz)) {
-    const int bx = 1 - 8 * kx, by = 1 - 8 * ky, bz = 1 - 8 * kz;
+// A wavefront holds one block: its voxels and a one-voxel halo, the per-axis
+// corner values, and the list of cells that are worth evaluating.  rows[r] has,
+// for the 10 voxels of row r = (x + 1) * 10 + (y + 1), observed in bits 0..9,
+// sdf >= 0 in 10..19 and sdf <= -1e-30 in 20..29.
+constexpr uint32_t kRowObs = 1u, kRowPos = 1u << 10, kRowNeg = 1u << 20;
+struct Cells {
+  float sdf[kHalo * kHalo * kHalo];
+  uint32_t rows[kHalo * kHalo];
+  AxisCorner ax[3][8][2];  // [axis][cell][sign]
+  uint16_t list[kBlockVox];
+};
+constexpr int kMcWaves = 4;  // wavefronts per workgroup
+
+// Loads the block.  False when no cell can give a triangle: a cell's first
+// corner sample reads its own voxel, so a block without an observed voxel is
+// left before its halo is read.  `regular`: every cell samples exactly its own
+// voxel and the 26 around it, with weights in [0.25, 0.75] (true but for
+// coordinates so large that rounding moves them).
+__device__ __forceinline__ bool load_cells(const DmView &v, int ptr, Cells &C, bool &regular) {
+  const int lane = threadIdx.x & 63;
+  const int4 key = v.block_key[ptr];
+  const uint64_t *own = v.vox + (size_t)ptr * kBlockVox;
+  uint64_t w[8];
 #pragma unroll
-    for (int ci = 0; ci < 8; ++ci) {
-      const AxisCorner &ax = X[(ci >> 2) & 1], &ay = Y[(ci >> 1) & 1], &az = Z[ci & 1];
-      float dd = 0.f;
+  for (int x = 0; x < 8; ++x) w[x] = ldg(own + 64 * x + lane);
+  int nb = -1;
+  if (lane < 27) nb = find_block(v, key.x + lane % 3 - 1, key.y + (lane / 3) % 3 - 1, key.z + lane / 9 - 1);
+  bool any = false;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const bool ox = (cxm >> k) & 1, oy = (cym >> k) & 1, oz = (czm >> k) & 1;
-        const int h = ((ox ? ax.i1 : ax.i0) + bx) * 100 + ((oy ? ay.i1 : ay.i0) + by) * 10 + (oz ? az.i1 : az.i0) + bz;
-        if (!H.obs[h]) return false;
-        const float a = ox ? ax.w : 1.f - ax.w;
-        const float b = oy ? ay.w : 1.f - ay.w;
-        const float g = oz ? az.w : 1.f - az.w;
-        dd += a * b * g * H.sdf[h];
-      }
-      if (kWant) { pc[ci] = mk(ax.p, ay.p, az.p); d[ci] = dd; }
-      if (dd < 0.f) cube += c_corner_bit[ci];
+  for (int x = 0; x < 8; ++x) any |= (w[x] >> 56) != 0;
+  if (!__ballot(any)) return false;
+  // the halo: 128 ends of the block's own rows, then 36 whole rows of 10
+  uint64_t hw[8];
+  int hr[8], hz[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int e = min(64 * k + lane, 487);
+    int x, y, z;
+    if (k < 2) {
+      x = 1 + (e >> 4);
+      y = 1 + ((e >> 1) & 7);
+      z = (e & 1) * 9;
+    } else {
+      const int q = (e - 128) / 10;
+      z = (e - 128) - 10 * q;
+      x = q < 20 ? (q < 10 ? 0 : 9) : 1 + ((q - 20) >> 1);
+      y = q < 20 ? (q < 10 ? q : q - 10) : (q & 1) * 9;
     }
-    return true;
+    const int o = (x + 7) / 8 + 3 * ((y + 7) / 8) + 9 * ((z + 7) / 8);
+    const int hp = __shfl(nb, o, 64);
+    const uint64_t word = ldg(v.vox + ((size_t)(hp >= 0 ? hp : ptr) * kBlockVox + ((x + 7) & 7) * 64 +
+                                       ((y + 7) & 7) * 8 + ((z + 7) & 7)));
+    hw[k] = hp >= 0 ? word : 0ull;
+    hr[k] = x * 10 + y;
+    hz[k] = z;
   }
+  const float vs = v.voxel_size;
+  bool ok = true;
+  if (lane < 48) {
+    const int axis = lane >> 4, l = (lane >> 1) & 7, sign = lane & 1;
+    const int g = (axis == 0 ? key.x : axis == 1 ? key.y : key.z) * 8 + l;
+    const float P = vs / 2.f;
+    const AxisCorner a = axis_corner((float)g * vs + 0.f, sign ? P : -P, vs);
+    C.ax[axis][l][sign] = a;
+    ok = a.i0 == g - 1 + sign && a.i1 == g + sign && a.w >= 0.25f && a.w <= 0.75f;
+  }
+  regular = __ballot(!ok) == 0;
+  for (int r = lane; r < kHalo * kHalo; r += 64) C.rows[r] = 0;
+  wave_lds();
+  // the block's own rows: lane = 8 y + z, so a ballot's byte y is a row
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const float s = vox_sdf(w[x]);
+    const int sh = lane & 56;
+    const uint32_t o = (uint32_t)(__ballot((w[x] >> 56) != 0) >> sh) & 0xFF;
+    const uint32_t p = (uint32_t)(__ballot(s >= 0.f) >> sh) & 0xFF;
+    const uint32_t n = (uint32_t)(__ballot(s <= -1e-30f) >> sh) & 0xFF;
+    const int r = (x + 1) * 10 + (lane >> 3) + 1;
+    C.sdf[r * 10 + (lane & 7) + 1] = s;
+    if ((lane & 7) == 0) C.rows[r] = (o << 1) | (p << 11) | (n << 21);
+  }
+  wave_lds();
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (64 * k + lane < 488) {
+      const float s = vox_sdf(hw[k]);
+      C.sdf[hr[k] * 10 + hz[k]] = s;
+      const uint32_t bits = ((hw[k] >> 56) ? kRowObs : 0u) | (s >= 0.f ? kRowPos : 0u) | (s <= -1e-30f ? kRowNeg : 0u);
+      atomicOr(&C.rows[hr[k]], bits << hz[k]);
+    }
+  wave_lds();
+  return true;
+}
+
+// Lists the block's cells whose 27 voxels are all observed and neither all
+// >= 0 (every corner sample is then >= 0: cube 0) nor all below zero (cube
+// 255), in cell order; all cells of a block that is not regular.
+__device__ __forceinline__ int list_cells(Cells &C, bool regular) {
+  const int lane = threadIdx.x & 63, y = lane >> 3, z = lane & 7;
+  uint32_t m[kHalo];
+#pragma unroll
+  for (int x = 0; x < kHalo; ++x) m[x] = C.rows[x * 10 + y] & C.rows[x * 10 + y + 1] & C.rows[x * 10 + y + 2];
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  int n = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const uint32_t t = (m[x] & m[x + 1] & m[x + 2]) >> z;
+    const bool take = !regular || ((t & 7) == 7 && ((t >> 10) & 7) != 7 && ((t >> 20) & 7) != 7);
+    const uint64_t b = __ballot(take);
+    if (take) C.list[n + __popcll(b & below)] = (uint16_t)(64 * x + lane);
+    n += __popcll(b);
+  }
+  wave_lds();
+  return n;
+}
+
+// The 8 corner samples of a listed cell of a regular block.
+__device__ __forceinline__ int cell_samples(const Cells &C, int li, float *d) {
+  const int lx = li >> 6, ly = (li >> 3) & 7, lz = li & 7;
+  float s[27];
+#pragma unroll
+  for (int k = 0; k < 27; ++k) s[k] = C.sdf[(lx + k / 9) * 100 + (ly + (k / 3) % 3) * 10 + lz + k % 3];
+  const float wx[2] = {C.ax[0][lx][0].w, C.ax[0][lx][1].w}, wy[2] = {C.ax[1][ly][0].w, C.ax[1][ly][1].w},
+              wz[2] = {C.ax[2][lz][0].w, C.ax[2][lz][1].w};
+  // sample k: offsets (0,0,0) (1,0,0) (0,1,0) (0,0,1) (1,1,0) (0,1,1) (1,0,1) (1,1,1)
+  constexpr uint8_t cxm = 0xD2, cym = 0xB4, czm = 0xE8;
+  int cube = 0;
+#pragma unroll
+  for (int ci = 0; ci < 8; ++ci) {
+    const int cx = (ci >> 2) & 1, cy = (ci >> 1) & 1, cz = ci & 1;
+    float dd = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int ox = (cxm >> k) & 1, oy = (cym >> k) & 1, oz = (czm >> k) & 1;
+      const float a = ox ? wx[cx] : 1.f - wx[cx];
+      const float b = oy ? wy[cy] : 1.f - wy[cy];
+      const float g = oz ? wz[cz] : 1.f - wz[cz];
+      dd += a * b * g * s[(cx + ox) * 9 + (cy + oy) * 3 + cz + oz];
+    }
+    d[ci] = dd;
+    if (dd < 0.f) cube += c_corner_bit[ci];
+  }
+  return cube;
+}
+
+// Voxel at global index g: from the halo when inside it, else from the table.
+__device__ __forceinline__ bool halo_voxel(const DmView &v, const Cells &C, int4 key, int gx, int gy, int gz,
+                                           float &sdf) {
+  const int hx = gx - 8 * key.x + 1, hy = gy - 8 * key.y + 1, hz = gz - 8 * key.z + 1;
+  if ((unsigned)hx < kHalo && (unsigned)hy < kHalo && (unsigned)hz < kHalo) {
+    sdf = C.sdf[hx * 100 + hy * 10 + hz];
+    return (C.rows[hx * 10 + hy] >> hz) & 1;
+  }
+  BlockCache bc;
+  bc.init();
+  const uint64_t w = voxel_at(v, gx, gy, gz, bc);
+  sdf = vox_sdf(w);
+  return (w >> 56) != 0;
+}
+
+// The same samples for any indices and weights; -1 when a sample is missing.
+__device__ __noinline__ int cell_samples_any(const DmView &v, const Cells &C, int4 key, int li, float *d, int stride) {
+  const AxisCorner *X = C.ax[0][li >> 6], *Y = C.ax[1][(li >> 3) & 7], *Z = C.ax[2][li & 7];
+  constexpr uint8_t cxm = 0xD2, cym = 0xB4, czm = 0xE8;
+  int cube = 0;
 #pragma unroll 1
   for (int ci = 0; ci < 8; ++ci) {
-    const AxisCorner &ax = X[(ci >> 2) & 1], &ay = Y[(ci >> 1) & 1], &az = Z[ci & 1];
+    const AxisCorner ax = X[(ci >> 2) & 1], ay = Y[(ci >> 1) & 1], az = Z[ci & 1];
     float dd = 0.f;
 #pragma unroll 1
     for (int k = 0; k < 8; ++k) {
       const bool ox = (cxm >> k) & 1, oy = (cym >> k) & 1, oz = (czm >> k) & 1;
       float sv;
-      if (!halo_voxel(v, H, kx, ky, kz, ox ? ax.i1 : ax.i0, oy ? ay.i1 : ay.i0, oz ? az.i1 : az.i0, sv)) return false;
+      if (!halo_voxel(v, C, key, ox ? ax.i1 : ax.i0, oy ? ay.i1 : ay.i0, oz ? az.i1 : az.i0, sv)) return -1;
       const float a = ox ? ax.w : 1.f - ax.w;
       const float b = oy ? ay.w : 1.f - ay.w;
       const float g = oz ? az.w : 1.f - az.w;
       dd += a * b * g * sv;
     }
-    if (kWant) { pc[ci] = mk(ax.p, ay.p, az.p); d[ci] = dd; }
+    if (d) d[ci * stride] = dd;
     if (dd < 0.f) cube += c_corner_bit[ci];
   }
-  return true;
+  return cube;
 }
 
+__device__ __forceinline__ bool outside_box(const BoxArg &box, int gx, int gy, int gz, float vs) {
+  const f3 c = mk((float)gx * vs + 0.f, (float)gy * vs + 0.f, (float)gz * vs + 0.f);
+  return (double)c.x < box.lo[0] || (double)c.y < box.lo[1] || (double)c.z < box.lo[2] ||
+         (double)c.x > box.hi[0] || (double)c.y > box.hi[1] || (double)c.z > box.hi[2];
+}
 
-__global__ __launch_bounds__(kCellThreads) void k_mc_count(const DmView *__restrict__ vp, const int *__restrict__ list,
-                                                           BoxArg box, uint8_t *__restrict__ cubes,
+// Bound by memory latency (the block's key, its neighbours' pool entries,
+// then their voxels), so a block takes one wavefront with all its loads in
+// flight, and as many blocks as registers and LDS allow are resident.  Cells
+// without a sign change or with an unobserved voxel, nearly all, are dropped
+// on bit masks; the others are packed into full wavefronts.
+__global__ __launch_bounds__(64 * kMcWaves) void k_mc_count(const DmView *__restrict__ vp, const int *__restrict__ list,
+                                                           int n, BoxArg box, uint8_t *__restrict__ cubes,
                                                            int *__restrict__ block_tri) {
-  __shared__ Halo H;
-  __shared__ int red[kCellThreads / 64 + 1];
+  __shared__ Cells S[kMcWaves];
+  __shared__ uint64_t out[kMcWaves][kBlockVox / 8];
   const DmView &v = *vp;
-  const int ptr = list[blockIdx.x];
-  const int4 key = v.block_key[ptr];
-  load_halo(v, key.x, key.y, key.z, H);
-  const int li = threadIdx.x;
-  const int gx = key.x * 8 + (li >> 6), gy = key.y * 8 + ((li >> 3) & 7), gz = key.z * 8 + (li & 7);
-  int cube = 0, ntri = 0, cb;
-  if (cell_eval<false>(v, H, key.x, key.y, key.z, gx, gy, gz, box, nullptr, nullptr, cb)) {
-    cube = cb;
-    ntri = mc_num_tri(c_mc_tri[cube]);
-    if (ntri == 0) cube = 0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int blk = blockIdx.x * kMcWaves + wave;
+  if (blk >= n) return;
+  Cells &C = S[wave];
+  const int ptr = list[blk];
+  bool regular;
+  int cells = 0;
+  if (load_cells(v, ptr, C, regular)) cells = list_cells(C, regular);
+  int ntri = 0;
+  if (cells) {
+    const int4 key = v.block_key[ptr];
+    uint8_t *cb = (uint8_t *)out[wave];
+    out[wave][lane] = 0;
+    wave_lds();
+    for (int k = lane; k < cells; k += 64) {
+      const int li = C.list[k];
+      if (box.use &&
+          outside_box(box, key.x * 8 + (li >> 6), key.y * 8 + ((li >> 3) & 7), key.z * 8 + (li & 7), v.voxel_size))
+        continue;
+      float d[8];
+      const int cube = regular ? cell_samples(C, li, d) : cell_samples_any(v, C, key, li, nullptr, 0);
+      const int nt = cube > 0 ? mc_num_tri(c_mc_tri[cube]) : 0;
+      if (nt) cb[li] = (uint8_t)cube;
+      ntri += nt;
+    }
+    wave_lds();
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ntri += __shfl_xor(ntri, o, 64);
+    if (ntri) ((uint64_t *)(cubes + (size_t)blk * kBlockVox))[lane] = out[wave][lane];  // else never read
   }
-  cubes[(size_t)blockIdx.x * kBlockVox + li] = (uint8_t)cube;
-  int tot;
-  wg_exclusive_scan<kCellThreads>(ntri, red, tot);
-  if (li == 0) block_tri[blockIdx.x] = tot;
+  if (lane == 0) block_tri[blk] = ntri;
 }
 
 // VertexInterpolation at isolevel 0 (meshExtractor.cu:95-123)
@@ -243,47 +353,91 @@ __device__ __forceinline__ uint64_t edge_id(int gx, int gy, int gz, int e) {
          ((((uint64_t)(cy + (int)off)) & m) << 20) | (((uint64_t)(cz + (int)off)) & m);
 }
 
-__global__ __launch_bounds__(kCellThreads) void k_mc_emit(const DmView *__restrict__ vp, const int *__restrict__ list,
-                                                          BoxArg box, const uint8_t *__restrict__ cubes,
+// A wavefront per block with triangles.  64 of its cells at a time leave their
+// corner samples in LDS; then a lane takes a vertex, so that neighbouring
+// lanes write neighbouring vertices.
+__global__ __launch_bounds__(64 * kMcWaves) void k_mc_emit(const DmView *__restrict__ vp, const int *__restrict__ list,
+                                                          int n, const uint8_t *__restrict__ cubes,
                                                           const int *__restrict__ block_tri,
                                                           const long long *__restrict__ block_off, long long cap,
                                                           float *__restrict__ pos, float *__restrict__ col,
                                                           uint64_t *__restrict__ eid) {
-  if (block_tri[blockIdx.x] == 0 || block_off[blockIdx.x] >= cap) return;  // uniform per workgroup
-  __shared__ Halo H;
-  __shared__ int red[kCellThreads / 64 + 1];
+  __shared__ Cells S[kMcWaves];
+  __shared__ float D[kMcWaves][8][64];       // [corner][cell of this pass]
+  __shared__ uint16_t tri[kMcWaves][64 * 5];  // triangle -> cell of this pass | number in the cell << 8
   const DmView &v = *vp;
-  const int ptr = list[blockIdx.x];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int blk = blockIdx.x * kMcWaves + wave;
+  if (blk >= n || block_tri[blk] == 0 || block_off[blk] >= cap) return;
+  Cells &C = S[wave];
+  const int ptr = list[blk];
   const int4 key = v.block_key[ptr];
-  load_halo(v, key.x, key.y, key.z, H);
-  const int li = threadIdx.x;
-  const int cube = cubes[(size_t)blockIdx.x * kBlockVox + li];
-  const uint64_t word = c_mc_tri[cube];
-  const int ntri = cube ? mc_num_tri(word) : 0;
-  int tot;
-  const long long t0 = block_off[blockIdx.x] + wg_exclusive_scan<kCellThreads>(ntri, red, tot);
-  if (ntri == 0 || t0 >= cap) return;
-  const int gx = key.x * 8 + (li >> 6), gy = key.y * 8 + ((li >> 3) & 7), gz = key.z * 8 + (li & 7);
-  f3 pc[8];
-  float d[8];
-  int cube_e;
-  cell_eval<true>(v, H, key.x, key.y, key.z, gx, gy, gz, box, pc, d, cube_e);  // true: the count pass kept it
-  const uint32_t rgbw = vox_rgbw(v.vox[(size_t)ptr * kBlockVox + li]);
-  const float cr = (float)(rgbw & 0xFF) / 255.f, cg = (float)((rgbw >> 8) & 0xFF) / 255.f,
-              cb = (float)((rgbw >> 16) & 0xFF) / 255.f;
-  for (int k = 0; k < ntri; ++k) {
-    const long long t = t0 + k;
-    if (t >= cap) break;
+  const uint8_t *cb = cubes + (size_t)blk * kBlockVox;
+  uint8_t cube_of[8];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int e = mc_tri_edge(word, 3 * k + j);
-      const int a = c_edge_a[e], b = c_edge_b[e];
-      const f3 p = vertex_interp(pc[a], pc[b], d[a], d[b]);
-      const size_t o = (size_t)t * 9 + 3 * j;
-      if (pos) { pos[o] = p.x; pos[o + 1] = p.y; pos[o + 2] = p.z; }
-      if (col) { col[o] = cr; col[o + 1] = cg; col[o + 2] = cb; }
-      if (eid) eid[(size_t)t * 3 + j] = edge_id(gx, gy, gz, e);
+  for (int x = 0; x < 8; ++x) cube_of[x] = ldg(cb + 64 * x + lane);
+  bool regular;
+  if (!load_cells(v, ptr, C, regular)) return;  // the count pass saw observed voxels
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  int cells = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const uint64_t b = __ballot(cube_of[x] != 0);
+    if (cube_of[x]) C.list[cells + __popcll(b & below)] = (uint16_t)(64 * x + lane);
+    cells += __popcll(b);
+  }
+  wave_lds();
+  long long t0 = block_off[blk];
+  for (int c0 = 0; c0 < cells; c0 += 64) {
+    const bool have = c0 + lane < cells;
+    int nt = 0;
+    if (have) {
+      const int li = C.list[c0 + lane];
+      nt = mc_num_tri(c_mc_tri[cb[li]]);
+      if (regular) {
+        float d[8];
+        cell_samples(C, li, d);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) D[wave][k][lane] = d[k];
+      } else {
+        cell_samples_any(v, C, key, li, &D[wave][0][lane], 64);
+      }
     }
+    int incl = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += u;
+    }
+    for (int k = 0; k < nt; ++k) tri[wave][incl - nt + k] = (uint16_t)(lane | k << 8);
+    const int total = __shfl(incl, 63, 64);
+    wave_lds();
+    const int lim = (int)min((long long)total, cap - t0);  // triangles past cap are not written
+    for (int q = lane; q < 3 * lim; q += 64) {
+      const int e3 = tri[wave][q / 3], c = e3 & 0xFF, li = C.list[c0 + c];
+      const int e = mc_tri_edge(c_mc_tri[cb[li]], 3 * (e3 >> 8) + q % 3);
+      const int ea = c_edge_a[e], eb = c_edge_b[e];
+      const int lx = li >> 6, ly = (li >> 3) & 7, lz = li & 7;
+      const size_t o = (size_t)t0 * 3 + q;
+      if (pos) {
+        const f3 pa = mk(C.ax[0][lx][(ea >> 2) & 1].p, C.ax[1][ly][(ea >> 1) & 1].p, C.ax[2][lz][ea & 1].p);
+        const f3 pb = mk(C.ax[0][lx][(eb >> 2) & 1].p, C.ax[1][ly][(eb >> 1) & 1].p, C.ax[2][lz][eb & 1].p);
+        const f3 p = vertex_interp(pa, pb, D[wave][ea][c], D[wave][eb][c]);
+        pos[3 * o] = p.x;
+        pos[3 * o + 1] = p.y;
+        pos[3 * o + 2] = p.z;
+      }
+      if (col) {
+        const uint32_t rgbw = vox_rgbw(v.vox[(size_t)ptr * kBlockVox + li]);
+        col[3 * o] = (float)(rgbw & 0xFF) / 255.f;
+        col[3 * o + 1] = (float)((rgbw >> 8) & 0xFF) / 255.f;
+        col[3 * o + 2] = (float)((rgbw >> 16) & 0xFF) / 255.f;
+      }
+      if (eid) eid[o] = edge_id(8 * key.x + lx, 8 * key.y + ly, 8 * key.z + lz, e);
+    }
+    wave_lds();
+    t0 += total;
+    if (t0 >= cap) break;
   }
 }
 
@@ -398,7 +552,8 @@ int dm_mesh_extract(dm_volume *vol, const double *box_lo, const double *box_hi, 
   if (int rc = dev_alloc(boff, (size_t)n * 8)) return rc;
   hipLaunchKernelGGL(k_block_list, dim3((nb + 255) / 256), dim3(256), 0, st, vol->d_view, offs.as<long long>(),
                      list.as<int>());
-  hipLaunchKernelGGL(k_mc_count, dim3(n), dim3(kCellThreads), 0, st, vol->d_view, list.as<int>(), box,
+  hipLaunchKernelGGL(k_mc_count, dim3((n + kMcWaves - 1) / kMcWaves), dim3(64 * kMcWaves), 0, st, vol->d_view,
+                     list.as<int>(), n, box,
                      cubes.as<uint8_t>(), btri.as<int>());
   DM_HIP(hipGetLastError());
   long long *d_ntri = nullptr;
@@ -412,7 +567,8 @@ int dm_mesh_extract(dm_volume *vol, const double *box_lo, const double *box_hi, 
   if (pos) { if (int rc = dev_alloc(dpos, (size_t)m * 36)) return rc; }
   if (col) { if (int rc = dev_alloc(dcol, (size_t)m * 36)) return rc; }
   if (edge_ids) { if (int rc = dev_alloc(deid, (size_t)m * 24)) return rc; }
-  hipLaunchKernelGGL(k_mc_emit, dim3(n), dim3(kCellThreads), 0, st, vol->d_view, list.as<int>(), box,
+  hipLaunchKernelGGL(k_mc_emit, dim3((n + kMcWaves - 1) / kMcWaves), dim3(64 * kMcWaves), 0, st, vol->d_view,
+                     list.as<int>(), n,
                      cubes.as<uint8_t>(), btri.as<int>(), boff.as<long long>(), m, dpos.as<float>(),
                      dcol.as<float>(), deid.as<uint64_t>());
   DM_HIP(hipGetLastError());
@@ -471,7 +627,8 @@ int dm_mesh_extract_noalloc(dm_volume *vol, const double *box_lo, const double *
   long long T = 0;
   for (int c0 = 0; c0 < n; c0 += kNaChunk) {
     const int cn = std::min(kNaChunk, n - c0);
-    hipLaunchKernelGGL(k_mc_count, dim3(cn), dim3(kCellThreads), 0, st, vol->d_view, list + c0, box, cubes, btri);
+    hipLaunchKernelGGL(k_mc_count, dim3((cn + kMcWaves - 1) / kMcWaves), dim3(64 * kMcWaves), 0, st, vol->d_view,
+                       list + c0, cn, box, cubes, btri);
     DM_HIP(hipGetLastError());
     DM_TRY(scan_ints_ws(btri, cn, boff, wsum2, st, &d_total));
     long long Tc = 0;
@@ -479,7 +636,8 @@ int dm_mesh_extract_noalloc(dm_volume *vol, const double *box_lo, const double *
     DM_HIP(hipStreamSynchronize(st));
     const long long m = std::min<long long>(Tc, cap - std::min<long long>(T, cap));
     if (want && m > 0) {
-      hipLaunchKernelGGL(k_mc_emit, dim3(cn), dim3(kCellThreads), 0, st, vol->d_view, list + c0, box, cubes, btri,
+      hipLaunchKernelGGL(k_mc_emit, dim3((cn + kMcWaves - 1) / kMcWaves), dim3(64 * kMcWaves), 0, st, vol->d_view,
+                         list + c0, cn, cubes, btri,
                          boff, m, dev_pos ? dev_pos + (size_t)T * 9 : nullptr,
                          dev_col ? dev_col + (size_t)T * 9 : nullptr,
                          dev_edge_ids ? dev_edge_ids + (size_t)T * 3 : nullptr);

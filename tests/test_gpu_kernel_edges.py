@@ -219,3 +219,38 @@ def test_nearest_nodes_lanes_and_ties(nodes, verts):
     vnn = g.vertex_neighbours()[0]
     for a in range(0, len(P), 8192):
         np.testing.assert_array_equal(vnn[a:a + 8192], expect(P[a:a + 8192], None))
+
+
+# Marching cubes at the origin, across it, and where float coordinates are so
+# coarse (0.0078 m at 80 km, voxels of 0.02 m) that a cell's samples leave the
+# voxels around it or change weight; caps that end inside a block.  Same order and the same bits as
+# the FP32 restatement.
+@pytest.mark.parametrize("shift,irregular", [((0.0, 0.0, 0.0), False), ((-1.3, 0.9, -2.1), False),
+                                            ((80000.0, 0.0, 0.0), True), ((0.0, -80000.0, 0.0), False),
+                                            ((0.0, 0.0, 81000.0), True)])
+def test_mesh_cells_near_and_far(room, shift, irregular):
+    import oracle_lib as O
+    from test_gpu_mesh import check_same, mirror as mirror_slots
+    depth, poses = room
+    P = shifted(poses, shift)
+    vol = dm.TsdfVolume(small_tsdf(), SENS["rows"], SENS["cols"])
+    vol.props = small_tsdf()
+    for f in range(3):
+        vol.IntegrateScan(depth[f], None, SENS, P[f].astype(np.float32))
+    vs, half = np.float32(vol.props["voxel_size"]), np.float32(0.5)
+    g = np.arange(8) + 8 * vol.blocks()[0][:, int(np.argmax(np.abs(shift))), None]
+    moved = False  # an index or a weight of a cell's samples, in the kernel's float operations
+    for sign in (0, 1):
+        p = g.astype(np.float32) * vs + (vs / 2 if sign else -vs / 2)
+        q = (p - vs / 2) / vs
+        w = p / vs - np.floor(p / vs)
+        moved |= bool(((np.trunc(q + np.sign(q) * half) != g - 1 + sign) | (w < 0.25) | (w > 0.75)).any())
+    assert moved == irregular
+    o = O.mc_extract(mirror_slots(vol))
+    m = vol.ExtractMesh(max_triangles=1 << 20)
+    assert irregular or len(m) > 1000
+    check_same((m.triangles, m.colors, m.edge_ids), o)
+    for cap in (1, 2, 67, 130):
+        c = dm.MeshExtractor(cap).ExtractMesh(vol)
+        assert c.num_triangles_ == len(m) and len(c) == min(cap, len(m))
+        check_same((c.triangles, c.colors, c.edge_ids), tuple(a[:cap] for a in o))
