@@ -135,7 +135,9 @@ int Sess::init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols) {
   DM_TRY(dalloc(&d_ray_rgb, P * 3));
   DM_TRY(dalloc(&d_view, 1));
   DM_TRY(dalloc(&d_active, 1));
-  pinned_bytes = P * 7 + 1024;
+  // a frame's depth and colour, or two chunks of results; then read_small's 1 KiB
+  out_half = std::max<size_t>((P * 7 / 2 + 63) & ~(size_t)63, 256 << 10);
+  pinned_bytes = 2 * out_half + 1024;
   DM_HIP(hipHostMalloc((void **)&h_pinned, pinned_bytes, hipHostMallocDefault));
   // identity poses
   double I[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
@@ -233,9 +235,12 @@ int Sess::reserve_out() {
 }
 
 // The results pass through the two halves of the frame's pinned buffer: while
-// one chunk is moved to the caller's memory, the next is on its way.
+// one chunk is moved to the caller's memory, the next is on its way.  A chunk
+// costs about 8 us beside its bytes, so a small frame's chunks are not cut
+// below 256 KiB: 200x166 pixels with colour in 11 chunks 392 us a render, in 6
+// chunks 320 us.
 int Sess::read_out(const Out *out, int n) {
-  const size_t half = ((size_t)max_rows * max_cols * 7 / 2 + 63) & ~(size_t)63;
+  const size_t half = out_half;
   struct Chunk { uint8_t *dst; const uint8_t *src; size_t bytes; };
   std::vector<Chunk> chunks;
   for (int k = 0; k < n; ++k)
@@ -259,7 +264,7 @@ int Sess::read_out(const Out *out, int n) {
 }
 
 int Sess::read_small(void *dst, const void *src, size_t bytes) {
-  uint8_t *slot = h_pinned + (((size_t)max_rows * max_cols * 7 + 191) & ~(size_t)63);  // past both halves
+  uint8_t *slot = h_pinned + 2 * out_half;  // past both halves
   DM_HIP(hipMemcpyAsync(slot, src, bytes, hipMemcpyDeviceToHost, stream));
   DM_HIP(hipStreamSynchronize(stream));
   memcpy(dst, slot, bytes);

@@ -41,6 +41,7 @@ struct Sess {
   uint8_t *d_rgb = nullptr;
   uint8_t *h_pinned = nullptr;   // pinned staging for host inputs
   size_t pinned_bytes = 0;
+  size_t out_half = 0;           // bytes of one half of it, for results
   float *d_ray_depth = nullptr;  // raycast outputs for host readback
   uint8_t *d_ray_rgb = nullptr;
   float *d_pack = nullptr;       // packed maps for host readback (7 floats per pixel, allocated on first use)

@@ -143,14 +143,18 @@ def test_integration_operand_range(room, scale):
 
 
 # Host results pass in chunks of half the frame's pinned buffer: images from
-# one pixel up, smaller than the volume's frame, every output and fewer of them.
-@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 5), (33, 31), (240, 320)])
-def test_raycast_outputs_in_chunks(room, rows, cols):
+# one pixel up, smaller than the volume's frame and as large, with the smallest
+# chunk (a frame of 200x166) and a larger one; every output and fewer of them.
+@pytest.mark.parametrize("rows,cols,frame", [(1, 1, (240, 320)), (3, 5, (240, 320)), (33, 31, (240, 320)),
+                                            (240, 320, (240, 320)), (166, 200, (166, 200)), (2, 1, (2, 1))])
+def test_raycast_outputs_in_chunks(room, rows, cols, frame):
     import ctypes as C
     from dynamap_amd import _native as N
     depth, poses = room
-    vol = dm.TsdfVolume(small_tsdf(), SENS["rows"], SENS["cols"])
-    vol.IntegrateScan(depth[0], None, SENS, poses[0].astype(np.float32))
+    vol = dm.TsdfVolume(small_tsdf(), *frame)
+    view = dict(SENS, rows=min(frame[0], SENS["rows"]), cols=min(frame[1], SENS["cols"]))
+    vol.IntegrateScan(np.ascontiguousarray(depth[0][:view["rows"], :view["cols"]]), None, view,
+                      poses[0].astype(np.float32))
     sens = dict(rows=rows, cols=cols, fx=0.8 * cols + 1, fy=0.8 * cols + 1, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
     Tf = np.ascontiguousarray(poses[0], np.float32)
     d, v, n, c = vol.Raycast(Tf, sens)
