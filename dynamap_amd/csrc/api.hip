@@ -111,8 +111,8 @@ int Sess::init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols) {
   DM_TRY(dalloc(&h.newkeys, (size_t)h.newcap, false));
   DM_TRY(dalloc(&h.newdslot, (size_t)h.newcap, false));
   DM_TRY(dalloc(&h.newnext, (size_t)h.newcap, false));
-  DM_TRY(dalloc(&h.newrank, (size_t)h.newcap, false));
-  DM_TRY(dalloc(&h.newlen, (size_t)h.newcap, false));
+  DM_TRY(dalloc(&h.newslot, (size_t)h.newcap, false));
+  DM_TRY(dalloc(&h.newwin, (size_t)h.newcap, false));
   DM_TRY(dalloc(&h.bucket_head, (size_t)p.num_buckets, false));
   DM_HIP(hipMemsetAsync(h.bucket_head, 0xff, (size_t)p.num_buckets * 4, stream));
   DM_TRY(dalloc(&h.ctr, (size_t)C_COUNT));
@@ -686,6 +686,7 @@ int dm_volume_restore(dm_volume *vol, const void *buf, uint64_t size) {
     DM_HIP(hipMemcpyAsync(x.first, p, x.second, hipMemcpyHostToDevice, S.stream));
     p += x.second;
   }
+  for (int k : {C_N_NEW, C_N_INS, C_CURSOR, C_TICKET}) H.ctr[k] = 0;  // as between frames
   DM_HIP(hipMemcpyAsync(S.h.ctr, H.ctr, sizeof H.ctr, hipMemcpyHostToDevice, S.stream));
   // blocks beyond the snapshot's are unused again
   const size_t rest = (size_t)(S.props.num_blocks - H.num_alloc);

@@ -48,7 +48,7 @@ enum Ctr : int {
   C_NNEW = 12,       // keys inserted by the last allocation
   C_ICP_STOP = 13,   // level + 1 of the ICP level that ended early this frame, 0 = none
   C_NUM_FREE = 14,   // freed pool indices waiting in free_list (a stack; reused first)
-  C_ICP_TICKET = 15, // workgroups of the running linearisation that have stored their record (0 between launches)
+  C_TICKET = 15,     // workgroups of the running linearisation or allocation that are done (0 between launches)
   C_COUNT = 16
 };
 
@@ -92,8 +92,8 @@ struct DmView {
   uint64_t *newkeys;    // newcap
   int32_t *newdslot;    // newcap
   int32_t *newnext;     // newcap
-  int32_t *newrank;     // newcap (rank, or -1 when dropped)
-  int32_t *newlen;      // newcap (bucket list length, written by rank 0)
+  int32_t *newslot;     // newcap (slot in the bucket, or -1 when dropped)
+  int32_t *newwin;      // newcap (winners of the bucket at its first winner, else 0)
   int32_t *bucket_head; // num_buckets, -1 = empty
   int32_t *ctr;         // C_COUNT
   // current frame input (device)
@@ -141,6 +141,7 @@ void launch_alloc(const Launch &L);
 // traversal kernel only (profiling); count_unique also marks the pool index
 // of every block found in v.visited
 void launch_alloc_rays(const Launch &L, bool count_unique = false);
+void launch_alloc_lists(const Launch &L);  // the rest of launch_alloc: takes in the keys that the rays noted
 void launch_integrate(const Launch &L);
 void launch_raycast(const Launch &L);
 // HashTable::DeleteBlock over a list of n block coordinates (one session,

@@ -654,6 +654,7 @@ int dm_server_profile(dm_server *srv, int32_t frame, int32_t reps, double *stage
         total_ms += ms;
       }
     }
+    if (st == 6) launch_alloc_lists(L);
     stage_ms[st] = total_ms / reps;
     if (work && (st == 4 || st == 6)) {
       int64_t sum_vis = 0, sum_visit = 0, sum_alloc = 0;
@@ -676,6 +677,7 @@ int dm_server_profile(dm_server *srv, int32_t frame, int32_t reps, double *stage
       DM_HIP(hipMemsetAsync(S.h.visited, 0, ((size_t)S.h.num_blocks + 31) / 32 * 4, srv->stream));
     }
     launch_alloc_rays(L, true);
+    launch_alloc_lists(L);
     DM_HIP(hipStreamSynchronize(srv->stream));
     int64_t uniq = 0;
     for (int t : act) {

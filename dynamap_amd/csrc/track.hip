@@ -451,14 +451,14 @@ __device__ __forceinline__ void icp_record(const DmView &v, float val, int level
       if (__hip_atomic_fetch_add(gt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
           min(kIcpGroup, nwg - g * kIcpGroup) - 1) {
         __hip_atomic_store(gt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        l = __hip_atomic_fetch_add(&v.ctr[C_ICP_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
+        l = __hip_atomic_fetch_add(&v.ctr[C_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
       }
       last = l;
     }
   }
   __syncthreads();
   if (!last) return;
-  if (threadIdx.x == 0) v.ctr[C_ICP_TICKET] = 0;
+  if (threadIdx.x == 0) v.ctr[C_TICKET] = 0;
   icp_finish(v, level, it, nwg, S);
 }
 

@@ -38,11 +38,48 @@ __device__ __forceinline__ bool win_bit(int x, int y, int z, uint32_t &idx) {
 }
 __device__ __forceinline__ bool test_bit(const uint32_t *map, uint32_t idx) { return (ldg(map + (idx >> 5)) >> (idx & 31)) & 1u; }
 
+__device__ __forceinline__ int key_bucket(const DmView &v, uint64_t key) {
+  int x, y, z;
+  unpack_key(key, x, y, z);
+  return hash_bucket(x, y, z, v.num_buckets);
+}
+
+// A workgroup's traversal state in LDS: the set of the blocks its rays have
+// already handled (looked up, and noted when missing), since neighbouring
+// rays visit mostly the same blocks, so that each is looked up in the global
+// table about once per workgroup; and the key-set slots of the new keys it was
+// first to note.
+constexpr int kSeenSlots = 1024;
+constexpr int kSeenProbes = 8;
+constexpr int kNewSlots = 1024;
+struct RayWG {
+  unsigned long long seen[kSeenSlots];
+  int32_t slots[kNewSlots];
+  int nnew, base, visits;
+};
+
+// Entry idx of the frame's key list: the key in slot h of the key set, chained
+// into its bucket's list (order irrelevant).
+__device__ __forceinline__ void list_new_key(const DmView &v, int idx, uint64_t key, int32_t h) {
+  if (idx < v.newcap) {
+    v.newkeys[idx] = key;
+    v.newdslot[idx] = h;
+    v.newnext[idx] = atomicExch(&v.bucket_head[key_bucket(v, key)], idx);
+  } else {
+    // no room in the frame's key list: release the slot so that a later frame
+    // can insert the key
+    atomicExch((unsigned long long *)&v.dset[h], 0ull);
+    atomicAdd(&v.ctr[C_DSET_OVF], 1);
+  }
+}
+
 // Record a block that is missing from the table in the per-frame key set.
 // A plain read first: once a key is in the set, later visitors return
 // without an atomic (a missing free-space block near the camera is visited
-// by thousands of rays).
-__device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key) {
+// by thousands of rays).  The list entry is left to the workgroup's end, where
+// one addition to the list's length serves all its keys: the length is one
+// address, and one addition per key took 1.3 ms of a first frame at 4 mm.
+__device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key, RayWG &wg) {
   uint32_t h = (uint32_t)mix64(key) & (uint32_t)v.dset_mask;
   for (int probe = 0; probe <= v.dset_mask; ++probe) {
     uint64_t cur = __atomic_load_n((unsigned long long *)&v.dset[h], __ATOMIC_RELAXED);
@@ -50,16 +87,9 @@ __device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key) {
     if (cur == 0ull) {
       const uint64_t prev = atomicCAS((unsigned long long *)&v.dset[h], 0ull, (unsigned long long)key);
       if (prev == 0ull) {
-        int idx = atomicAdd(&v.ctr[C_N_NEW], 1);
-        if (idx < v.newcap) {
-          v.newkeys[idx] = key;
-          v.newdslot[idx] = (int32_t)h;
-        } else {
-          // no room in the frame's key list: release the slot so that a
-          // later frame can insert the key
-          atomicExch((unsigned long long *)&v.dset[h], 0ull);
-          atomicAdd(&v.ctr[C_DSET_OVF], 1);
-        }
+        const int k = atomicAdd(&wg.nnew, 1);
+        if (k < kNewSlots) wg.slots[k] = (int32_t)h;
+        else list_new_key(v, atomicAdd(&v.ctr[C_N_NEW], 1), key, (int32_t)h);
         return;
       }
       if (prev == key) return;
@@ -69,12 +99,6 @@ __device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key) {
   atomicAdd(&v.ctr[C_DSET_OVF], 1);
 }
 
-// Per-workgroup set of the blocks its rays have already handled (looked up,
-// and noted when missing): neighbouring rays visit mostly the same blocks,
-// so each block is looked up in the global table about once per workgroup.
-constexpr int kSeenSlots = 1024;
-constexpr int kSeenProbes = 8;
-
 // kCount (profiling only): also mark the pool index of every block found in
 // the table in v.visited, so that the distinct blocks of a traversal can be
 // counted.
@@ -83,7 +107,8 @@ constexpr int kSeenProbes = 8;
 // reach the workgroup set and the per-frame key set; outside the window the
 // hash table is probed.
 template <bool kCount>
-__device__ __forceinline__ void visit_block(const DmView &v, int x, int y, int z, unsigned long long *seen) {
+__device__ __forceinline__ void visit_block(const DmView &v, int x, int y, int z, RayWG &wg) {
+  unsigned long long *seen = wg.seen;
   if (!in_key_range(x, y, z)) { atomicAdd(&v.ctr[C_DROP_RANGE], 1); return; }
   uint32_t widx;
   const bool in_win = !kCount && win_bit(x, y, z, widx);
@@ -107,7 +132,7 @@ __device__ __forceinline__ void visit_block(const DmView &v, int x, int y, int z
       return;
     }
   }
-  note_new_key(v, key);
+  note_new_key(v, key, wg);
 }
 
 // AllocateFromDepthKernel (tsdf.cu:357-452), one thread per pixel, 16x16
@@ -116,7 +141,7 @@ __device__ __forceinline__ void visit_block(const DmView &v, int x, int y, int z
 // (b + step) * bs boundary for both directions and the extra "neg_ray" block.
 // D: the traversal is bounded by the L1 distance to the end block.
 template <bool kCount>
-__device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, unsigned long long *seen) {
+__device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, RayWG &wg) {
   if (u >= v.cols || r >= v.rows) return 0;
   const int i = r * v.cols + u;
   const float d = v.depth[i];
@@ -160,11 +185,11 @@ __device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, unsigned
   if (bx != ex && dir.x < 0) { dx--; neg = true; }
   if (by != ey && dir.y < 0) { dy--; neg = true; }
   if (bz != ez && dir.z < 0) { dz--; neg = true; }
-  visit_block<kCount>(v, bx, by, bz, seen);
+  visit_block<kCount>(v, bx, by, bz, wg);
   int nvisit = 1;
   if (neg) {
     bx += dx; by += dy; bz += dz;
-    visit_block<kCount>(v, bx, by, bz, seen);
+    visit_block<kCount>(v, bx, by, bz, wg);
     ++nvisit;
   }
   const long long bound64 = llabs((long long)ex - bx) + llabs((long long)ey - by) + llabs((long long)ez - bz);
@@ -183,17 +208,37 @@ __device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, unsigned
       win_bit(bx + bound, by + bound, bz + bound, widx)) {
     win_bit(bx, by, bz, widx);
     const uint32_t ix = (uint32_t)stx, iy = (uint32_t)(sty * kWin), iz = (uint32_t)(stz * kWin * kWin);
-    for (int it = 0; it < bound; ++it) {
-      const bool sx = mtx < mty && mtx < mtz;
-      const bool sy = !(mtx < mty) && mty < mtz;
-      const bool sz = !sx && !sy;
-      mtx += sx ? dtx : 0.0f;
-      mty += sy ? dty : 0.0f;
-      mtz += sz ? dtz : 0.0f;
-      widx += sx ? ix : sy ? iy : iz;
-      if (!test_bit(v.allocmap, widx))
-        visit_block<kCount>(v, (int)(widx & (kWin - 1)) - kWin / 2, (int)((widx / kWin) & (kWin - 1)) - kWin / 2,
-                            (int)(widx / (kWin * kWin)) - kWin / 2, seen);
+    // kAhead steps at a time: their map words are loaded together (past the end
+    // the last block's again), so a ray waits for memory once per group
+    // instead of once per step.
+    constexpr int kAhead = 8;
+    for (int it = 0; it < bound; it += kAhead) {
+      uint32_t at[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const bool sx = mtx < mty && mtx < mtz;
+        const bool sy = !(mtx < mty) && mty < mtz;
+        const bool sz = !sx && !sy;
+        mtx += sx ? dtx : 0.0f;
+        mty += sy ? dty : 0.0f;
+        mtz += sz ? dtz : 0.0f;
+        if (it + k < bound) widx += sx ? ix : sy ? iy : iz;
+        at[k] = widx;
+      }
+      uint32_t word[kAhead], missing = 0;
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) word[k] = ldg(v.allocmap + (at[k] >> 5));
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) missing |= (~(word[k] >> (at[k] & 31)) & 1u) << k;
+      while (missing) {
+        const int k = __builtin_ctz(missing);
+        missing &= missing - 1;
+        uint32_t w = at[0];
+#pragma unroll
+        for (int q = 1; q < kAhead; ++q) w = k == q ? at[q] : w;
+        visit_block<kCount>(v, (int)(w & (kWin - 1)) - kWin / 2, (int)((w / kWin) & (kWin - 1)) - kWin / 2,
+                            (int)(w / (kWin * kWin)) - kWin / 2, wg);
+      }
     }
     return nvisit + bound;
   }
@@ -209,7 +254,7 @@ __device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, unsigned
     mty += sy ? dty : 0.0f;
     bz += sz ? stz : 0;
     mtz += sz ? dtz : 0.0f;
-    visit_block<kCount>(v, bx, by, bz, seen);
+    visit_block<kCount>(v, bx, by, bz, wg);
   }
   return nvisit + bound;
 }
@@ -223,128 +268,120 @@ __global__ __launch_bounds__(256) void k_alloc_rays(const DmView *__restrict__ v
   const int tiles_x = (v.cols + 15) >> 4;
   const int tile = blockIdx.x;
   if (tile >= tiles_x * ((v.rows + 15) >> 4)) return;
-  __shared__ int visits;
-  __shared__ unsigned long long seen[kSeenSlots];
-  for (int k = threadIdx.x; k < kSeenSlots; k += 256) seen[k] = 0ull;
-  if (threadIdx.x == 0) visits = 0;
+  __shared__ RayWG wg;
+  for (int k = threadIdx.x; k < kSeenSlots; k += 256) wg.seen[k] = 0ull;
+  if (threadIdx.x == 0) wg.visits = wg.nnew = 0;
   __syncthreads();
   const int u = (tile % tiles_x) * 16 + (threadIdx.x & 15);
   const int r = (tile / tiles_x) * 16 + (threadIdx.x >> 4);
-  const int n = alloc_ray<kCount>(v, u, r, seen);
-  if (n) atomicAdd(&visits, n);
+  const int n = alloc_ray<kCount>(v, u, r, wg);
+  if (n) atomicAdd(&wg.visits, n);
   __syncthreads();
-  if (threadIdx.x == 0 && visits) atomicAdd(&v.ctr[C_NVISIT], visits);
-}
-
-
-__device__ __forceinline__ int key_bucket(const DmView &v, uint64_t key) {
-  int x, y, z;
-  unpack_key(key, x, y, z);
-  return hash_bucket(x, y, z, v.num_buckets);
-}
-
-// Chain the new keys of each bucket into a list (order irrelevant).
-__global__ __launch_bounds__(256) void k_alloc_link(const DmView *__restrict__ views, const int *__restrict__ active) {
-  const int slot_ = active[blockIdx.y];
-  if (slot_ < 0) return;
-  const DmView &v = views[slot_];
-  int n = min(v.ctr[C_N_NEW], v.newcap);
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    int b = key_bucket(v, v.newkeys[i]);
-    v.newnext[i] = atomicExch(&v.bucket_head[b], i);
+  const int nnew = min(wg.nnew, kNewSlots);
+  if (threadIdx.x == 0) {
+    if (wg.visits) atomicAdd(&v.ctr[C_NVISIT], wg.visits);
+    if (nnew) wg.base = atomicAdd(&v.ctr[C_N_NEW], nnew);
   }
+  if (nnew == 0) return;
+  __syncthreads();
+  for (int k = threadIdx.x; k < nnew; k += 256) {
+    const int32_t h = wg.slots[k];
+    list_new_key(v, wg.base + k, __atomic_load_n((unsigned long long *)&v.dset[h], __ATOMIC_RELAXED), h);
+  }
+}
+
+// Adds the number of lanes with `take` to *counter with one addition for the
+// wavefront; returns this lane's place.
+__device__ __forceinline__ int wave_append(int32_t *counter, bool take) {
+  const unsigned long long m = __ballot(take);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (m && lane == __builtin_ctzll(m)) base = atomicAdd(counter, __popcll(m));
+  return m ? __shfl(base, __builtin_ctzll(m), 64) + __popcll(m & ((1ull << lane) - 1ull)) : 0;
 }
 
 // Canonical rank of each new key within its bucket (ascending packed key);
 // the first `free` keys of a bucket win (K: no overflow chain, the rest drop).
+// A winner's slot is its rank after the bucket's entries; the first also
+// takes the number of the bucket's winners.
 __global__ __launch_bounds__(256) void k_alloc_rank(const DmView *__restrict__ views, const int *__restrict__ active) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
-  int n = min(v.ctr[C_N_NEW], v.newcap);
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const uint64_t key = v.newkeys[i];
-    const int b = key_bucket(v, key);
-    int rank = 0, len = 0;
-    for (int j = v.bucket_head[b]; j >= 0; j = v.newnext[j]) {
-      rank += v.newkeys[j] < key;
-      ++len;
+  const int n = min(v.ctr[C_N_NEW], v.newcap);
+  for (int i0 = blockIdx.x * 256; i0 < n; i0 += gridDim.x * 256) {
+    const int i = i0 + threadIdx.x;
+    int slot = -1;
+    if (i < n) {
+      const uint64_t key = v.newkeys[i];
+      const int b = key_bucket(v, key);
+      const int cnt = bucket_count(v, bucket_ptr(v, b));
+      int rank = 0, len = 0;
+      for (int j = v.bucket_head[b]; j >= 0; j = v.newnext[j]) {
+        rank += v.newkeys[j] < key;
+        ++len;
+      }
+      const int freeb = v.bucket_size - cnt;
+      if (rank < freeb) slot = cnt + rank;
+      v.newslot[i] = slot;
+      v.newwin[i] = slot >= 0 && rank == 0 ? min(len, freeb) : 0;
     }
-    const int freeb = v.bucket_size - bucket_count(v, bucket_ptr(v, b));
-    if (rank < freeb) {
-      v.newrank[i] = rank;
-      atomicAdd(&v.ctr[C_N_INS], 1);
-    } else {
-      v.newrank[i] = -1;
-    }
-    v.newlen[i] = len;
+    wave_append(&v.ctr[C_N_INS], slot >= 0);
   }
 }
 
-// Insert the winners.  D: if the pool cannot take every insertion of the
-// frame, nothing is inserted and all new keys count as dropped_pool.
+// Insert the winners, publish the bucket counts and clear the per-frame
+// structures.  D: if the pool cannot take every insertion of the frame, nothing is
+// inserted and all new keys count as dropped_pool.  The last workgroup with
+// keys (the first when there are none) closes the frame's counters: only
+// workgroups that hold keys, and the first, have read them for good.
 __global__ __launch_bounds__(256) void k_alloc_commit(const DmView *__restrict__ views, const int *__restrict__ active) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
-  const int n = min(v.ctr[C_N_NEW], v.newcap);
+  const int n_all = v.ctr[C_N_NEW];
+  const int n = min(n_all, v.newcap);
+  if (blockIdx.x != 0 && (int)blockIdx.x * 256 >= n) return;
   const int nalloc = v.ctr[C_NUM_ALLOC];
   const int nins = v.ctr[C_N_INS];
   const int nfree = v.ctr[C_NUM_FREE];
-  if (nalloc + max(0, nins - nfree) > v.num_blocks) return;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const int rank = v.newrank[i];
-    if (rank < 0) continue;
-    const uint64_t key = v.newkeys[i];
-    int x, y, z;
-    unpack_key(key, x, y, z);
-    const int b = hash_bucket(x, y, z, v.num_buckets);
-    uint8_t *bk = v.buckets + (size_t)b * (size_t)v.bstride;
-    const int slot = *(const int32_t *)(bk + 12 * v.bucket_size) + rank;
-    // freed pool indices first, top of the stack down (Heap::Consume,
-    // heap.cu:14-17), then fresh ones
-    const int q = atomicAdd(&v.ctr[C_CURSOR], 1);
-    const int ptr = q < nfree ? v.free_list[nfree - 1 - q] : nalloc + (q - nfree);
-    ((uint64_t *)bk)[slot] = key;
-    ((int32_t *)(bk + 8 * v.bucket_size))[slot] = ptr;
-    v.block_key[ptr] = make_int4(x, y, z, 1);
-    uint32_t widx;
-    if (win_bit(x, y, z, widx)) atomicOr(&v.allocmap[widx >> 5], 1u << (widx & 31));
-  }
-}
-
-// Publish bucket counts, clear the per-frame structures.
-__global__ __launch_bounds__(256) void k_alloc_finish(const DmView *__restrict__ views, const int *__restrict__ active) {
-  const int slot_ = active[blockIdx.y];
-  if (slot_ < 0) return;
-  const DmView &v = views[slot_];
-  const int n = min(v.ctr[C_N_NEW], v.newcap);
-  const bool pool_ok = v.ctr[C_NUM_ALLOC] + max(0, v.ctr[C_N_INS] - v.ctr[C_NUM_FREE]) <= v.num_blocks;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const uint64_t key = v.newkeys[i];
-    const int b = key_bucket(v, key);
-    v.dset[v.newdslot[i]] = 0ull;
-    v.bucket_head[b] = -1;
-    if (pool_ok && v.newrank[i] == 0) {
-      int32_t *cnt = (int32_t *)(v.buckets + (size_t)b * (size_t)v.bstride + 12 * v.bucket_size);
-      const int freeb = v.bucket_size - *cnt;
-      *cnt += min(v.newlen[i], freeb);
+  const bool pool_ok = nalloc + max(0, nins - nfree) <= v.num_blocks;
+  for (int i0 = blockIdx.x * 256; i0 < n; i0 += gridDim.x * 256) {
+    const int i = i0 + threadIdx.x;
+    const int slot = i < n ? v.newslot[i] : -1;
+    const bool win = pool_ok && slot >= 0;
+    const int q = wave_append(&v.ctr[C_CURSOR], win);
+    if (i < n) {
+      const uint64_t key = v.newkeys[i];
+      int x, y, z;
+      unpack_key(key, x, y, z);
+      const int b = hash_bucket(x, y, z, v.num_buckets);
+      v.dset[v.newdslot[i]] = 0ull;
+      v.bucket_head[b] = -1;
+      if (win) {
+        uint8_t *bk = v.buckets + (size_t)b * (size_t)v.bstride;
+        // freed pool indices first, top of the stack down (Heap::Consume,
+        // heap.cu:14-17), then fresh ones
+        const int ptr = q < nfree ? v.free_list[nfree - 1 - q] : nalloc + (q - nfree);
+        ((uint64_t *)bk)[slot] = key;
+        ((int32_t *)(bk + 8 * v.bucket_size))[slot] = ptr;
+        const int won = v.newwin[i];
+        if (won) *(int32_t *)(bk + 12 * v.bucket_size) = slot + won;  // slot: the count so far
+        v.block_key[ptr] = make_int4(x, y, z, 1);
+        uint32_t widx;
+        if (win_bit(x, y, z, widx)) atomicOr(&v.allocmap[widx >> 5], 1u << (widx & 31));
+      }
     }
   }
-}
-
-// Counter epilogue (one thread per session): runs after k_alloc_finish.
-__global__ void k_alloc_close(const DmView *__restrict__ views, const int *__restrict__ active) {
-  const int slot_ = active[blockIdx.x];
-  if (slot_ < 0) return;
-  const DmView &v = views[slot_];
+  __syncthreads();  // the workgroup has read the counters
   if (threadIdx.x != 0) return;
-  const int n_all = v.ctr[C_N_NEW];
-  const int n = min(n_all, v.newcap);
-  const int nins = v.ctr[C_N_INS];
-  const int nfree = v.ctr[C_NUM_FREE];
-  if (v.ctr[C_NUM_ALLOC] + max(0, nins - nfree) <= v.num_blocks) {
-    v.ctr[C_NUM_ALLOC] += max(0, nins - nfree);
+  const int nwg = max(1, min((int)gridDim.x, (n + 255) / 256));
+  if (nwg > 1) {
+    if (atomicAdd(&v.ctr[C_TICKET], 1) != nwg - 1) return;
+    v.ctr[C_TICKET] = 0;
+  }
+  if (pool_ok) {
+    v.ctr[C_NUM_ALLOC] = nalloc + max(0, nins - nfree);
     v.ctr[C_NUM_FREE] = max(0, nfree - nins);
     v.ctr[C_DROP_BUCKET] += n - nins;
     v.ctr[C_NNEW] = nins;
@@ -1555,15 +1592,17 @@ __global__ __launch_bounds__(256, 6) void k_raycast(const DmView *__restrict__ v
 static constexpr unsigned kListWG = 64;    // workgroups per session for the new-key passes
 static constexpr unsigned kDilateWG = 256;  // workgroups per session for the dilation (64 blocks each at a time)
 
+void launch_alloc_lists(const Launch &L) {
+  if (L.nact <= 0) return;
+  hipLaunchKernelGGL(k_alloc_rank, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
+  hipLaunchKernelGGL(k_alloc_commit, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
+}
+
 void launch_alloc(const Launch &L) {
   if (L.nact <= 0) return;
   hipLaunchKernelGGL(k_alloc_rays<false>, dim3((unsigned)L.max_tiles, (unsigned)L.nact), dim3(256), 0, L.stream,
                      L.views, L.active);
-  hipLaunchKernelGGL(k_alloc_link, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
-  hipLaunchKernelGGL(k_alloc_rank, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
-  hipLaunchKernelGGL(k_alloc_commit, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
-  hipLaunchKernelGGL(k_alloc_finish, dim3(kListWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
-  hipLaunchKernelGGL(k_alloc_close, dim3((unsigned)L.nact), dim3(64), 0, L.stream, L.views, L.active);
+  launch_alloc_lists(L);
 }
 
 void launch_alloc_rays(const Launch &L, bool count_unique) {

@@ -258,3 +258,60 @@ def test_mesh_cells_near_and_far(room, shift, irregular):
         c = dm.MeshExtractor(cap).ExtractMesh(vol)
         assert c.num_triangles_ == len(m) and len(c) == min(cap, len(m))
         check_same((c.triangles, c.colors, c.edge_ids), tuple(a[:cap] for a in o))
+
+
+# Allocation where a workgroup's lists end: one pixel, ragged tiles, and a 16x16
+# image of rays so far apart that one tile notes more keys than its list (1024)
+# and its set of handled blocks hold; a window face crossed; a table with full buckets
+# next.  The slots' keys and the dropped keys equal the oracle's after each
+# of several frames, the same frame twice among them.
+@pytest.mark.parametrize("rows,cols,fx,props,shift", [
+    (1, 1, 10.0, {}, 0.0), (17, 33, 30.0, {}, 0.0), (16, 16, 5.0, dict(voxel_size=0.008), 0.0),
+    (16, 16, 5.0, dict(voxel_size=0.008), 15.9), (16, 16, 5.0, dict(voxel_size=0.008, num_buckets=1024), 0.0),
+    (9, 11, 9.0, dict(voxel_size=0.02, num_blocks=512), 0.0)])
+def test_allocation_lists(room, rows, cols, fx, props, shift):
+    import oracle_lib as O
+    from test_gpu_volume import table_keys
+    depth, poses = room
+    sens = dict(rows=rows, cols=cols, fx=fx, fy=fx, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    P = shifted(poses, (shift, 0, 0))
+    props = small_tsdf(**{"num_buckets": 1 << 15, "num_blocks": 1 << 15, **props})
+    vol = dm.TsdfVolume(props, rows, cols)
+    ora = O.OracleVolume(props, 32)
+    most = 0
+    for f, oy in ((0, 0), (0, 0), (1, 60), (2, 120)):
+        d = np.ascontiguousarray(depth[f][oy:oy + rows, 40:40 + cols])
+        Tf = P[f].astype(np.float32)
+        before = vol.GetNumAllocatedBlocks()
+        vol.AllocateFromDepth(d, sens, Tf)
+        ora.allocate(d, sens, Tf.astype(np.float64))
+        most = max(most, vol.GetNumAllocatedBlocks() - before)
+        np.testing.assert_array_equal(table_keys(vol.GetHashEntries()), ora.table()[0])
+        c, o = vol.counters(), ora.dropped()
+        assert c["dropped_bucket"] == o["bucket"] and c["dropped_pool"] == o["pool"] and c["dropped_keyset"] == 0
+    if fx == 5.0:
+        assert most > 2048
+    assert (ora.dropped()["pool"] > 0) == (props["num_blocks"] == 512)
+
+
+# More new keys in one frame than the frame's list holds (4096): the list is
+# filled, the rest is counted and taken in by a later frame as far as there is room.
+def test_allocation_list_overflow(room):
+    import oracle_lib as O
+    from test_gpu_volume import table_keys
+    depth, poses = room
+    sens = dict(rows=32, cols=32, fx=9.0, fy=9.0, cx=15.5, cy=15.5)
+    d, Tf = np.ascontiguousarray(depth[0][:32, :32]), poses[0].astype(np.float32)
+    ora = O.OracleVolume(small_tsdf(voxel_size=0.008, num_buckets=1 << 16, num_blocks=1 << 16), 32)
+    ora.allocate(d, sens, Tf.astype(np.float64))
+    assert ora.num_alloc() > 5000
+    vol = dm.TsdfVolume(small_tsdf(voxel_size=0.008, num_buckets=1 << 16, num_blocks=4096), 32, 32)
+    vol.AllocateFromDepth(d, sens, Tf)
+    c = vol.counters()
+    assert c["allocated"] == 4096 and c["dropped_keyset"] >= ora.num_alloc() - 4096 and c["dropped_pool"] == 0
+    vol.AllocateFromDepth(d, sens, Tf)
+    c = vol.counters()
+    assert c["allocated"] == 4096 and c["dropped_pool"] > 0
+    xyz = vol.blocks()[0]
+    full = {tuple(k) for k in ora.blocks()[0]}
+    assert len({tuple(k) for k in xyz}) == 4096 and all(tuple(k) in full for k in xyz)
