@@ -29,14 +29,22 @@ namespace dm {
 constexpr int kBilatMaxR = 7;
 constexpr int kTile = 16;
 
+// Bound by the exponentials: one per tap, of the depth difference; the other,
+// of the offset in the window, is the same for every pixel and comes from a
+// table that the workgroup fills once.  The window is unrolled for its radius.
+template <int r>
 __global__ __launch_bounds__(256) void k_bilateral(const float *__restrict__ in, float *__restrict__ out, int rows,
-                                                  int cols, int r, float inv2sd2, float inv2ss2) {
-  __shared__ float tile[(kTile + 2 * kBilatMaxR) * (kTile + 2 * kBilatMaxR)];
-  const int W = kTile + 2 * r;
+                                                  int cols, float inv2sd2, float inv2ss2) {
+  constexpr int W = kTile + 2 * r, D = 2 * r + 1;
+  __shared__ float tile[W * W], space[D * D];
   const int u0 = blockIdx.x * kTile - r, v0 = blockIdx.y * kTile - r;
   for (int k = threadIdx.x; k < W * W; k += 256) {
     const int uu = u0 + k % W, vv = v0 + k / W;
     tile[k] = (uu >= 0 && vv >= 0 && uu < cols && vv < rows) ? in[(size_t)vv * cols + uu] : 0.f;
+  }
+  if (threadIdx.x < D * D) {
+    const int i = (int)threadIdx.x % D - r, j = (int)threadIdx.x / D - r;
+    space[threadIdx.x] = expf(-(float)(i * i + j * j) * inv2ss2);
   }
   __syncthreads();
   const int tu = threadIdx.x & 15, tv = threadIdx.x >> 4;
@@ -46,40 +54,48 @@ __global__ __launch_bounds__(256) void k_bilateral(const float *__restrict__ in,
   float res = 0.f;
   if (dc > 0.f) {
     float sw = 0.f, sd = 0.f;
-    for (int j = -r; j <= r; ++j)
-      for (int i = -r; i <= r; ++i) {
-        const float d = tile[(tv + r + j) * W + tu + r + i];
-        if (!(d > 0.f)) continue;  // also outside the image (staged as 0)
+    for (int j = 0; j < D; ++j)
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        const float d = tile[(tv + j) * W + tu + i];
         const float dd = d - dc;
-        const float w = expf(-(dd * dd) * inv2sd2) * expf(-(float)(i * i + j * j) * inv2ss2);
-        sw = sw + w;
-        sd = sd + w * d;
+        const float w = expf(-(dd * dd) * inv2sd2) * space[j * D + i];
+        const bool take = d > 0.f;  // also outside the image (staged as 0)
+        sw = take ? sw + w : sw;
+        sd = take ? sd + w * d : sd;
       }
     res = sd / sw;
   }
   out[(size_t)v * cols + u] = res;
 }
 
+// Bound by memory latency: the 25 loads are issued before the first is used
+// (a pixel outside the image loads the centre's again and is not taken).
 __global__ __launch_bounds__(256) void k_pyr_down(const float *__restrict__ in, int rows, int cols,
                                                  float *__restrict__ out, int orows, int ocols, float thr) {
   const int u = blockIdx.x * kTile + (threadIdx.x & 15), v = blockIdx.y * kTile + (threadIdx.x >> 4);
   if (u >= ocols || v >= orows) return;
   const int cu = 2 * u, cv = 2 * v;
-  const float dc = in[(size_t)cv * cols + cu];
+  float d[25];
+#pragma unroll
+  for (int k = 0; k < 25; ++k) {
+    const int x = cu + k % 5 - 2, y = cv + k / 5 - 2;
+    const bool in_image = x >= 0 && y >= 0 && x < cols && y < rows;
+    d[k] = ldg(in + (in_image ? (size_t)y * cols + x : (size_t)cv * cols + cu));
+    if (!in_image) d[k] = 0.f;
+  }
+  const float dc = d[12];
   float res = 0.f;
   if (dc > 0.f) {
     const float b[5] = {1.f, 4.f, 6.f, 4.f, 1.f};
     float sw = 0.f, sd = 0.f;
-    for (int j = -2; j <= 2; ++j)
-      for (int i = -2; i <= 2; ++i) {
-        const int x = cu + i, y = cv + j;
-        if (x < 0 || y < 0 || x >= cols || y >= rows) continue;
-        const float d = in[(size_t)y * cols + x];
-        if (!(d > 0.f) || !(fabsf(d - dc) < thr)) continue;
-        const float w = b[i + 2] * b[j + 2];
-        sw = sw + w;
-        sd = sd + w * d;
-      }
+#pragma unroll
+    for (int k = 0; k < 25; ++k) {
+      const bool take = d[k] > 0.f && fabsf(d[k] - dc) < thr;
+      const float w = b[k % 5] * b[k / 5];
+      sw = take ? sw + w : sw;
+      sd = take ? sd + w * d[k] : sd;
+    }
     res = sd / sw;
   }
   out[(size_t)v * ocols + u] = res;
@@ -88,8 +104,20 @@ __global__ __launch_bounds__(256) void k_pyr_down(const float *__restrict__ in, 
 void launch_bilateral(const float *in, float *out, int rows, int cols, int r, float sigma_d, float sigma_s,
                       hipStream_t st) {
   const dim3 grid((unsigned)((cols + kTile - 1) / kTile), (unsigned)((rows + kTile - 1) / kTile));
-  hipLaunchKernelGGL(k_bilateral, grid, dim3(256), 0, st, in, out, rows, cols, r, 1.0f / (2.0f * sigma_d * sigma_d),
-                     1.0f / (2.0f * sigma_s * sigma_s));
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, in, out, rows, cols, 1.0f / (2.0f * sigma_d * sigma_d),
+                       1.0f / (2.0f * sigma_s * sigma_s));
+  };
+  switch (r) {
+    case 0: run(k_bilateral<0>); break;
+    case 1: run(k_bilateral<1>); break;
+    case 2: run(k_bilateral<2>); break;
+    case 3: run(k_bilateral<3>); break;
+    case 4: run(k_bilateral<4>); break;
+    case 5: run(k_bilateral<5>); break;
+    case 6: run(k_bilateral<6>); break;
+    default: run(k_bilateral<kBilatMaxR>); break;
+  }
 }
 
 }  // namespace dm

@@ -315,3 +315,25 @@ def test_allocation_list_overflow(room):
     xyz = vol.blocks()[0]
     full = {tuple(k) for k in ora.blocks()[0]}
     assert len({tuple(k) for k in xyz}) == 4096 and all(tuple(k) in full for k in xyz)
+
+
+# Every filter radius, and pyramid levels down to nothing, at sizes that leave
+# parts of a tile and of the window outside the image; pixels without depth and
+# depth edges included.  The exponentials of the GPU and host libraries may
+# differ in the last bit, so 2e-6 of the largest depth.
+@pytest.mark.parametrize("radius", range(8))
+@pytest.mark.parametrize("rows,cols", [(1, 1), (17, 33), (50, 39)])
+def test_depth_filters_ragged(room, radius, rows, cols):
+    import oracle_lib as O
+    d = room[0][0][40:40 + rows, 100:100 + cols].copy()
+    d.flat[::7] = 0.0
+    d.flat[3::11] *= np.float32(1.05)
+    g, o = dm.bilateral_filter(d, radius, 0.03, 2.5), O.bilateral(d, radius, 0.03, 2.5, bits=32)
+    np.testing.assert_array_equal(g == 0, o == 0)
+    assert np.abs(g - o).max() <= 2e-6 * np.abs(o).max()
+    levels = dm.depth_pyramid(d, 0.01 * (radius + 1), 4)
+    for l in range(1, 4):
+        assert levels[l].shape == (rows >> l, cols >> l)
+        if levels[l].size:
+            o = O.pyr_down(levels[l - 1], 0.01 * (radius + 1), bits=32)
+            assert np.abs(levels[l] - o).max() <= 2e-6 * np.abs(o).max()
