@@ -91,11 +91,6 @@ __global__ __launch_bounds__(256) void k_source_maps(const DmView *__restrict__ 
   v.snorm[l][t] = n;
 }
 
-__device__ __forceinline__ bool bad3(float4 n) {
-  return !(fabsf(n.x) <= 3.4e38f) || !(fabsf(n.y) <= 3.4e38f) || !(fabsf(n.z) <= 3.4e38f) ||
-         (n.x == 0.f && n.y == 0.f && n.z == 0.f);
-}
-
 constexpr int kVals = 30;
 
 // Association and gates of one pixel (buildNLSKernel, gnSolver.cu:55-195).
@@ -105,67 +100,121 @@ constexpr int kVals = 30;
 // transform, projection and gates are in FP64 (the pixel choice and the
 // inclusion decisions follow the FP64 geometry); residual and Jacobian are
 // FP32.
-struct IcpAssoc {
-  f3 p, pq, n;    // transformed source point, p - q, model normal
-  float qw, vw;   // model and source intensities
-  int pu, pv, j;  // associated model pixel
+//
+// The pixels of a thread go through the three rounds of loads (source point and
+// normal; model point and normal; the model intensity's neighbours) side by
+// side, every load unconditional at a safe index: taken one pixel after the
+// other, each load behind the test of the one before, an iteration of a coarse
+// level was 12 rounds of memory latency (17 us at 80x60 pixels, now 14;
+// 24 -> 21 at 640x480; 16 sessions at level 0 74 -> 58).  The rest of an
+// iteration is a chain too: 7000 of 34000 cycles the four pixels' arithmetic on
+// few wavefronts, 3000 the tickets, 3500 the records, 9000 the step.  One pixel
+// per thread in workgroups of 1024 took as long (the same wavefronts' work
+// on the same compute unit).
+constexpr int kIcpPer = kIcpPix / 256;  // pixels per thread
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+struct IcpPixel {
+  double px, py, pz;    // transformed source point
+  f32x4 Q, NT;          // model point (w: intensity) and normal
+  f3 N;                 // source normal
+  float vw;             // source intensity
+  float xp, xm, yp, ym; // model intensity beside the associated pixel
+  bool ok, inner;       // associated; with the four neighbours inside the image
 };
-__device__ __forceinline__ bool icp_assoc(const DmView &v, int level, const Intr &s, int i, IcpAssoc &a) {
-  const float4 V = v.svert[level][i];
-  const float4 N = v.snorm[level][i];
-  const float4 *tv = v.tvert[level];
-  const float4 *tn = v.tnorm[level];
-  bool ok = V.z >= v.icp_dmin && V.z <= v.icp_dmax && !bad3(N);
-  const double *Td = v.posed + PD_TINC;
-  double px = 0.0, py = 0.0, pz = 0.0;
-  int pu = -1, pv = -1, j = 0;
-  float4 Q = make_float4(0.f, 0.f, 0.f, 0.f), NT = Q;
-  if (ok) {
-    const double X = V.x, Y = V.y, Z = V.z;
-    px = Td[0] * X + Td[1] * Y + Td[2] * Z + Td[3];
-    py = Td[4] * X + Td[5] * Y + Td[6] * Z + Td[7];
-    pz = Td[8] * X + Td[9] * Y + Td[10] * Z + Td[11];
-    pu = to_i32d(round(((double)s.fx * px) / pz + (double)s.cx));
-    pv = to_i32d(round(((double)s.fy * py) / pz + (double)s.cy));
-    ok = !(pu < 0 || pv < 0 || pu >= s.cols || pv >= s.rows);
+__device__ __forceinline__ double uniform_f64(double x) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+struct IcpPose { double m[12]; };
+__device__ __forceinline__ IcpPose icp_pose(const DmView &v) {
+  double m[12];
+#pragma unroll
+  for (int k = 0; k < 12; ++k) m[k] = ldg(v.posed + PD_TINC + k);
+  IcpPose T;
+#pragma unroll
+  for (int k = 0; k < 12; ++k) T.m[k] = uniform_f64(m[k]);
+  return T;
+}
+__device__ __forceinline__ bool bad3(f32x4 n) {
+  return !(fabsf(n.x) <= 3.4e38f) || !(fabsf(n.y) <= 3.4e38f) || !(fabsf(n.z) <= 3.4e38f) ||
+         (n.x == 0.f && n.y == 0.f && n.z == 0.f);
+}
+__device__ __forceinline__ void icp_pixels(const DmView &v, int level, const Intr &s, int P, IcpPose &T,
+                                           IcpPixel (&a)[kIcpPer]) {
+  const f32x4 *sv = reinterpret_cast<const f32x4 *>(v.svert[level]), *sn = reinterpret_cast<const f32x4 *>(v.snorm[level]);
+  const f32x4 *tv = reinterpret_cast<const f32x4 *>(v.tvert[level]), *tn = reinterpret_cast<const f32x4 *>(v.tnorm[level]);
+  f32x4 V[kIcpPer], N[kIcpPer];
+#pragma unroll
+  for (int q = 0; q < kIcpPer; ++q) {
+    const int i = min((int)blockIdx.x * kIcpPix + q * 256 + (int)threadIdx.x, P - 1);
+    V[q] = ldg(sv + i);
+    N[q] = ldg(sn + i);
   }
-  if (ok) {
-    j = pv * s.cols + pu;
-    Q = tv[j];
-    NT = tn[j];
-    ok = Q.z >= v.icp_dmin && Q.z <= v.icp_dmax && !bad3(NT);
+  T = icp_pose(v);
+  const double *Td = T.m;
+  int j[kIcpPer];
+#pragma unroll
+  for (int q = 0; q < kIcpPer; ++q) {
+    IcpPixel &x = a[q];
+    x.ok = (int)blockIdx.x * kIcpPix + q * 256 + (int)threadIdx.x < P && V[q].z >= v.icp_dmin &&
+           V[q].z <= v.icp_dmax && !bad3(N[q]);
+    const double X = V[q].x, Y = V[q].y, Z = V[q].z;
+    x.px = Td[0] * X + Td[1] * Y + Td[2] * Z + Td[3];
+    x.py = Td[4] * X + Td[5] * Y + Td[6] * Z + Td[7];
+    x.pz = Td[8] * X + Td[9] * Y + Td[10] * Z + Td[11];
+    const int pu = to_i32d(round(((double)s.fx * x.px) / x.pz + (double)s.cx));
+    const int pv = to_i32d(round(((double)s.fy * x.py) / x.pz + (double)s.cy));
+    x.ok = x.ok && !(pu < 0 || pv < 0 || pu >= s.cols || pv >= s.rows);
+    x.inner = x.ok && pu >= 1 && pv >= 1 && pu < s.cols - 1 && pv < s.rows - 1;
+    x.N = mk(N[q].x, N[q].y, N[q].z);
+    x.vw = V[q].w;
+    j[q] = x.ok ? pv * s.cols + pu : 0;
   }
-  if (ok) {
-    const double X = N.x, Y = N.y, Z = N.z;
-    const double nrx = Td[0] * X + Td[1] * Y + Td[2] * Z;
-    const double nry = Td[4] * X + Td[5] * Y + Td[6] * Z;
-    const double nrz = Td[8] * X + Td[9] * Y + Td[10] * Z;
-    const double ct = (double)NT.x * nrx + (double)NT.y * nry + (double)NT.z * nrz;
-    const double dqx = px - (double)Q.x, dqy = py - (double)Q.y, dqz = pz - (double)Q.z;
-    ok = fabs(ct) > 0.95105651629515357 && sqrt(dqx * dqx + dqy * dqy + dqz * dqz) <= (double)v.dist_max;
-    a.p = mk((float)px, (float)py, (float)pz);
-    a.pq = mk((float)dqx, (float)dqy, (float)dqz);
+#pragma unroll
+  for (int q = 0; q < kIcpPer; ++q) {
+    a[q].Q = ldg(tv + j[q]);
+    a[q].NT = ldg(tn + j[q]);
   }
-  a.n = mk(NT.x, NT.y, NT.z);
-  a.qw = Q.w;
-  a.vw = V.w;
-  a.pu = pu;
-  a.pv = pv;
-  a.j = j;
-  return ok;
+  if (v.w_photo > 0.f) {
+#pragma unroll
+    for (int q = 0; q < kIcpPer; ++q) {
+      const int dx = a[q].inner ? 1 : 0, dy = a[q].inner ? s.cols : 0;
+      a[q].xp = ldg((const float *)(tv + j[q] + dx) + 3);
+      a[q].xm = ldg((const float *)(tv + j[q] - dx) + 3);
+      a[q].yp = ldg((const float *)(tv + j[q] + dy) + 3);
+      a[q].ym = ldg((const float *)(tv + j[q] - dy) + 3);
+    }
+  }
+}
+// The gates; p: the transformed source point, pq: p - q.
+__device__ __forceinline__ bool icp_gate(const DmView &v, const IcpPose &T, const IcpPixel &x, f3 &p, f3 &pq) {
+  const double *Td = T.m;
+  const double X = x.N.x, Y = x.N.y, Z = x.N.z;
+  const double nrx = Td[0] * X + Td[1] * Y + Td[2] * Z;
+  const double nry = Td[4] * X + Td[5] * Y + Td[6] * Z;
+  const double nrz = Td[8] * X + Td[9] * Y + Td[10] * Z;
+  const double ct = (double)x.NT.x * nrx + (double)x.NT.y * nry + (double)x.NT.z * nrz;
+  const double dqx = x.px - (double)x.Q.x, dqy = x.py - (double)x.Q.y, dqz = x.pz - (double)x.Q.z;
+  p = mk((float)x.px, (float)x.py, (float)x.pz);
+  pq = mk((float)dqx, (float)dqy, (float)dqz);
+  // sqrt(d2) <= dist_max, from the squares unless they are equal to 1e-12
+  const double d2 = dqx * dqx + dqy * dqy + dqz * dqz, dm = (double)v.dist_max, m2 = dm * dm;
+  bool near = dm >= 0.0 && d2 < m2;
+  if (!(fabs(d2 - m2) > 1e-12 * m2)) near = sqrt(d2) <= dm;
+  return x.ok && x.Q.z >= v.icp_dmin && x.Q.z <= v.icp_dmax && !bad3(x.NT) && fabs(ct) > 0.95105651629515357 && near;
 }
 
-// Per-pixel terms of one Gauss-Newton linearisation at pyramid level `level`
+// Per-pixel terms of one Gauss-Newton linearisation
 // accumulated into vals (upper JtJ 21, Jtr 6, geometric count, r^2,
 // photometric count); the photometric term adds w_photo Jp Jp^T and
 // w_photo Jp rp.
-__device__ __forceinline__ void icp_pixel(const DmView &v, int level, const Intr &s, int i, float *vals) {
-  IcpAssoc as;
-  if (!icp_assoc(v, level, s, i, as)) return;
-  const float4 *tv = v.tvert[level];
-  const f3 p = as.p, n = as.n;
+__device__ __forceinline__ void icp_terms(const DmView &v, const Intr &s, const IcpPose &T, const IcpPixel &x,
+                                          float *vals) {
+  f3 p, pq;
+  if (!icp_gate(v, T, x, p, pq)) return;
+  const f3 n = mk(x.NT.x, x.NT.y, x.NT.z);
   float pvl[kVals];
-  const float r = dot(as.pq, n);
+  const float r = dot(pq, n);
   const f3 c = cross(p, n);
   const float J[6] = {c.x, c.y, c.z, n.x, n.y, n.z};
   int k = 0;
@@ -178,11 +227,10 @@ __device__ __forceinline__ void icp_pixel(const DmView &v, int level, const Intr
   pvl[27] = 1.f;
   pvl[28] = r * r;
   pvl[29] = 0.f;
-  if (v.w_photo > 0.f && as.pu >= 1 && as.pv >= 1 && as.pu < s.cols - 1 && as.pv < s.rows - 1) {
-    const int j = as.j;
-    const float gx = (tv[j + 1].w - tv[j - 1].w) * 0.5f;
-    const float gy = (tv[j + s.cols].w - tv[j - s.cols].w) * 0.5f;
-    const float rp = as.qw - as.vw;
+  if (v.w_photo > 0.f && x.inner) {
+    const float gx = (x.xp - x.xm) * 0.5f;
+    const float gy = (x.yp - x.ym) * 0.5f;
+    const float rp = x.Q.w - x.vw;
     const float iz = 1.0f / p.z;
     const f3 G = mk(gx * s.fx * iz, gy * s.fy * iz, -(gx * s.fx * p.x + gy * s.fy * p.y) * iz * iz);
     const f3 cg = cross(p, G);
@@ -205,22 +253,20 @@ __device__ __forceinline__ void icp_pixel(const DmView &v, int level, const Intr
 // [J, r, 1] in columns 0-7 and photometric sqrt(w_photo) [Jp, rp] with a 1 in
 // columns 8-15 (zeros where a term does not apply).  F^T F summed over the
 // pixels holds J^T J and J^T r of both terms, r^2 and both counts.
-__device__ __forceinline__ void icp_features(const DmView &v, int level, const Intr &s, int i, float swp,
-                                             float *f) {
+__device__ __forceinline__ void icp_features(const DmView &v, const Intr &s, const IcpPose &T, const IcpPixel &x,
+                                             float swp, float *f) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) f[k] = 0.f;
-  IcpAssoc as;
-  if (!icp_assoc(v, level, s, i, as)) return;
-  const float4 *tv = v.tvert[level];
-  const f3 p = as.p, n = as.n;
-  const float r = dot(as.pq, n);
+  f3 p, pq;
+  if (!icp_gate(v, T, x, p, pq)) return;
+  const f3 n = mk(x.NT.x, x.NT.y, x.NT.z);
+  const float r = dot(pq, n);
   const f3 c = cross(p, n);
   f[0] = c.x; f[1] = c.y; f[2] = c.z; f[3] = n.x; f[4] = n.y; f[5] = n.z; f[6] = r; f[7] = 1.f;
-  if (v.w_photo > 0.f && as.pu >= 1 && as.pv >= 1 && as.pu < s.cols - 1 && as.pv < s.rows - 1) {
-    const int j = as.j;
-    const float gx = (tv[j + 1].w - tv[j - 1].w) * 0.5f;
-    const float gy = (tv[j + s.cols].w - tv[j - s.cols].w) * 0.5f;
-    const float rp = as.qw - as.vw;
+  if (v.w_photo > 0.f && x.inner) {
+    const float gx = (x.xp - x.xm) * 0.5f;
+    const float gy = (x.yp - x.ym) * 0.5f;
+    const float rp = x.Q.w - x.vw;
     const float iz = 1.0f / p.z;
     const f3 G = mk(gx * s.fx * iz, gy * s.fy * iz, -(gx * s.fx * p.x + gy * s.fy * p.y) * iz * iz);
     const f3 cg = cross(p, G);
@@ -276,6 +322,10 @@ __device__ __forceinline__ float record_value(const float *p) {
 __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepLds &S) {
   const int k = threadIdx.x & 31, j = threadIdx.x >> 5;
   if (threadIdx.x < PD_COUNT) S.pd[threadIdx.x] = v.posed[threadIdx.x];
+  // the session's parameters, on their way with the records
+  const float lambda = v.lambda, min_inc = v.min_inc, max_inc = v.max_inc;
+  bool last = it == v.iters[level], none = true;  // none: no finer level takes iterations
+  for (int l = 0; l < level; ++l) none = none && v.iters[l] == 0;
   auto value = [&](int t) { return record_value(v.partials + (size_t)min(t, nwg - 1) * kIcpVals + k); };
 #pragma unroll 1
   for (int h = 0; h < 2; ++h) {  // leaves 128 h .. 128 h + 127
@@ -320,7 +370,7 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
   double xi[6] = {0, 0, 0, 0, 0, 0};
   if (mx > 0.0) {
     const double sc = 1.0 / mx;
-    const double alpha = (double)v.lambda * (mx * sc) / (double)it;
+    const double alpha = (double)lambda * (mx * sc) / (double)it;
     const int row = lane < 6 ? lane : 5;
     double A[6], L[6], D[6];
 #pragma unroll
@@ -381,7 +431,7 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
     acc[q] = S.pd[PD_ACC + q] + xi[q];
     prev[q] = S.pd[PD_PREVACC + q];
   }
-  const bool stop = level_converged(acc, prev, (double)v.min_inc);
+  const bool stop = level_converged(acc, prev, (double)min_inc);
 #pragma unroll
   for (int q = 0; q < 6; ++q)
     if (lane == q) {
@@ -389,11 +439,10 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
       v.posed[PD_PREVACC + q] = prev[q];
     }
   if (stop && lane == 0) v.ctr[C_ICP_STOP] = level + 1;
-  bool last = it == v.iters[level] || stop;
-  for (int l = 0; l < level; ++l) last = last && v.iters[l] == 0;
+  last = (last || stop) && none;
   if (last) {
     const double ssum = acc[0] + acc[1] + acc[2] + acc[3] + acc[4] + acc[5];
-    if (ssum != ssum || isinf(ssum) || ssum >= (double)v.max_inc) {
+    if (ssum != ssum || isinf(ssum) || ssum >= (double)max_inc) {
       tinc = r4 == c4 ? 1.0 : 0.0;
       if (lane == 0) atomicAdd(&v.ctr[C_ICP_FAIL], 1);
     }
@@ -432,8 +481,8 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
 // each group's last one counts for the session.
 // The step in the reduction's launch saves a launch per iteration, most of
 // them no-ops because the level has converged: at 640x480 reduction and step
-// took 18 + 13 us at level 0 and 1.1 + 1.1 us when converged, now 26 and 1.1;
-// a 320x240 frame's 19 iterations 148 -> 136 us of kernels and 19 launches less.
+// took 18 + 13 us at level 0 and 1.1 + 1.1 us when converged, in one launch 26 and
+// 1.1; a 320x240 frame's 19 iterations 148 -> 136 us of kernels and 19 launches less.
 constexpr int kIcpGroup = 16;
 __device__ __forceinline__ void icp_record(const DmView &v, float val, int level, int it, int nwg, int solve,
                                            IcpStepLds &S) {
@@ -451,7 +500,8 @@ __device__ __forceinline__ void icp_record(const DmView &v, float val, int level
       if (__hip_atomic_fetch_add(gt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
           min(kIcpGroup, nwg - g * kIcpGroup) - 1) {
         __hip_atomic_store(gt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        l = __hip_atomic_fetch_add(&v.ctr[C_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
+        l = ng == 1 ||
+            __hip_atomic_fetch_add(&v.ctr[C_TICKET], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ng - 1;
       }
       last = l;
     }
@@ -478,11 +528,11 @@ __global__ __launch_bounds__(256) void k_icp_reduce(const DmView *__restrict__ v
   float vals[kVals];
 #pragma unroll
   for (int k = 0; k < kVals; ++k) vals[k] = 0.f;
+  IcpPose T;
+  IcpPixel px[kIcpPer];
+  icp_pixels(v, level, s, P, T, px);
 #pragma unroll
-  for (int q = 0; q < kIcpPix / 256; ++q) {
-    const int i = blockIdx.x * kIcpPix + q * 256 + threadIdx.x;
-    if (i < P) icp_pixel(v, level, s, i, vals);
-  }
+  for (int q = 0; q < kIcpPer; ++q) icp_terms(v, s, T, px[q], vals);
   // wavefront tree (wave_sum) then LDS across the four waves
 #pragma unroll
   for (int k = 0; k < kVals; ++k) vals[k] = wave_sum(vals[k]);
@@ -530,16 +580,13 @@ __global__ __launch_bounds__(256) void k_icp_reduce_mfma(const DmView *__restric
   float *F = feat[wave];
   const float swp = v.w_photo > 0.f ? sqrtf(v.w_photo) : 0.f;
   icp_f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int q = 0; q < kIcpPix / 256; ++q) {
-    const int i = blockIdx.x * kIcpPix + q * 256 + threadIdx.x;
-    float f[16];
-    if (i < P) {
-      icp_features(v, level, s, i, swp, f);
-    } else {
+  IcpPose T;
+  IcpPixel px[kIcpPer];
+  icp_pixels(v, level, s, P, T, px);
 #pragma unroll
-      for (int k = 0; k < 16; ++k) f[k] = 0.f;
-    }
+  for (int q = 0; q < kIcpPer; ++q) {
+    float f[16];
+    icp_features(v, s, T, px[q], swp, f);
 #pragma unroll
     for (int k = 0; k < 16; ++k) F[lane * kFeatPitch + k] = f[k];
     __syncthreads();
