@@ -154,6 +154,7 @@ void launch_delete(const DmView *view, const int4 *req, int n, unsigned long lon
 // live blocks whose centre lies farther than radius from c, appended to req
 // (capacity: the pool size) with *nreq counting them
 void launch_select_far(const DmView *view, const double c[3], double radius, int4 *req, int *nreq, hipStream_t st);
+void launch_session_reset(const DmView &h, const double *init_pose, hipStream_t st);
 void rebuild_far_maps(const Launch &L);  // clear and rebuild bricks/coarse/allocmap (not for graph capture)
 void launch_source_maps(const Launch &L);
 // ICP linearisation at one level (one FP32 record per workgroup); with solve,

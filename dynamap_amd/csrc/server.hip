@@ -35,8 +35,6 @@ struct Trace {
   int next_frame = -1;  // trace frame the live session continues at; -1 when it cannot continue
 };
 
-int sess_reset(Sess &S, const double init_pose[16]);
-
 }  // namespace dm
 
 using namespace dm;
@@ -62,30 +60,6 @@ struct dm_server {
 
 namespace dm {
 
-int sess_reset(Sess &S, const double init_pose[16]) {
-  int n = 0;
-  DM_HIP(hipMemcpyAsync(&n, S.h.ctr + C_NUM_ALLOC, 4, hipMemcpyDeviceToHost, S.stream));
-  DM_HIP(hipStreamSynchronize(S.stream));
-  n = std::min(std::max(n, 0), S.h.num_blocks);
-  DM_HIP(hipMemsetAsync(S.h.buckets, 0, (size_t)S.h.num_buckets * S.h.bstride, S.stream));
-  DM_HIP(hipMemsetAsync(S.h.vox, 0, (size_t)n * kBlockVox * 8, S.stream));
-  DM_HIP(hipMemsetAsync(S.h.blk_near, 0, (size_t)n, S.stream));
-  DM_HIP(hipMemsetAsync(S.h.bricks, 0, kBrickCount * sizeof(ulonglong2), S.stream));
-  DM_HIP(hipMemsetAsync(S.h.allocmap, 0, kWinWords * 4, S.stream));
-  DM_HIP(hipMemsetAsync(S.h.coarse, 0, (size_t)kCoarseWords * 4, S.stream));
-  DM_HIP(hipMemsetAsync(S.h.ctr, 0, C_COUNT * 4, S.stream));
-  double pd[PD_COUNT] = {0};
-  for (int k = 0; k < 16; ++k) {
-    const double I = (k % 5 == 0) ? 1.0 : 0.0;
-    pd[PD_T + k] = I; pd[PD_TPREV + k] = I; pd[PD_TINC + k] = I;
-    pd[PD_TINIT + k] = init_pose ? init_pose[k] : I;
-  }
-  DM_HIP(hipMemcpyAsync(S.h.posed, pd, sizeof pd, hipMemcpyHostToDevice, S.stream));
-  DM_HIP(hipStreamSynchronize(S.stream));
-  S.frames = 0;
-  return DM_OK;
-}
-
 static bool same_shape(const Sess &S, const Trace &t) {
   return memcmp(&S.props, &t.props, sizeof(dm_tsdf_props)) == 0 && S.max_rows == t.sensor.rows &&
          S.max_cols == t.sensor.cols;
@@ -102,8 +76,22 @@ static int apply_trace(Sess &S, const Trace &t) {
   return DM_OK;
 }
 
+// The resets run on the server's stream, behind its last batch; admit waits
+// for all of them at its end.
+static int sess_reset(dm_server *srv, Sess &S, const double init_pose[16]) {
+  launch_session_reset(S.h, init_pose, srv->stream);
+  DM_HIP(hipGetLastError());
+  S.frames = 0;
+  return DM_OK;
+}
+
 // Admit waiting traces in request order while slots and budget allow.
 static int admit(dm_server *srv, const std::vector<int> &want) {
+  bool any = false;
+  const auto done = [&](int r) -> int {
+    if (any) DM_HIP(hipStreamSynchronize(srv->stream));
+    return r;
+  };
   for (int ti : want) {
     Trace &t = srv->traces[ti];
     if (t.sess) continue;
@@ -115,8 +103,8 @@ static int admit(dm_server *srv, const std::vector<int> &want) {
     for (size_t k = 0; k < srv->pool.size(); ++k)
       if (same_shape(*srv->pool[k], t)) { S = srv->pool[k]; srv->pool.erase(srv->pool.begin() + k); break; }
     if (S) {
-      int r = sess_reset(*S, t.init_pose);
-      if (r != DM_OK) return r;
+      const int r = sess_reset(srv, *S, t.init_pose);
+      if (r != DM_OK) { srv->pool.push_back(S); return done(r); }
     } else {
       // free pooled sessions of other shapes if their memory is needed
       while (!srv->pool.empty()) {
@@ -127,16 +115,17 @@ static int admit(dm_server *srv, const std::vector<int> &want) {
       }
       S = new Sess();
       int r = S->init(t.props, t.sensor.rows, t.sensor.cols);
-      if (r == DM_OK) r = sess_reset(*S, t.init_pose);
-      if (r != DM_OK) { S->release(); delete S; return r; }
+      if (r == DM_OK) r = sess_reset(srv, *S, t.init_pose);
+      if (r != DM_OK) { S->release(); delete S; return done(r); }
     }
     apply_trace(*S, t);
     t.sess = S;
     t.slot = slot;
     srv->slot_trace[slot] = ti;
     srv->used_bytes += t.bytes;
+    any = true;
   }
-  return DM_OK;
+  return done(DM_OK);
 }
 
 static void retire(dm_server *srv, int ti) {

@@ -877,6 +877,36 @@ __global__ __launch_bounds__(256) void k_clear_far_maps(const DmView *__restrict
   for (size_t w = (size_t)blockIdx.x * 256 + threadIdx.x; w < (size_t)kCoarseWords; w += stride) v.coarse[w] = 0u;
 }
 
+// A session back at its start: table, voxels in use, empty-space bits,
+// counters and poses.  Bound by the stores (57 MB at 2 cm, most of it the
+// bits and the table).  The pool's fill is read here, so that the host need
+// not wait for it: 7 clears, 2 copies and 2 waits took about 80 us a session,
+// the two kernels 30.
+__device__ __forceinline__ void clear_bytes(void *p, size_t bytes) {
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
+  u64x2 *q = (u64x2 *)p;
+  for (size_t k = t; k < bytes / 16; k += stride) stg(q + k, u64x2{0, 0});
+  for (size_t k = (bytes & ~(size_t)15) + t; k < bytes; k += stride) stg((uint8_t *)p + k, (uint8_t)0);
+}
+__global__ __launch_bounds__(256) void k_session_clear(DmView v) {
+  const size_t n = (size_t)min(max(v.ctr[C_NUM_ALLOC], 0), v.num_blocks);
+  clear_bytes(v.buckets, (size_t)v.num_buckets * v.bstride);
+  clear_bytes(v.vox, n * kBlockVox * 8);
+  clear_bytes(v.blk_near, n);
+  clear_bytes(v.bricks, kBrickCount * sizeof(ulonglong2));
+  clear_bytes(v.allocmap, kWinWords * 4);
+  clear_bytes(v.coarse, (size_t)kCoarseWords * 4);
+}
+struct InitPose { double T[16]; };
+__global__ __launch_bounds__(128) void k_session_open(DmView v, InitPose init) {
+  const int t = threadIdx.x;
+  if (t < C_COUNT) v.ctr[t] = 0;
+  if (t < PD_COUNT) {
+    const double I = (t & 15) % 5 == 0 ? 1.0 : 0.0;
+    v.posed[t] = t >= PD_TINIT && t < PD_TINIT + 16 ? init.T[t - PD_TINIT] : t < PD_ACC ? I : 0.0;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Raycast (GenerateDepthKernel / GenerateRgbKernel, tsdf.cu:470-526).
 // K: samples are GetInterpolatedVoxel at T * getPoint3d(i, z).
@@ -1636,6 +1666,15 @@ void rebuild_far_maps(const Launch &L) {
   hipLaunchKernelGGL(k_clear_far_maps, dim3(1024, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
   hipLaunchKernelGGL(k_dilate_near, dim3(kDilateWG, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
   hipLaunchKernelGGL(k_mark_allocated, dim3(256, (unsigned)L.nact), dim3(256), 0, L.stream, L.views, L.active);
+}
+
+void launch_session_reset(const DmView &h, const double *init_pose, hipStream_t st) {
+  static_assert(PD_T == 0 && PD_TPREV == 16 && PD_TINC == 32 && PD_ACC == 48 && PD_COUNT <= 128 && C_COUNT <= 128,
+                "the matrices come first");
+  InitPose init;
+  for (int k = 0; k < 16; ++k) init.T[k] = init_pose ? init_pose[k] : k % 5 == 0 ? 1.0 : 0.0;
+  hipLaunchKernelGGL(k_session_clear, dim3(2048), dim3(256), 0, st, h);
+  hipLaunchKernelGGL(k_session_open, dim3(1), dim3(128), 0, st, h, init);
 }
 
 void launch_delete(const DmView *view, const int4 *req, int n, unsigned long long *dmask, int *touched, int *counts,

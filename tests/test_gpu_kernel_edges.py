@@ -337,3 +337,23 @@ def test_depth_filters_ragged(room, radius, rows, cols):
         if levels[l].size:
             o = O.pyr_down(levels[l - 1], 0.01 * (radius + 1), bits=32)
             assert np.abs(levels[l] - o).max() <= 2e-6 * np.abs(o).max()
+
+
+# Sessions taken from the server's pool and cleared on the device: runs after
+# the first equal it bit for bit, batched and frame by frame, with pools and
+# tables of sizes that are no multiple of the clear's words, and bucket records
+# of one and several lines.
+@pytest.mark.parametrize("props", [dict(num_blocks=9999), dict(num_blocks=6007, num_buckets=5003, bucket_size=3),
+                                   dict(bucket_size=25)])
+def test_server_sessions_cleared(props):
+    N = dm._native
+    w = configs.WORKLOADS["rigid-320x240-2cm"]
+    srv = dm.Server(4, 240, 320)
+    for k in range(3):
+        d, c, g = configs.make_sequence("rigid-320x240-2cm", 4, session=k)
+        srv.add_trace(small_tsdf(**props), w["icp"], w["sensor"], g[0], d, c)
+    first = srv.run(N.DM_RUN_BATCHED, 0, 4, want_poses=True)["poses"]
+    assert np.abs(first[:, 1:, :3, 3] - first[:, :1, :3, 3]).max() > 1e-3
+    for mode in (N.DM_RUN_BATCHED, N.DM_RUN_PER_FRAME_DEV, N.DM_RUN_BATCHED):
+        np.testing.assert_array_equal(srv.run(mode, 0, 4, want_poses=True)["poses"], first)
+    srv.close()
