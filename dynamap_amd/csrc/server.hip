@@ -543,8 +543,8 @@ int dm_server_run(dm_server *srv, int32_t mode, int32_t first_frame, int32_t nfr
 // Time each stage of the batched pipeline with HIP events on the server's
 // stream, over the admitted sessions at trace frame `frame` (the sessions'
 // state is advanced by the timed launches).  stage_ms[k] = mean duration of
-// one launch of stage k: 0 source maps, 1 ICP reduction (level 0),
-// 2 ICP solve, 3 allocation (all six kernels), 4 integration, 5 raycast,
+// one launch of stage k: 0 source maps, 1 ICP iteration (level 0), 2 its
+// linearisation alone, 3 allocation (all kernels), 4 integration, 5 raycast,
 // 6 ray traversal kernel alone.  work (summed over sessions, per launch):
 // [0] pixels, [1] visible blocks, [2] block visits of the traversal, [3] new
 // blocks of the frame, [4] sessions, [5] allocated blocks, [6] distinct blocks

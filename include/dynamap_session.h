@@ -116,8 +116,8 @@ DM_API int dm_server_run(dm_server *srv, int32_t mode, int32_t first_frame, int3
                          int64_t *batches);
 /* Time each stage of the batched pipeline (HIP events on the server's
  * stream) over the admitted sessions at trace frame `frame`; advances their
- * state.  stage_ms[7]: source maps, ICP reduction (level 0), ICP solve,
- * allocation (all kernels), integration, raycast, ray traversal alone.
+ * state.  stage_ms[7]: source maps, ICP iteration (level 0), its linearisation
+ * alone, allocation (all kernels), integration, raycast, ray traversal alone.
  * work[7]: pixels, visible blocks, traversal block visits, blocks inserted
  * by the frame, sessions, allocated blocks, distinct blocks visited by the
  * traversal. */

@@ -199,10 +199,12 @@ def test_nonrigid_step_node_counts(nodes):
 
 
 # Nearest nodes where a query's lanes change in number (64 below 16384 queries,
-# 8 below 65536, then 1) and where the nodes fill, miss and pass a tile of 1024.
+# 8 below 65536, then 1) and where the nodes fill, miss and pass a tile of 1024
+# and a group of 32.
 # Whole coordinates: squared distances are exact and full of ties, which go to
 # the lower index.
-@pytest.mark.parametrize("nodes,verts", [(5, 16383), (1023, 16384), (1025, 65535), (1024, 65536), (2049, 300)])
+@pytest.mark.parametrize("nodes,verts", [(5, 16383), (1023, 16384), (1025, 65535), (1024, 65536), (2049, 300),
+                                         (5, 65537), (33, 65536), (1087, 68000)])
 def test_nearest_nodes_lanes_and_ties(nodes, verts):
     rng = np.random.default_rng(nodes + verts)
     cell = rng.permutation(41 ** 3)[:max(verts, nodes)]
