@@ -167,12 +167,13 @@ def test_raycast_outputs_in_chunks(room, rows, cols, frame):
 
 # One Gauss-Newton step against the FP64 oracle on random clouds (normals in
 # every direction, so that every motion is observable and the step is unique):
-# 5 nodes, 16 (one workgroup of the PCG), 17 (one node in a second), and 300,
+# 5 nodes, 16 (one workgroup of the PCG), 17 (one node in a second), 32 and 33
+# (the same of the preconditioner), and 300,
 # some of whose rows have more than 16 blocks.  PCG runs to its tolerance.  The GPU
 # stores the blocks in FP32 (6e-8 relative); with the damping and the weights
 # here the systems' condition numbers stay below 1e4, so 1e-3 of the largest
 # motion bounds the difference.
-@pytest.mark.parametrize("nodes", [5, 16, 17, 300])
+@pytest.mark.parametrize("nodes", [5, 16, 17, 32, 33, 300])
 def test_nonrigid_step_node_counts(nodes):
     import oracle_lib as O
     from test_oracle_nonrigid import random_cloud
