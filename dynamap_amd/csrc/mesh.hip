@@ -294,7 +294,8 @@ __device__ __forceinline__ bool outside_box(const BoxArg &box, int gx, int gy, i
 // then their voxels), so a block takes one wavefront with all its loads in
 // flight, and as many blocks as registers and LDS allow are resident.  Cells
 // without a sign change or with an unobserved voxel, nearly all, are dropped
-// on bit masks; the others are packed into full wavefronts.
+// on bit masks; the others are packed into full wavefronts.  Room at 8 mm 353 ->
+// 43 us, at 2 cm 42 -> 10 (against 512 threads per block evaluating every cell).
 __global__ __launch_bounds__(64 * kMcWaves) void k_mc_count(const DmView *__restrict__ vp, const int *__restrict__ list,
                                                            int n, BoxArg box, uint8_t *__restrict__ cubes,
                                                            int *__restrict__ block_tri) {
@@ -355,7 +356,8 @@ __device__ __forceinline__ uint64_t edge_id(int gx, int gy, int gz, int e) {
 
 // A wavefront per block with triangles.  64 of its cells at a time leave their
 // corner samples in LDS; then a lane takes a vertex, so that neighbouring
-// lanes write neighbouring vertices.
+// lanes write neighbouring vertices.  At 8 mm 82 -> 33 us, at 2 cm 36 -> 20
+// (against a lane per cell writing its triangles one by one).
 __global__ __launch_bounds__(64 * kMcWaves) void k_mc_emit(const DmView *__restrict__ vp, const int *__restrict__ list,
                                                           int n, const uint8_t *__restrict__ cubes,
                                                           const int *__restrict__ block_tri,
