@@ -1428,7 +1428,7 @@ __device__ __forceinline__ int beam_steps(const DmView &v, const Intr &s, const 
   const float hx = 0.5f * (float)(ww - 1), hy = 0.5f * (float)(wh - 1);
   const float uc = (float)(u - (lane & (ww - 1))) + hx, rc = (float)(r - lane / ww) + hy;
   const f3 pd = rot(T, mk((uc - s.cx) * ifx, (rc - s.cy) * ify, 1.0f)) * inv_vs;
-  const float ex = hx * ifx * inv_vs, ey = hy * ify * inv_vs;
+  const float ex = hx * fabsf(ifx) * inv_vs, ey = hy * fabsf(ify) * inv_vs;  // a mirrored sensor's is negative
   const float d = fmaxf(fmaxf(fabsf(T.m[0]) * ex + fabsf(T.m[1]) * ey, fabsf(T.m[4]) * ex + fabsf(T.m[5]) * ey),
                         fabsf(T.m[8]) * ex + fabsf(T.m[9]) * ey);
   const float zcap = fminf(zmax, 5.25f / d);

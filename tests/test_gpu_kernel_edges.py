@@ -360,3 +360,31 @@ def test_server_sessions_cleared(props):
     for mode in (N.DM_RUN_BATCHED, N.DM_RUN_PER_FRAME_DEV, N.DM_RUN_BATCHED):
         np.testing.assert_array_equal(srv.run(mode, 0, 4, want_poses=True)["poses"], first)
     srv.close()
+
+
+# The shared first steps' bound with mirrored axes (a focal length below zero,
+# which the server takes): a camera rolled by 45 degrees, so that the two axes'
+# shares of the bound are equal in size, before a wall at 1 m with an opening in
+# front of the middle of every wavefront, behind which there is nothing the
+# tracking may use.  The bundle's middle ray runs free through the opening; the
+# rays beside it must find the wall, or the second frame cannot be tracked.
+@pytest.mark.parametrize("sx,sy", [(1, 1), (1, -1), (-1, 1), (-1, -1)])
+def test_raycast_shared_steps_mirrored_sensor(sx, sy):
+    import oracle_lib as O
+    n, near = 32, (1.0, 0.97)
+    icp = dict(configs.ICP_DEPTH, max_depth=1.5)
+    props = dict(configs.TSDF_2CM, voxel_size=0.01, truncation_distance=0.03, num_buckets=1 << 18, num_blocks=1 << 18)
+    sens = dict(rows=n, cols=n, fx=5.0 * sx, fy=5.0 * sy, cx=(n - 1) / 2, cy=(n - 1) / 2)
+    c = np.sqrt(0.5)
+    pose = np.eye(4)
+    pose[:2, :2] = [[c, -c], [c, c]]
+    mid = (np.arange(n) % 8 >= 2) & (np.arange(n) % 8 < 6)
+    D = np.stack([np.where(mid[:, None] & mid[None], z + 1.5, z) for z in near]).astype(np.float32)
+    o = O.OraclePipeline(props, icp, sens, pose, bits=64)
+    To = np.stack([o.process_frame(d, None) for d in D])
+    assert To[1, 2, 3] > 0.025  # of the 0.03 m between the frames
+    srv = dm.Server(1, n, n)
+    srv.add_trace(props, icp, sens, pose, D)
+    Tg = srv.run(0, 0, 2, want_poses=True)["poses"][0]
+    srv.close()
+    assert np.abs(Tg - To).max() < 1e-3  # a tenth of a voxel
