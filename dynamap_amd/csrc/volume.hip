@@ -1408,8 +1408,8 @@ __device__ __forceinline__ bool far_run(const DmView &v, f3 po, f3 pd, float z, 
 // ...) along the ray through the middle of the wavefront's pixels.  The step's
 // block B has its dilated bit clear, so no block within one of it is near;
 // the rays of the wavefront lie within D voxels of the middle one per axis
-// (D grows with z; the bound holds for any 3x3 part of the pose), and with
-// D <= 5.25 every voxel a ray's sample reads at that z, floor(p - 1) - e to
+// (D grows with |z|; the bound holds for any 3x3 part of the pose and either
+// sign of the focal lengths and of z), and with D <= 5.25 every voxel a ray's sample reads at that z, floor(p - 1) - e to
 // floor(p + 1) + e with the middle ray's p in [8 B - 1/2, 8 B + 7 1/2), stays
 // within a block of B: 5.5 - e would do.  The rest of the margin covers z taken
 // as min_depth + k big instead of the sum of k roundings (at most 0.1 voxel,
@@ -1422,7 +1422,7 @@ __device__ __forceinline__ int beam_steps(const DmView &v, const Intr &s, const 
                                           float ify, int u, int r, int tw_log2, float big, int max_steps) {
   constexpr int kMost = 512;
   const float zmax = v.max_depth;
-  if (!((float)kMost * 6.0e-8f * zmax * inv_vs < 0.1f)) return 0;
+  if (!((float)kMost * 6.0e-8f * fmaxf(zmax, fabsf(v.min_depth)) * inv_vs < 0.1f)) return 0;
   const int lane = threadIdx.x & 63;
   const int ww = tw_log2 == 4 ? 8 : 1 << tw_log2, wh = 64 / ww;  // the wavefront's pixels
   const float hx = 0.5f * (float)(ww - 1), hy = 0.5f * (float)(wh - 1);
@@ -1431,12 +1431,12 @@ __device__ __forceinline__ int beam_steps(const DmView &v, const Intr &s, const 
   const float ex = hx * fabsf(ifx) * inv_vs, ey = hy * fabsf(ify) * inv_vs;  // a mirrored sensor's is negative
   const float d = fmaxf(fmaxf(fabsf(T.m[0]) * ex + fabsf(T.m[1]) * ey, fabsf(T.m[4]) * ex + fabsf(T.m[5]) * ey),
                         fabsf(T.m[8]) * ex + fabsf(T.m[9]) * ey);
-  const float zcap = fminf(zmax, 5.25f / d);
+  const float zcap = 5.25f / d;
   int n = 0;
   while (n < kMost) {
     const float zk = v.min_depth + (float)(n + lane) * big;
     const float px = po.x + pd.x * zk, py = po.y + pd.y * zk, pz = po.z + pd.z * zk;
-    bool far = zk < zcap && fabsf(px) < 1.0e6f && fabsf(py) < 1.0e6f && fabsf(pz) < 1.0e6f;
+    bool far = zk < zmax && fabsf(zk) < zcap && fabsf(px) < 1.0e6f && fabsf(py) < 1.0e6f && fabsf(pz) < 1.0e6f;
     if (far) {
       const unsigned X = floordiv8((int)floorf(px + 0.5f)) + kWin / 2, Y = floordiv8((int)floorf(py + 0.5f)) + kWin / 2,
                      Z = floordiv8((int)floorf(pz + 0.5f)) + kWin / 2;

@@ -388,3 +388,31 @@ def test_raycast_shared_steps_mirrored_sensor(sx, sy):
     Tg = srv.run(0, 0, 2, want_poses=True)["poses"][0]
     srv.close()
     assert np.abs(Tg - To).max() < 1e-3  # a tenth of a voxel
+
+
+# A minimum depth below zero: the rays begin behind the camera, where they lie
+# as far apart as in front.  The map is made while the camera turns, so that
+# surfaces stand on both sides.  Bounds as in test_raycast_ragged_views.
+@pytest.mark.parametrize("n,fx", [(33, 20.0), (64, 40.0), (40, 12.0)])
+@pytest.mark.parametrize("dmin", [-1.5, -3.0])
+def test_raycast_negative_minimum_depth(n, fx, dmin):
+    def turned(a):
+        c, s = np.cos(a), np.sin(a)
+        R = np.eye(4)
+        R[:3, :3] = [[c, 0, s], [0, 1, 0], [-s, 0, c]]
+        return pose @ R
+
+    sc = configs.Scene(1, configs.SEED_BASE + 1002)
+    pose = sc.trajectory(1, configs.SEED_BASE + 1002)[0]
+    props = small_tsdf(min_sensor_depth=dmin)
+    vol = dm.TsdfVolume(props, SENS["rows"], SENS["cols"])
+    for a in np.arange(9) * 0.7:
+        vol.IntegrateScan(sc.render(turned(a), SENS, 7, noise=False)[0], None, SENS, turned(a).astype(np.float32))
+    sens = dict(rows=n, cols=n, fx=fx, fy=fx, cx=(n - 1) / 2, cy=(n - 1) / 2)
+    Tf = turned(0.35).astype(np.float32)
+    gd = vol.Raycast(Tf, sens)[0]
+    od = mirror(vol, props).raycast(Tf.astype(np.float64), sens)[0]
+    hit = od > 0
+    assert 0 < hit.sum() < hit.size  # some rays end at a surface behind the camera
+    assert np.mean((gd > 0) == hit) >= 0.999
+    assert np.mean(np.abs(gd - od)[hit & (gd > 0)] <= 1e-5) >= 0.999
