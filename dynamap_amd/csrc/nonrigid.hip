@@ -311,7 +311,12 @@ __device__ __forceinline__ uint32_t pair_key(int a, int b) {
   return a <= b ? ((uint32_t)a << kNodeBits) | (uint32_t)b : ((uint32_t)b << kNodeBits) | (uint32_t)a;
 }
 
-// contributions: data (v, slot a <= slot b) then ARAP (edge, role)
+// contributions: data (v, slot a <= slot b) then ARAP (edge, role).  A slot is
+// empty (-1) where fewer than kNK nodes lie at a finite distance (a vertex or
+// nodes with coordinates that are not finite, or so large that the squares
+// overflow).  Its contributions keep their place but add nothing: those of a
+// vertex go to block (0, 0) with weights 0, those of an edge to the node's own
+// block with a zero record.
 __global__ __launch_bounds__(256) void k_nr_contrib_emit(const int *__restrict__ node_of_vertex,
                                                         const int *__restrict__ vnn, const long long *__restrict__ off,
                                                         int64_t nv, const int *__restrict__ nbr, int nn,
@@ -328,7 +333,8 @@ __global__ __launch_bounds__(256) void k_nr_contrib_emit(const int *__restrict__
     }
     for (int a = 0; a < kNK; ++a)
       for (int b = a; b < kNK; ++b) {
-        keys[o] = pair_key(vnn[kNK * t + a], vnn[kNK * t + b]);
+        const int na = vnn[kNK * t + a], nb = vnn[kNK * t + b];
+        keys[o] = na < 0 || nb < 0 ? 0u : pair_key(na, nb);
         codes[o] = (uint32_t)(t * 16 + a * 4 + b);
         ++o;
       }
@@ -336,7 +342,7 @@ __global__ __launch_bounds__(256) void k_nr_contrib_emit(const int *__restrict__
   }
   const int64_t e = t - nv;  // ARAP edge e = i * K + k
   if (e >= (int64_t)nn * kNK) return;
-  const int i = (int)(e / kNK), j = nbr[e];
+  const int i = (int)(e / kNK), j = nbr[e] < 0 ? i : nbr[e];
   const long long o = arap_base + 3 * e;
   keys[o] = pair_key(i, i);      codes[o] = kArapTag | (uint32_t)(e * 4 + 0);
   keys[o + 1] = pair_key(j, j);  codes[o + 1] = kArapTag | (uint32_t)(e * 4 + 1);
@@ -345,9 +351,10 @@ __global__ __launch_bounds__(256) void k_nr_contrib_emit(const int *__restrict__
 
 // Per contribution, the weights of the block's two nodes at the vertex (the
 // normalised blend weights of slots a and b; 1 for a vertex that is itself
-// a node); ARAP contributions get 0 (unused).
+// a node, 0 with an empty slot); ARAP contributions get 0 (unused).
 __global__ __launch_bounds__(256) void k_nr_contrib_weights(const uint32_t *__restrict__ codes, long long nc,
                                                            const int *__restrict__ node_of_vertex,
+                                                           const int *__restrict__ vnn,
                                                            const float *__restrict__ vnn_wn, float2 *__restrict__ cw) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= nc) return;
@@ -355,8 +362,9 @@ __global__ __launch_bounds__(256) void k_nr_contrib_weights(const uint32_t *__re
   float2 w = make_float2(0.f, 0.f);
   if (!(code & kArapTag)) {
     const int64_t v = code >> 4;
+    const int64_t a = kNK * v + ((code >> 2) & 3), b = kNK * v + (code & 3);
     if (node_of_vertex[v] >= 0) w = make_float2(1.f, 1.f);
-    else w = make_float2(vnn_wn[kNK * v + ((code >> 2) & 3)], vnn_wn[kNK * v + (code & 3)]);
+    else if (vnn[a] >= 0 && vnn[b] >= 0) w = make_float2(vnn_wn[a], vnn_wn[b]);
   }
   cw[i] = w;
 }
@@ -476,11 +484,11 @@ __device__ __forceinline__ void blend_vertex(const float *__restrict__ verts, co
     b = dq[nd];
   } else {
     b = dq8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const dq8 r0 = dq[vnn[kNK * v]];
+    const dq8 r0 = dq[max(vnn[kNK * v], 0)];
 #pragma unroll
     for (int k = 0; k < kNK; ++k) {
-      const dq8 q = dq[vnn[kNK * v + k]];
-      float w = vnn_w[kNK * v + k];
+      const dq8 q = dq[max(vnn[kNK * v + k], 0)];
+      float w = vnn_w[kNK * v + k];  // 0 for an empty slot (-1)
       const float dt = r0.rw * q.rw + r0.rx * q.rx + r0.ry * q.ry + r0.rz * q.rz;
       if (dt < 0.f) w = -w;
       b.rw = b.rw + w * q.rw; b.rx = b.rx + w * q.rx; b.ry = b.ry + w * q.ry; b.rz = b.rz + w * q.rz;
@@ -684,15 +692,21 @@ __device__ __forceinline__ void data_mesh_vertex(const float pv[3], const float 
   nr_data_record(p, nt, q, pose, o);
 }
 // ARAP edge e = i * K + k (j = k-th neighbour of i): a = T_i g_j, b = T_j g_j,
-// w_ij = max(w_i[k], w_j[k]) (nonRigidICP.cu:494-515); out[8 e] = a, b, w
+// w_ij = max(w_i[k], w_j[k]) (nonRigidICP.cu:494-515); out[8 e] = a, b, w, all
+// zero for an empty slot (j = -1)
 __device__ __forceinline__ void arap_edge(const double *__restrict__ T, const float *__restrict__ verts,
                                           const int *__restrict__ node_vid, const int *__restrict__ nbr,
                                           const float *__restrict__ nbr_w, int e, double *__restrict__ out) {
   const int i = e / kNK, k = e - i * kNK, j = nbr[e];
+  double *o = out + 8 * (size_t)e;
+  if (j < 0) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) o[r] = 0.0;
+    return;
+  }
   const double *Ti = T + 16 * (size_t)i, *Tj = T + 16 * (size_t)j;
   const int64_t gv = node_vid[j];
   const double g0 = verts[3 * gv], g1 = verts[3 * gv + 1], g2 = verts[3 * gv + 2];
-  double *o = out + 8 * (size_t)e;
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
     o[r] = Ti[4 * r] * g0 + Ti[4 * r + 1] * g1 + Ti[4 * r + 2] * g2 + Ti[4 * r + 3];
@@ -1610,7 +1624,7 @@ static int graph_finish(dm_graph *g) {
   DM_TRY(sort_pairs(k0.as<uint32_t>(), k1.as<uint32_t>(), c0.as<uint32_t>(), g->codes, nc, 2 * kNodeBits, st));
   DM_TRY(g->dalloc(&g->cw, nc));
   hipLaunchKernelGGL(k_nr_contrib_weights, dim3(grid_of(nc)), dim3(256), 0, st, g->codes, nc, g->node_of_vertex,
-                     g->vnn_wn, g->cw);
+                     g->vnn, g->vnn_wn, g->cw);
   DM_TRY(dev_alloc(flag, nc * 4));
   DM_TRY(dev_alloc(frank, nc * 8));
   hipLaunchKernelGGL(k_flag_heads, dim3(grid_of(nc)), dim3(256), 0, st, k1.as<uint32_t>(), nc, 0u, flag.as<int>());
@@ -2197,7 +2211,7 @@ int dm_graph_update_nodes(dm_graph *g) {
   if (!g) { set_error("null argument"); return DM_E_INVALID; }
   DM_TRY(graph_links(g));
   hipLaunchKernelGGL(k_nr_contrib_weights, dim3(grid_of(g->ncontrib)), dim3(256), 0, g->stream, g->codes,
-                     g->ncontrib, g->node_of_vertex, g->vnn_wn, g->cw);
+                     g->ncontrib, g->node_of_vertex, g->vnn, g->vnn_wn, g->cw);
   DM_HIP(hipGetLastError());
   DM_HIP(hipStreamSynchronize(g->stream));
   return DM_OK;

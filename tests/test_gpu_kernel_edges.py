@@ -416,3 +416,52 @@ def test_raycast_negative_minimum_depth(n, fx, dmin):
     assert 0 < hit.sum() < hit.size  # some rays end at a surface behind the camera
     assert np.mean((gd > 0) == hit) >= 0.999
     assert np.mean(np.abs(gd - od)[hit & (gd > 0)] <= 1e-5) >= 0.999
+
+
+# Vertices, some of them nodes, that are not finite or so far away that squared
+# distances overflow: their empty neighbour slots (-1) add nothing.  The other
+# vertices' and nodes' neighbours, the block pattern, the blended mesh and a
+# Gauss-Newton step are those of the graph without them (bound of the step as in
+# test_nonrigid_step_node_counts).
+def test_graph_empty_neighbour_slots():
+    from test_oracle_nonrigid import random_cloud
+    V, Nn = random_cloud(3000, 5)
+    bad = np.float32([[np.nan, 0, 0], [0, np.inf, 0], [0, 0, 1e30], [np.nan] * 3, [-np.inf, 0, np.inf], [3e25, 0, 0]])
+    ids = np.linspace(0, len(V) - 1, 40).astype(np.int32)
+    V2, N2 = np.concatenate([V, bad]), np.concatenate([Nn, np.tile(np.float32([0, 0, 1]), (len(bad), 1))])
+    ids2 = np.concatenate([ids, len(V) + np.arange(3, dtype=np.int32)])
+    size = float((V.max(0) - V.min(0)).max())
+    kw = dict(dgw=2.0 * size / len(ids) ** (1 / 3))
+    g, h = dm.DefGraph(V, Nn, node_ids=ids, **kw), dm.DefGraph(V2, N2, node_ids=ids2, **kw)
+    (_, nbr, nw), (_, nbr2, nw2) = g.nodes(), h.nodes()
+    np.testing.assert_array_equal(nbr2[:40], nbr)
+    np.testing.assert_array_equal(nw2[:40], nw)
+    assert (nbr2[40:] == -1).all() and (nw2[40:] == 0).all()
+    (vnn, vw), (vnn2, vw2) = g.vertex_neighbours(), h.vertex_neighbours()
+    np.testing.assert_array_equal(vnn2[:3000], vnn)
+    np.testing.assert_array_equal(vw2[:3000], vw)
+    want = np.full((6, 4), -1)
+    want[2, 0] = 42  # the third is a node and finite: its own nearest
+    np.testing.assert_array_equal(vnn2[3000:], want)
+    assert h.num_blocks() == g.num_blocks() + 3  # the three nodes' own
+    T = np.tile(np.eye(4), (43, 1, 1))
+    T[:, :3, 3] = np.random.default_rng(1).normal(0, 0.01, (43, 3))
+    g.set_transforms(T[:40])
+    h.set_transforms(T)
+    for a, b in zip(dm.DqBlender(g).blendMesh(), dm.DqBlender(h).blendMesh()):
+        np.testing.assert_array_equal(b[:3000], a)
+    g.set_transforms(np.tile(np.eye(4), (40, 1, 1)))
+    h.set_transforms(np.tile(np.eye(4), (43, 1, 1)))
+    target = (V + 0.004 * np.sin(V[:, [1, 2, 0]] / size * 3)).astype(np.float32)
+    kw = dict(gn_iterations=1, pcg_iterations=400, pcg_tol=1e-9, damping=1.0)
+    s = dm.NonRigidICP(**kw).solve_mesh(g, target, Nn, np.eye(4))
+    # no target for the others: a zero normal
+    s2 = dm.NonRigidICP(**kw).solve_mesh(h, np.concatenate([target, np.zeros((6, 3), np.float32)]),
+                                        np.concatenate([Nn, np.zeros((6, 3), np.float32)]), np.eye(4))
+    assert s2["residuals"] == s["residuals"] > 2000
+    moved = np.abs(g.transforms() - np.eye(4)).max()
+    assert moved > 1e-4
+    assert np.abs(h.transforms()[:40] - g.transforms()).max() <= 1e-3 * moved
+    np.testing.assert_array_equal(h.transforms()[40:], np.tile(np.eye(4), (3, 1, 1)))
+    h.defGraphUpdateNodes()
+    np.testing.assert_array_equal(h.vertex_neighbours()[0], vnn2)
