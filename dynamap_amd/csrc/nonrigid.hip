@@ -229,7 +229,8 @@ __global__ __launch_bounds__(256) void k_nr_knn(const float *__restrict__ verts,
     for (int k = 0; k < kNK; ++k) d[k] = INFINITY;
     for (int t = 0; t < m; ++t) {
       float x = dist2(t);
-      if (t * step == self) x = INFINITY;
+      // fminf and fmaxf would both keep d[k] beside a NaN and so list it twice
+      if (x != x || t * step == self) x = INFINITY;
 #pragma unroll
       for (int k = 0; k < kNK; ++k) {
         const float lo = fminf(d[k], x);

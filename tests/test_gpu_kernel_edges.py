@@ -465,3 +465,26 @@ def test_graph_empty_neighbour_slots():
     np.testing.assert_array_equal(h.transforms()[40:], np.tile(np.eye(4), (3, 1, 1)))
     h.defGraphUpdateNodes()
     np.testing.assert_array_equal(h.vertex_neighbours()[0], vnn2)
+
+
+# Nodes without coordinates among those that the one-lane search looks at first
+# (65536 queries or more): they are nobody's neighbours and change nobody's.
+# Whole coordinates as in test_nearest_nodes_lanes_and_ties.
+@pytest.mark.parametrize("nodes,verts", [(1087, 68000), (2049, 66000)])
+def test_nearest_nodes_without_coordinates(nodes, verts):
+    rng = np.random.default_rng(nodes)
+    cell = rng.permutation(41 ** 3)[:verts]
+    V = np.stack([cell // 1681, cell // 41 % 41, cell % 41], 1).astype(np.float32)
+    ids = rng.permutation(verts)[:nodes].astype(np.int32)
+    Q = V[ids].astype(np.int64)
+    lost = np.arange(0, nodes, 32)[1::2]
+    V[ids[lost]] = np.nan
+    g = dm.DefGraph(V, np.tile(np.float32([0, 0, 1]), (verts, 1)), dgw=20.0, node_ids=ids)
+    vnn = g.vertex_neighbours()[0]
+    for a in range(0, verts, 8192):
+        P = V[a:a + 8192]
+        key = ((np.nan_to_num(P).astype(np.int64)[:, None] - Q[None]) ** 2).sum(2) * nodes + np.arange(nodes)
+        key[:, lost] = 1 << 40
+        want = np.sort(np.partition(key, 3, 1)[:, :4], 1) % nodes
+        want[np.isnan(P[:, 0])] = -1
+        np.testing.assert_array_equal(vnn[a:a + 8192], want)
