@@ -203,6 +203,12 @@ __device__ __forceinline__ uint32_t to_u8(float x) {
   return (uint32_t)x;
 }
 
+// Orders a wavefront's LDS writes and reads before its later ones by other lanes.
+__device__ __forceinline__ void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---- lane sums through DPP row permutes
 // x moved across lanes by a DPP pattern
 template <int kCtrl> __device__ __forceinline__ float dpp_f32(float x) {

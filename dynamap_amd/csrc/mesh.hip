@@ -93,12 +93,6 @@ __device__ __forceinline__ AxisCorner axis_corner(float c, float off, float vs) 
   return a;
 }
 
-// Orders a wavefront's LDS writes before its later reads by other lanes.
-__device__ __forceinline__ void wave_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // A wavefront holds one block: its voxels and a one-voxel halo, the per-axis
 // corner values, and the list of cells that are worth evaluating.  rows[r] has,
 // for the 10 voxels of row r = (x + 1) * 10 + (y + 1), observed in bits 0..9,

@@ -420,6 +420,7 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
 #pragma unroll
   for (int q = 0; q < 16; ++q)
     if (e == q) S.m[q] = E[q];
+  wave_lds();
   const double *Ti = S.pd + PD_TINC;
   double tinc = S.m[4 * r4] * Ti[c4] + S.m[4 * r4 + 1] * Ti[4 + c4] + S.m[4 * r4 + 2] * Ti[8 + c4] +
                 S.m[4 * r4 + 3] * Ti[12 + c4];
@@ -447,11 +448,13 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
       if (lane == 0) atomicAdd(&v.ctr[C_ICP_FAIL], 1);
     }
     if (lane < 16) S.t[e] = tinc;
+    wave_lds();
     const double *Tp = S.pd + PD_TPREV;
     const double T = Tp[4 * r4] * S.t[c4] + Tp[4 * r4 + 1] * S.t[4 + c4] + Tp[4 * r4 + 2] * S.t[8 + c4] +
                      Tp[4 * r4 + 3] * S.t[12 + c4];
     const double Tf = (double)(float)T;  // the inverse is the float pose's
-    if (lane < 16) S.m[e] = Tf;
+    if (lane < 16) S.m[e] = Tf;  // its last readers are before the wave_lds above
+    wave_lds();
     const double inv = r4 == 3 ? (c4 == 3 ? 1.0 : 0.0)
                        : c4 < 3 ? S.m[4 * c4 + r4]
                                 : -(S.m[r4] * S.m[3] + S.m[4 + r4] * S.m[7] + S.m[8 + r4] * S.m[11]);
