@@ -741,6 +741,7 @@ int dm_session_create(const dm_tsdf_props *props, const dm_icp_props *icp, const
   if (r == DM_OK) {
     s->push_view();
     hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);  // init_pose is the caller's
     if (e != hipSuccess) r = hip_fail(e, "session view");
   }
   if (r != DM_OK) { s->release(); delete s; return r; }

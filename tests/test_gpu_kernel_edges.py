@@ -488,3 +488,23 @@ def test_nearest_nodes_without_coordinates(nodes, verts):
         want = np.sort(np.partition(key, 3, 1)[:, :4], 1) % nodes
         want[np.isnan(P[:, 0])] = -1
         np.testing.assert_array_equal(vnn[a:a + 8192], want)
+
+
+# The initial pose is read before the session's creation returns: the caller's
+# array is changed right after it.
+def test_session_reads_initial_pose_before_return(room):
+    import ctypes as C
+    from dynamap_amd import _native as N
+    depth, poses = room
+    w = configs.WORKLOADS["rigid-320x240-2cm"]
+    for _ in range(4):
+        T = np.ascontiguousarray(poses[1], np.float64)
+        keep, h = T.copy(), C.c_void_p()
+        N.check(N.lib().dm_session_create(C.byref(configs.tsdf_props(small_tsdf())), C.byref(configs.icp_props(w["icp"])),
+                                          C.byref(configs.sensor(SENS)), N.ptr(T), C.byref(h)))
+        T[:] = np.nan
+        got = np.zeros((4, 4))
+        d = np.ascontiguousarray(depth[1])
+        N.check(N.lib().dm_session_process_frame(h, N.ptr(d), None, 0, N.ptr(got)))
+        N.lib().dm_session_destroy(h)
+        np.testing.assert_array_equal(got, keep)
