@@ -226,9 +226,9 @@ int Sess::stage_rgb(const uint8_t *host_rgb) {
   return DM_OK;
 }
 
-int Sess::reserve_out() {
+int Sess::reserve_out(bool pack) {
   const size_t P = (size_t)max_rows * max_cols;
-  if (!d_pack) DM_TRY(dalloc(&d_pack, P * 7, false));
+  if (pack && !d_pack) DM_TRY(dalloc(&d_pack, P * 7, false));
   for (hipEvent_t &e : ev_out)
     if (!e) DM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return DM_OK;
@@ -458,7 +458,7 @@ int dm_volume_raycast(dm_volume *vol, const float pose[16], const dm_sensor *sen
                       float *host_vertex, float *host_normal, uint8_t *host_rgb) {
   if (!vol || !pose) { set_error("null argument"); return DM_E_INVALID; }
   DM_TRY(vol->set_sensor(sensor));
-  DM_TRY(vol->reserve_out());
+  DM_TRY(vol->reserve_out(host_vertex || host_normal));
   vol->push_view(pose);
   Launch L = vol->launch();
   L.ray_depth = vol->d_ray_depth;
@@ -798,7 +798,7 @@ int dm_session_get_pose(dm_session *s, double pose[16]) {
 int dm_session_source_maps(dm_session *s, const float *host_depth, const uint8_t *host_rgb, int32_t level,
                            float *host_vertex, float *host_normal, float *host_intensity) {
   if (!s || !host_depth || level < 0 || level >= kLevels) { set_error("invalid argument"); return DM_E_INVALID; }
-  DM_TRY(s->reserve_out());
+  DM_TRY(s->reserve_out(host_vertex || host_normal || host_intensity));
   DM_TRY(s->frame_from_host(host_depth, host_rgb, nullptr));
   DM_TRY(s->stage_depth(host_depth));
   DM_TRY(s->stage_rgb(host_rgb));

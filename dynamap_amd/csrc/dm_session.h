@@ -44,7 +44,7 @@ struct Sess {
   size_t out_half = 0;           // bytes of one half of it, for results
   float *d_ray_depth = nullptr;  // raycast outputs for host readback
   uint8_t *d_ray_rgb = nullptr;
-  float *d_pack = nullptr;       // packed maps for host readback (7 floats per pixel, allocated on first use)
+  float *d_pack = nullptr;       // packed maps for host readback (7 floats per pixel, allocated when a map is first asked for)
   hipEvent_t ev_out[2] = {nullptr, nullptr};
   float *d_depth_f = nullptr;    // bilateral-filtered depth for tracking (when enabled)
   int filt_r = 0;                // filter radius, 0 = off
@@ -62,7 +62,7 @@ struct Sess {
   int stage_depth(const float *host_depth);  // upload the frame through pinned memory; h.depth / h.rgb are set
   int stage_rgb(const uint8_t *host_rgb);    // by frame_from_host
   int frame_from_host(const float *host_depth, const uint8_t *host_rgb, const float *pose);
-  int reserve_out();
+  int reserve_out(bool pack);  // pack: with d_pack
   struct Out { void *dst; const void *src; size_t bytes; };
   int read_out(const Out *out, int n);       // device results to host memory; waits
   int read_small(void *dst, const void *src, size_t bytes);  // up to 1 KiB; waits for the stream

@@ -508,3 +508,33 @@ def test_session_reads_initial_pose_before_return(room):
         N.check(N.lib().dm_session_process_frame(h, N.ptr(d), None, 0, N.ptr(got)))
         N.lib().dm_session_destroy(h)
         np.testing.assert_array_equal(got, keep)
+
+
+# Results that need no packed copy on the device take no memory for one: 448 MB
+# at 4000x4000 pixels.
+def test_depth_render_takes_no_map_memory():
+    import ctypes as C
+    from dynamap_amd import _native as N
+    n = 4000
+    sens = dict(rows=n, cols=n, fx=3000.0, fy=3000.0, cx=2000.0, cy=2000.0)
+    vol = dm.TsdfVolume(small_tsdf(), n, n)
+    T, d, v = np.eye(4, dtype=np.float32), np.ones((n, n), np.float32), np.ones((n, n, 3), np.float32)
+    rt = C.CDLL("libamdhip64.so.7")  # the runtime that the library links
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert rt.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    def taken(vertex):
+        before = free()
+        N.check(N.lib().dm_volume_raycast(vol._h, N.ptr(T), C.byref(configs.sensor(sens)), N.ptr(d), vertex, None, None))
+        return before - free()
+
+    taken(None)  # whatever a first launch takes
+    vol.close()
+    vol = dm.TsdfVolume(small_tsdf(), n, n)
+    assert taken(None) < 28 * n * n / 2
+    assert not d.any()
+    assert taken(N.ptr(v)) >= 28 * n * n / 2
+    assert not v.any()
