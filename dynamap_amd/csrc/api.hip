@@ -136,7 +136,7 @@ int Sess::init(const dm_tsdf_props &p, uint32_t rows, uint32_t cols) {
   DM_TRY(dalloc(&d_view, 1));
   DM_TRY(dalloc(&d_active, 1));
   // a frame's depth and colour, or two chunks of results; then read_small's 1 KiB
-  out_half = std::max<size_t>((P * 7 / 2 + 63) & ~(size_t)63, 256 << 10);
+  out_half = std::max<size_t>(((P * 7 + 1) / 2 + 63) & ~(size_t)63, 256 << 10);
   pinned_bytes = 2 * out_half + 1024;
   DM_HIP(hipHostMalloc((void **)&h_pinned, pinned_bytes, hipHostMallocDefault));
   // identity poses
