@@ -44,18 +44,28 @@ __device__ __forceinline__ int key_bucket(const DmView &v, uint64_t key) {
   return hash_bucket(x, y, z, v.num_buckets);
 }
 
+// Adds the number of active lanes with `take` to *counter with one addition for the
+// wavefront; returns this lane's place.
+__device__ __forceinline__ int wave_append(int32_t *counter, bool take) {
+  const unsigned long long m = __ballot(take);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (m && lane == __builtin_ctzll(m)) base = atomicAdd(counter, __popcll(m));
+  return m ? __shfl(base, __builtin_ctzll(m), 64) + __popcll(m & ((1ull << lane) - 1ull)) : 0;
+}
+
 // A workgroup's traversal state in LDS: the set of the blocks its rays have
 // already handled (looked up, and noted when missing), since neighbouring
 // rays visit mostly the same blocks, so that each is looked up in the global
 // table about once per workgroup; and the key-set slots of the new keys it was
-// first to note.
+// first to note, up to `room`.
 constexpr int kSeenSlots = 1024;
 constexpr int kSeenProbes = 8;
 constexpr int kNewSlots = 1024;
 struct RayWG {
   unsigned long long seen[kSeenSlots];
   int32_t slots[kNewSlots];
-  int nnew, base, visits;
+  int nnew, base, visits, room;
 };
 
 // Entry idx of the frame's key list: the key in slot h of the key set, chained
@@ -69,7 +79,7 @@ __device__ __forceinline__ void list_new_key(const DmView &v, int idx, uint64_t 
     // no room in the frame's key list: release the slot so that a later frame
     // can insert the key
     atomicExch((unsigned long long *)&v.dset[h], 0ull);
-    atomicAdd(&v.ctr[C_DSET_OVF], 1);
+    wave_append(&v.ctr[C_DSET_OVF], true);
   }
 }
 
@@ -79,6 +89,13 @@ __device__ __forceinline__ void list_new_key(const DmView &v, int idx, uint64_t 
 // by thousands of rays).  The list entry is left to the workgroup's end, where
 // one addition to the list's length serves all its keys: the length is one
 // address, and one addition per key took 1.3 ms of a first frame at 4 mm.
+// Keys beyond the workgroup's room are listed at once.  The rooms of all
+// workgroups together are half the list, the set has twice the list's slots
+// and a key that the list has no room for leaves its slot again, so the keys that
+// stay fill at most three quarters of the set.  Without that bound the keys held
+// back filled it where a frame has far more new blocks than the list's length
+// (250 000 against a pool of 32 768), and each further key walked all of it: 1.6 s
+// a frame, now 3.9 ms.
 __device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key, RayWG &wg) {
   uint32_t h = (uint32_t)mix64(key) & (uint32_t)v.dset_mask;
   for (int probe = 0; probe <= v.dset_mask; ++probe) {
@@ -88,8 +105,8 @@ __device__ __forceinline__ void note_new_key(const DmView &v, uint64_t key, RayW
       const uint64_t prev = atomicCAS((unsigned long long *)&v.dset[h], 0ull, (unsigned long long)key);
       if (prev == 0ull) {
         const int k = atomicAdd(&wg.nnew, 1);
-        if (k < kNewSlots) wg.slots[k] = (int32_t)h;
-        else list_new_key(v, atomicAdd(&v.ctr[C_N_NEW], 1), key, (int32_t)h);
+        if (k < wg.room) wg.slots[k] = (int32_t)h;
+        else list_new_key(v, wave_append(&v.ctr[C_N_NEW], true), key, (int32_t)h);
         return;
       }
       if (prev == key) return;
@@ -267,18 +284,25 @@ __global__ __launch_bounds__(256) void k_alloc_rays(const DmView *__restrict__ v
   if (slot_ < 0) return;
   const DmView &v = views[slot_];
   const int tiles_x = (v.cols + 15) >> 4;
-  const int tile = blockIdx.x;
-  if (tile >= tiles_x * ((v.rows + 15) >> 4)) return;
+  const int tile = blockIdx.x, ntiles = tiles_x * ((v.rows + 15) >> 4);
+  if (tile >= ntiles) return;
   __shared__ RayWG wg;
   for (int k = threadIdx.x; k < kSeenSlots; k += 256) wg.seen[k] = 0ull;
-  if (threadIdx.x == 0) wg.visits = wg.nnew = 0;
+  if (threadIdx.x == 0) {
+    wg.visits = wg.nnew = 0;
+    // below 4 per workgroup the list is so short that the keys on their way out of
+    // the set crowd it: 1 at a list of 4096 took 19 ms a frame of 250 000 new
+    // blocks, none takes 6.3
+    const int room = min(kNewSlots, v.newcap / 2 / ntiles);
+    wg.room = room < 4 ? 0 : room;
+  }
   __syncthreads();
   const int u = (tile % tiles_x) * 16 + (threadIdx.x & 15);
   const int r = (tile / tiles_x) * 16 + (threadIdx.x >> 4);
   const int n = alloc_ray<kCount>(v, u, r, wg);
   if (n) atomicAdd(&wg.visits, n);
   __syncthreads();
-  const int nnew = min(wg.nnew, kNewSlots);
+  const int nnew = min(wg.nnew, wg.room);
   if (threadIdx.x == 0) {
     if (wg.visits) atomicAdd(&v.ctr[C_NVISIT], wg.visits);
     if (nnew) wg.base = atomicAdd(&v.ctr[C_N_NEW], nnew);
@@ -289,16 +313,6 @@ __global__ __launch_bounds__(256) void k_alloc_rays(const DmView *__restrict__ v
     const int32_t h = wg.slots[k];
     list_new_key(v, wg.base + k, __atomic_load_n((unsigned long long *)&v.dset[h], __ATOMIC_RELAXED), h);
   }
-}
-
-// Adds the number of lanes with `take` to *counter with one addition for the
-// wavefront; returns this lane's place.
-__device__ __forceinline__ int wave_append(int32_t *counter, bool take) {
-  const unsigned long long m = __ballot(take);
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  if (m && lane == __builtin_ctzll(m)) base = atomicAdd(counter, __popcll(m));
-  return m ? __shfl(base, __builtin_ctzll(m), 64) + __popcll(m & ((1ull << lane) - 1ull)) : 0;
 }
 
 // Canonical rank of each new key within its bucket (ascending packed key);

@@ -538,3 +538,48 @@ def test_depth_render_takes_no_map_memory():
     assert not d.any()
     assert taken(N.ptr(v)) >= 28 * n * n / 2
     assert not v.any()
+
+
+@pytest.fixture(scope="module")
+def room_8mm():
+    depth, _, poses = configs.make_sequence("rigid-640x480-8mm", 2)
+    return depth, poses
+
+
+# The keys that a workgroup may hold back before it lists them: 109, 13, 6 and 4
+# in each of 1200 workgroups, of a first frame's 11 000 new blocks (the list is as
+# long as the pool; at 4 the second frame's blocks pass it).  The same slots and
+# drops as the oracle's.
+@pytest.mark.parametrize("num_blocks", [1 << 18, 1 << 15, 1 << 14, 11000])
+def test_allocation_room_of_workgroups(room_8mm, num_blocks):
+    import oracle_lib as O
+    from test_gpu_volume import table_keys
+    depth, poses = room_8mm
+    w = configs.WORKLOADS["rigid-640x480-8mm"]
+    props = dict(w["tsdf"], num_buckets=1 << 16, num_blocks=num_blocks)
+    vol, ora = dm.TsdfVolume(props, 480, 640), O.OracleVolume(props, 32)
+    for f in range(2):
+        Tf = poses[f].astype(np.float32)
+        vol.AllocateFromDepth(depth[f], w["sensor"], Tf)
+        ora.allocate(depth[f], w["sensor"], Tf.astype(np.float64))
+        np.testing.assert_array_equal(table_keys(vol.GetHashEntries()), ora.table()[0])
+        assert vol.counters()["dropped_pool"] == ora.dropped()["pool"]
+
+
+# A scene far beyond the pool: each frame's 250 000 new blocks against a list and a
+# pool of 4096 and 32768.  Every frame ends within 0.1 s (5 ms here; 0.45 and 1.6 s
+# when the keys held back filled the frame's set) and the pool fills.
+@pytest.mark.parametrize("num_blocks", [1 << 12, 1 << 15])
+def test_allocation_far_beyond_the_pool(num_blocks):
+    import time
+    w = configs.WORKLOADS["large-640x480-4mm"]
+    depth, _, poses = configs.make_sequence("large-640x480-4mm", 1)
+    vol = dm.TsdfVolume(dict(w["tsdf"], num_buckets=1 << 18, num_blocks=num_blocks), 480, 640)
+    Tf, took = poses[0].astype(np.float32), []
+    for _ in range(4):
+        t = time.perf_counter()
+        vol.AllocateFromDepth(depth[0], w["sensor"], Tf)
+        took.append(time.perf_counter() - t)
+    c = vol.counters()
+    assert c["allocated"] == num_blocks and c["dropped_keyset"] > 4 * 200000 and c["dropped_pool"] == 3 * num_blocks
+    assert min(took[1:]) < 0.1
