@@ -1563,17 +1563,23 @@ static int graph_build_nodes(dm_graph *g, const float *h_verts, const float *h_n
 }
 
 // Nearest nodes of nq queries (the nodes themselves with query_vid, else the
-// vertices): as many lanes per query as bring the launch to 4 wavefronts on
-// each of the 1024 SIMDs, and one from 65536 queries on, where leaving out
-// groups pays (60000 queries, 4048 nodes: 8 lanes 110 us, one 93; 40000: 86 and 108).
+// vertices).  Few queries take many lanes each, to fill the GPU; many take one,
+// which leaves out groups of nodes.  Measured in us at 300, 1100, 4048 and 9000
+// nodes of a cylinder:
+//   64 against 8 lanes   at 10240 queries  27/13  34/25  54/55  81/93
+//                        at 12288          31/13  39/25  62/53  93/93
+//   8 lanes against 1    at 59800 queries  25/28  53/62  120/109  201/177
+//                        at 66080          28/28  59/55  132/111  224/178
+// with vertices in the mesh's order.  In random order a wavefront's queries leave
+// out less together, and one lane gains from 120000 queries on only, so the second
+// line takes the latest of the four.
 static void launch_knn(dm_graph *g, const int *query_vid, int64_t nq, int *ids, float *w, float *wn) {
   auto run = [&](auto kernel, int lanes) {
     hipLaunchKernelGGL(kernel, dim3(grid_of((long long)nq * lanes)), dim3(256), 0, g->stream, g->verts, g->node_vid,
                        g->nn, query_vid, nq, g->props.dgw, ids, w, wn);
   };
-  const int64_t fill = 1 << 18;
-  if (nq * 4 >= fill) run(k_nr_knn<1>, 1);
-  else if (nq * 16 >= fill) run(k_nr_knn<8>, 8);
+  if (nq >= 65536) run(k_nr_knn<1>, 1);
+  else if (nq >= 12288) run(k_nr_knn<8>, 8);
   else run(k_nr_knn<64>, 64);
 }
 

@@ -199,8 +199,8 @@ def test_nonrigid_step_node_counts(nodes):
         assert np.bincount(pairs[:, 0]).max() > 16
 
 
-# Nearest nodes where a query's lanes change in number (64 below 16384 queries,
-# 8 below 65536, then 1) and where the nodes fill, miss and pass a tile of 1024
+# Nearest nodes where a query's lanes change in number (8 below 65536 queries,
+# then 1) and where the nodes fill, miss and pass a tile of 1024
 # and a group of 32.
 # Whole coordinates: squared distances are exact and full of ties, which go to
 # the lower index.
@@ -583,3 +583,10 @@ def test_allocation_far_beyond_the_pool(num_blocks):
     c = vol.counters()
     assert c["allocated"] == num_blocks and c["dropped_keyset"] > 4 * 200000 and c["dropped_pool"] == 3 * num_blocks
     assert min(took[1:]) < 0.1
+
+
+# The other change of a query's lanes in number (64 below 12288 queries, then 8),
+# of vertices and of nodes.
+@pytest.mark.parametrize("nodes,verts", [(1025, 12287), (1025, 12288), (12287, 12400), (12289, 12400)])
+def test_nearest_nodes_few_queries(nodes, verts):
+    test_nearest_nodes_lanes_and_ties(nodes, verts)
