@@ -435,11 +435,11 @@ __device__ __forceinline__ float merge_channel(float c, float w, float c_new, fl
 
 // a / b, correctly rounded, with b's reciprocal shared between quotients: the
 // steps of the IEEE division (reciprocal, one Newton step, two residual
-// corrections) without the scaling that it needs for extreme exponents.  The
-// caller keeps |b| and a nonzero |a| within 2^-80 .. 2^80.  (Compared with a / b
-// on 1.7e10 pairs, every mantissa of b and every b from 1 to 256 with every
-// mantissa of a among them; sqrt_nr with sqrtf on every x in 2^-90 .. 2^90: no
-// difference.)
+// corrections) without the scaling that it needs for extreme exponents, so for
+// |b| and |a| within 2^-80 .. 2^80, or a = 0.  Below that the residuals may
+// underflow and the quotient be some ulp off, still tiny and of a's sign.
+// (tests/test_shared_division.py restates these steps and sqrt_nr's for every
+// mantissa of b and x, with the hardware's reciprocal one ulp off either way.)
 __device__ __forceinline__ float recip_nr(float b) {
   const float r = __builtin_amdgcn_rcpf(b);
   return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
@@ -468,8 +468,9 @@ __device__ __forceinline__ int voxel_pixel(const Intr &s, f3 vc, float &dist) {
   dist = norm(mk(0.f, 0.f, 0.f) - vc);
   return pu >= 0 && pv >= 0 && pu < s.cols && pv < s.rows ? pv * s.cols + pu : -1;
 }
-// The same values where every operand is of ordinary size: the quotients share
-// one reciprocal, and roundf(x) for the pixels that matter is trunc(x +
+// The same values where every operand is of ordinary size (a numerator may be
+// smaller: beside the principal point its quotient moves no pixel, exact or not):
+// the quotients share one reciprocal, and roundf(x) for the pixels that matter is trunc(x +
 // pred(1/2)) with the image test on that sum (x = -1/2, which rounds to -1,
 // gives a negative sum).
 constexpr float kOrdLo = 0x1p-40f, kOrdHi = 0x1p40f;

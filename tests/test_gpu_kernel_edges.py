@@ -590,3 +590,30 @@ def test_allocation_far_beyond_the_pool(num_blocks):
 @pytest.mark.parametrize("nodes,verts", [(1025, 12287), (1025, 12288), (12287, 12400), (12289, 12400)])
 def test_nearest_nodes_few_queries(nodes, verts):
     test_nearest_nodes_lanes_and_ties(nodes, verts)
+
+
+# Camera coordinates far below the range that the integration's shared division
+# is exact in: a camera moved by less than 1e-20 m beside voxels at x = y = 0,
+# with the principal point on a pixel's centre and on its edge, against the FP32
+# transcription.
+@pytest.mark.parametrize("t", [0.0, 1e-20, -1e-30, 1e-41])
+@pytest.mark.parametrize("c", [0.0, -0.5, 7.5, 8.0])
+def test_integration_tiny_numerators(t, c):
+    import oracle_lib as O
+    sens = dict(rows=16, cols=16, fx=20.0, fy=20.0, cx=c, cy=c)
+    props = small_tsdf()
+    vol, ora = dm.TsdfVolume(props, 16, 16), O.OracleVolume(props, 32)
+    T = np.eye(4, dtype=np.float32)
+    T[0, 3], T[1, 3] = t, -t
+    d = np.full((16, 16), 1.0, np.float32)
+    d[1:] = 1.03  # a voxel's pixel shows in its value
+    for _ in range(2):
+        vol.IntegrateScan(d, None, sens, T)
+        ora.integrate_scan(d, None, sens, T.astype(np.float64))
+    gx, gs, _, gw = vol.blocks()
+    ox, os_, _, ow = ora.blocks()
+    gi, oi = np.lexsort(gx.T[::-1]), np.lexsort(ox.T[::-1])
+    np.testing.assert_array_equal(gx[gi], ox[oi])
+    np.testing.assert_array_equal(gw[gi], ow[oi])
+    np.testing.assert_array_equal(gs[gi], os_[oi].astype(np.float32))
+    assert (gw > 0).any()
