@@ -617,3 +617,49 @@ def test_integration_tiny_numerators(t, c):
     np.testing.assert_array_equal(gw[gi], ow[oi])
     np.testing.assert_array_equal(gs[gi], os_[oi].astype(np.float32))
     assert (gw > 0).any()
+
+
+# The shared first steps have their own pixels per wavefront for each tile width:
+# the same poses bit for bit at all four, batched at frame sizes that are no
+# multiple of the tiles, with a narrow and a wide field of view; the poses are
+# the oracle's within 1e-3 m.
+@pytest.mark.parametrize("rows,cols,fx", [(97, 131, 90.0), (66, 70, 30.0), (75, 203, 260.0)])
+def test_raycast_tile_widths(rows, cols, fx):
+    import oracle_lib as O
+    sens = dict(rows=rows, cols=cols, fx=fx, fy=fx, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    sc = configs.Scene(1, configs.SEED_BASE + 1002)
+    poses = sc.trajectory(5, configs.SEED_BASE + 1002)
+    D = np.stack([sc.render(p, sens, 7, noise=False)[0] for p in poses])
+    got = []
+    for width in (16, 8, 32, 64):
+        srv = dm.Server(2, 120, 220)  # frames smaller than the launch
+        srv.add_trace(small_tsdf(), configs.ICP_DEPTH, sens, poses[0], D)
+        srv.add_trace(small_tsdf(voxel_size=0.03, truncation_distance=0.09), configs.ICP_DEPTH, sens, poses[0], D)
+        srv.set_shapes(ray_tile_width=width)
+        got.append(srv.run(0, 0, 5, want_poses=True)["poses"])
+        srv.close()
+    for g in got[1:]:
+        np.testing.assert_array_equal(g, got[0])
+    o = O.OraclePipeline(small_tsdf(), configs.ICP_DEPTH, sens, poses[0], bits=64)
+    To = np.stack([o.process_frame(d, None) for d in D])
+    assert np.abs(To[-1, :3, 3] - To[0, :3, 3]).max() > 1e-3
+    assert np.abs(got[0][0] - To).max() < 1e-3
+
+
+# test_raycast_ragged_views where the oracle must see the room, so that the
+# comparison cannot pass on two empty images.
+@pytest.mark.parametrize("rows,cols,fx,dmin", [(1, 1, 60.0, 0.3), (7, 9, 12.0, 0.3), (17, 33, 30.0, 0.1),
+                                              (96, 97, 40.0, 0.3), (130, 63, 400.0, 1.2)])
+def test_raycast_ragged_views_see_the_room(room, rows, cols, fx, dmin):
+    depth, poses = room
+    props = small_tsdf(min_sensor_depth=dmin)
+    vol = dm.TsdfVolume(props, SENS["rows"], SENS["cols"])
+    for f in range(3):
+        vol.IntegrateScan(depth[f], None, SENS, poses[f].astype(np.float32))
+    sens = dict(rows=rows, cols=cols, fx=fx, fy=fx, cx=(cols - 1) / 2, cy=(rows - 1) / 2)
+    Tf = poses[1].astype(np.float32)
+    gd = vol.Raycast(Tf, sens)[0]
+    od = mirror(vol, props).raycast(Tf.astype(np.float64), sens)[0]
+    hit = od > 0
+    assert hit.any() and np.mean((gd > 0) == hit) >= 0.999
+    assert np.mean(np.abs(gd - od)[hit & (gd > 0)] <= 1e-5) >= 0.999
