@@ -106,9 +106,10 @@ struct Cells {
 };
 constexpr int kMcWaves = 4;  // wavefronts per workgroup
 
-// Loads the block.  False when no cell can give a triangle: a cell's first
-// corner sample reads its own voxel, so a block without an observed voxel is
-// left before its halo is read.  `regular`: every cell samples exactly its own
+// Loads the block.  False when no cell can give a triangle: on every axis one of a
+// cell's corner indices lies in the cell's block (regular or not, at any block
+// key), so some sample reads a voxel of the block, and a block without an observed
+// voxel is left before its halo is read.  `regular`: every cell samples exactly its own
 // voxel and the 26 around it, with weights in [0.25, 0.75] (true but for
 // coordinates so large that rounding moves them).
 __device__ __forceinline__ bool load_cells(const DmView &v, int ptr, Cells &C, bool &regular) {

@@ -8,6 +8,7 @@ import json
 import os
 
 import numpy as np
+import pytest
 
 import oracle_lib as O
 from dynamap_amd import _native as N
@@ -44,3 +45,20 @@ def test_product_table():
     out = np.zeros(256, np.uint64)
     assert lib.dm_mc_tri_table(out.ctypes.data_as(ctypes.c_void_p)) == 0
     check(out)
+
+
+@pytest.mark.parametrize("vs", [0.02, 0.05, 0.003])
+def test_cells_sample_their_own_block(vs):
+    """The extraction leaves a block without observed voxels at once: whatever
+    the rounding at large coordinates, on each axis a cell's corner samples have
+    a voxel index in the cell's own block (here at every cell coordinate of the
+    block keys' range, in the kernel's FP32 operations)."""
+    f, vs = np.float32, np.float32(vs)
+    for lo in range(-(1 << 23), 1 << 23, 1 << 21):
+        g = np.arange(lo, lo + (1 << 21))
+        own = np.zeros(len(g), bool)
+        for off in (-vs / f(2), vs / f(2)):
+            dual = (g.astype(f) * vs + f(0) + off) - vs / f(2)
+            for q in (dual / vs, (dual + vs) / vs):
+                own |= np.trunc(q + np.sign(q) * f(0.5)).astype(np.int64) >> 3 == g >> 3
+        assert own.all()
