@@ -352,10 +352,11 @@ __global__ __launch_bounds__(256) void k_nr_contrib_emit(const int *__restrict__
 
 // Per contribution, the weights of the block's two nodes at the vertex (the
 // normalised blend weights of slots a and b; 1 for a vertex that is itself
-// a node, 0 with an empty slot); ARAP contributions get 0 (unused).
+// a node); ARAP contributions get 0 (unused).  Both are 0 where either is, an
+// empty slot's among them: their product is, and such a contribution may stand
+// at another block than its nodes' (k_nr_contrib_emit).
 __global__ __launch_bounds__(256) void k_nr_contrib_weights(const uint32_t *__restrict__ codes, long long nc,
                                                            const int *__restrict__ node_of_vertex,
-                                                           const int *__restrict__ vnn,
                                                            const float *__restrict__ vnn_wn, float2 *__restrict__ cw) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= nc) return;
@@ -363,9 +364,9 @@ __global__ __launch_bounds__(256) void k_nr_contrib_weights(const uint32_t *__re
   float2 w = make_float2(0.f, 0.f);
   if (!(code & kArapTag)) {
     const int64_t v = code >> 4;
-    const int64_t a = kNK * v + ((code >> 2) & 3), b = kNK * v + (code & 3);
     if (node_of_vertex[v] >= 0) w = make_float2(1.f, 1.f);
-    else if (vnn[a] >= 0 && vnn[b] >= 0) w = make_float2(vnn_wn[a], vnn_wn[b]);
+    else w = make_float2(vnn_wn[kNK * v + ((code >> 2) & 3)], vnn_wn[kNK * v + (code & 3)]);
+    if (!(w.x > 0.f && w.y > 0.f)) w = make_float2(0.f, 0.f);
   }
   cw[i] = w;
 }
@@ -1631,7 +1632,7 @@ static int graph_finish(dm_graph *g) {
   DM_TRY(sort_pairs(k0.as<uint32_t>(), k1.as<uint32_t>(), c0.as<uint32_t>(), g->codes, nc, 2 * kNodeBits, st));
   DM_TRY(g->dalloc(&g->cw, nc));
   hipLaunchKernelGGL(k_nr_contrib_weights, dim3(grid_of(nc)), dim3(256), 0, st, g->codes, nc, g->node_of_vertex,
-                     g->vnn, g->vnn_wn, g->cw);
+                     g->vnn_wn, g->cw);
   DM_TRY(dev_alloc(flag, nc * 4));
   DM_TRY(dev_alloc(frank, nc * 8));
   hipLaunchKernelGGL(k_flag_heads, dim3(grid_of(nc)), dim3(256), 0, st, k1.as<uint32_t>(), nc, 0u, flag.as<int>());
@@ -2218,7 +2219,7 @@ int dm_graph_update_nodes(dm_graph *g) {
   if (!g) { set_error("null argument"); return DM_E_INVALID; }
   DM_TRY(graph_links(g));
   hipLaunchKernelGGL(k_nr_contrib_weights, dim3(grid_of(g->ncontrib)), dim3(256), 0, g->stream, g->codes,
-                     g->ncontrib, g->node_of_vertex, g->vnn, g->vnn_wn, g->cw);
+                     g->ncontrib, g->node_of_vertex, g->vnn_wn, g->cw);
   DM_HIP(hipGetLastError());
   DM_HIP(hipStreamSynchronize(g->stream));
   return DM_OK;
