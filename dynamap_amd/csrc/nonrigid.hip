@@ -22,7 +22,7 @@
 //
 // Per Gauss-Newton iteration (all on the graph's stream, no host round
 // trip): blend -> per-vertex data linearisation (association in FP64) ->
-// per-edge ARAP terms -> block assembly (one wavefront per block, FP64
+// per-edge ARAP terms -> block assembly (16 lanes per block, FP64
 // accumulation, FP32 storage; diagonal blocks also produce the rhs, the
 // damping and the FP64 inverse used as block-Jacobi preconditioner) ->
 // PCG with FP64 vectors and fixed-order FP64 dot products -> per-node

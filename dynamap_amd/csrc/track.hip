@@ -105,12 +105,11 @@ constexpr int kVals = 30;
 // normal; model point and normal; the model intensity's neighbours) side by
 // side, every load unconditional at a safe index: taken one pixel after the
 // other, each load behind the test of the one before, an iteration of a coarse
-// level was 12 rounds of memory latency (17 us at 80x60 pixels, now 14;
-// 24 -> 21 at 640x480; 16 sessions at level 0 74 -> 58).  The rest of an
-// iteration is a chain too: 7000 of 34000 cycles the four pixels' arithmetic on
-// few wavefronts, 3000 the tickets, 3500 the records, 9000 the step.  One pixel
-// per thread in workgroups of 1024 took as long (the same wavefronts' work
-// on the same compute unit).
+// level was 12 rounds of memory latency (16 sessions at level 0 74 -> 58 us; one
+// session's iterations at icp_record).  The rest of an iteration is a chain too:
+// 7000 of 34000 cycles the four pixels' arithmetic on few wavefronts, 3000 the
+// tickets, 3500 the records, 9000 the step.  One pixel per thread in workgroups
+// of 1024 took as long (the same wavefronts' work on the same compute unit).
 constexpr int kIcpPer = kIcpPix / 256;  // pixels per thread
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct IcpPixel {
@@ -483,9 +482,10 @@ __device__ void icp_finish(const DmView &v, int level, int it, int nwg, IcpStepL
 // count among themselves, in an unused value of the group's first record, and
 // each group's last one counts for the session.
 // The step in the reduction's launch saves a launch per iteration, most of
-// them no-ops because the level has converged: at 640x480 reduction and step
-// took 18 + 13 us at level 0 and 1.1 + 1.1 us when converged, in one launch 26 and
-// 1.1; a 320x240 frame's 19 iterations 148 -> 136 us of kernels and 19 launches less.
+// them no-ops because the level has converged.  A full iteration of one session
+// took, as reduction + step with the pixels' loads behind their tests, 13.4 + 9.0 us
+// at 640x480 with the photometric term (11.2 + 8.7 without) and 10.7 + 9.0 us at
+// 80x60; now 17.4 (15.3) and 14.1 us in one launch.
 constexpr int kIcpGroup = 16;
 __device__ __forceinline__ void icp_record(const DmView &v, float val, int level, int it, int nwg, int solve,
                                            IcpStepLds &S) {

@@ -228,7 +228,7 @@ __device__ __forceinline__ int alloc_ray(const DmView &v, int u, int r, RayWG &w
     // kAhead steps at a time: their map words are loaded together (past the end
     // the last block's again), so a ray waits for memory once per group
     // instead of once per step (640x480 / 8 mm 35 -> 27 us; 16 sessions, bound by
-    // VALU issue, 150 -> 147).
+    // VALU issue, 150 -> 144).
     constexpr int kAhead = 8;
     for (int it = 0; it < bound; it += kAhead) {
       uint32_t at[kAhead];
@@ -575,11 +575,11 @@ template <int S> __device__ __forceinline__ bool nbr_side(int x, int side, int &
 // this one's voxels are updated.  Straight code for ordinary operands, decided
 // once per block, lets those loads stay in flight (a branch per voxel made the
 // wavefront wait for all of them).
-// Bound by those latencies and the bytes: 16 sessions 365 -> 244 us (855 MB:
-// 3.5 TB/s), 640x480 / 8 mm 45 -> 33 us, 4 mm 328 -> 219 us, 320x240 / 2 cm
-// 13.5 -> 9.4 us.  Before, a workgroup took a block, every wavefront
+// Bound by those latencies and the bytes: 16 sessions 365 -> 225 us (931 MB
+// moved: 4.1 TB/s), 640x480 / 8 mm 45 -> 34 us, 4 mm 328 -> 219 us, 320x240 / 2 cm
+// 13.5 -> 9.9 us.  Before, a workgroup took a block, every wavefront
 // repeated its tests, each voxel its whole transform and two IEEE divisions
-// (1418 VALU instructions per wavefront of the 16-session launch, now 892).
+// (1418 VALU instructions per wavefront of the 16-session launch, now 848).
 __global__ __launch_bounds__(256) void k_integrate(const DmView *__restrict__ views, const int *__restrict__ active) {
   const int slot_ = active[blockIdx.y];
   if (slot_ < 0) return;
