@@ -498,7 +498,7 @@ def test_session_reads_initial_pose_before_return(room):
     depth, poses = room
     w = configs.WORKLOADS["rigid-320x240-2cm"]
     for _ in range(4):
-        T = np.ascontiguousarray(poses[1], np.float64)
+        T = np.array(poses[1], np.float64)  # its own copy: the fixture's stays
         keep, h = T.copy(), C.c_void_p()
         N.check(N.lib().dm_session_create(C.byref(configs.tsdf_props(small_tsdf())), C.byref(configs.icp_props(w["icp"])),
                                           C.byref(configs.sensor(SENS)), N.ptr(T), C.byref(h)))
